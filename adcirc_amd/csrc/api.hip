@@ -97,7 +97,10 @@ struct adcgpu_ctx {
   int jcg_cap = 0;              // resident k_jcg blocks on this device
   int jcg_halo = -1;            // row tiles each side a tile's rows reference (-1: any)
   int jcg_hrows = -1;           // rows each side staged in LDS with a tile's (-1: none)
-  int* jhrange = nullptr;       // per row tile: first and one past the last row it references
+  int* jhrange = nullptr;       // per 2048-row chunk: first and one past the last row it references
+  int jcg_bw = 0;               // matrix bandwidth: the widest |column - row|
+  JcgRegPlan jreg[2];           // the register kernel with one and two chunks per block
+  double* jhprev = nullptr;     // its neighbouring rows' previous d past the LDS
   unsigned* jlcol = nullptr;    // staged: the columns as 16-bit LDS positions, two slots a word
   int jcg_limit = 0;            // caller's limit on JCG blocks per launch (0: the device's)
   bool jcg_mem = false;         // more row tiles than blocks: k_jcg_mem
@@ -241,6 +244,7 @@ int set_jcg_grid(adcgpu_ctx* c) {
                     std::to_string(lim) + " blocks)");
   if (c->jmem_n < c->np) {
     for (double** p : {&c->juo, &c->jdpv, &c->jndv}) {
+      if (p == &c->jndv && c->ne > 0) continue;  // a mesh context has its own
       if (*p) {
         c->allocs.erase(std::find(c->allocs.begin(), c->allocs.end(), (void*)*p));
         (void)hipFree(*p);
@@ -283,7 +287,7 @@ int jcg_barrier_words(const adcgpu_ctx* c) { return jcg_barrier_words_for(c->jcg
 JcgArgs make_jcg_args(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh,
                       double* rhs, double* u, int n, int itmax, double zeta, double* eta2,
                       const double* eta1, const int* nodecode, bool prescaled,
-                      bool defer_unscal, const double* u2) {
+                      bool defer_unscal, const double* u2, int cpb) {
   JcgArgs a;
   std::memset(&a, 0, sizeof(a));  // padding too: batches compare whole structs
   a.n = n;
@@ -312,6 +316,14 @@ JcgArgs make_jcg_args(adcgpu_ctx* c, double* coef, const int* col, const int* nn
     a.hrows = -1;
     a.halo = -1;
   }
+  if (cpb > 0) {  // the register kernel
+    const JcgRegPlan& p = c->jreg[cpb - 1];
+    a.hrows = c->jcg_bw;
+    a.lds_doubles = p.lds_doubles;
+    a.ovf = p.ovf;
+    a.hmem = p.hmem;
+    a.hprev = c->jhprev;
+  }
   a.barrier_ticks = (long long)((double)c->clock_khz * 1000.0 * g_wait_seconds);
   a.flags = c->flags;
   a.eta2 = eta2;
@@ -323,12 +335,24 @@ JcgArgs make_jcg_args(adcgpu_ctx* c, double* coef, const int* col, const int* nn
   return a;
 }
 
+// Chunks per block of the register kernel for the context's own launches; 0:
+// another kernel.  One chunk per block while the blocks are all resident: half
+// the rows per thread and twice the CUs; two beyond that.
+int jcg_reg_cpb(const adcgpu_ctx* c) {
+  if (c->jcg_mem || c->prm.ilump != 0) return 0;
+  const int lim = c->jcg_limit > 0 ? std::min(c->jcg_limit, c->jcg_cap) : c->jcg_cap;
+  for (int cpb = 1; cpb <= 2; ++cpb)
+    if (c->jreg[cpb - 1].ok && jcg_reg_grid(c->np, cpb) <= lim) return cpb;
+  return 0;
+}
+
 int launch_jcg(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh, double* rhs,
                double* u, int n, int itmax, double zeta, double* eta2, const double* eta1,
                const int* nodecode, bool prescaled, bool defer_unscal,
                const double* u2 = nullptr) {
+  const int cpb = prescaled ? jcg_reg_cpb(c) : 0;
   JcgArgs a = make_jcg_args(c, coef, col, nneigh, rhs, u, n, itmax, zeta, eta2, eta1, nodecode,
-                            prescaled, defer_unscal, u2);
+                            prescaled, defer_unscal, u2, cpb);
   // a prescaling pass (k_rhs_node) has already cleared the barrier words
   if (!prescaled) {
     const int bar_words = jcg_barrier_words(c);
@@ -341,12 +365,24 @@ int launch_jcg(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh, d
       if (int rc = grow_events(c, c->jcg_events.size() + 256)) return rc;
     HIPCHK(hipEventRecord(c->jcg_events[c->ev_used].first, c->stream));
   }
-  const void* fn =
-      c->jcg_mem     ? (const void*)k_jcg_mem
-      : a.hrows >= 0 ? (u2 ? (const void*)k_jcg<true, true> : (const void*)k_jcg<false, true>)
-                     : (u2 ? (const void*)k_jcg<true, false> : (const void*)k_jcg<false, false>);
-  HIPCHK(hipLaunchCooperativeKernel(fn, dim3(c->jcg_grid), dim3(JCG_BLOCK), args,
-                                    (unsigned)jcg_stage_bytes(a.hrows), c->stream));
+  const void* fn = nullptr;
+  int grid = c->jcg_grid, threads = JCG_BLOCK;
+  size_t lds = 0;
+  if (cpb > 0) {
+    fn = cpb == 1 ? (u2 ? (const void*)k_jcg_reg<true, 1> : (const void*)k_jcg_reg<false, 1>)
+                  : (u2 ? (const void*)k_jcg_reg<true, 2> : (const void*)k_jcg_reg<false, 2>);
+    grid = jcg_reg_grid(n, cpb);
+    threads = RED_THREADS;
+    lds = (size_t)a.lds_doubles * 8;
+  } else if (c->jcg_mem) {
+    fn = (const void*)k_jcg_mem;
+  } else if (a.hrows >= 0) {
+    fn = u2 ? (const void*)k_jcg<true, true> : (const void*)k_jcg<false, true>;
+    lds = jcg_stage_bytes(a.hrows);
+  } else {
+    fn = u2 ? (const void*)k_jcg<true, false> : (const void*)k_jcg<false, false>;
+  }
+  HIPCHK(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(threads), args, (unsigned)lds, c->stream));
   if (c->profile) HIPCHK(hipEventRecord(c->jcg_events[c->ev_used++].second, c->stream));
   return 0;
 }
@@ -566,20 +602,23 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   }
   // a JCG block's rows reference rows at most this many blocks away
   const int halo_blocks = (bw + JCG_CPB * RED_CHUNK - 1) / (JCG_CPB * RED_CHUNK);
-  // per row tile of a JCG block, the rows its rows reference: [lo, hi)
-  const int ntile = (np + JCG_CPB * RED_CHUNK - 1) / (JCG_CPB * RED_CHUNK);
-  std::vector<int> hrange(2 * (size_t)ntile);
-  for (int tl = 0; tl < ntile; ++tl) {
-    hrange[2 * tl] = tl * JCG_CPB * RED_CHUNK;
-    hrange[2 * tl + 1] = std::min(np, (tl + 1) * JCG_CPB * RED_CHUNK);
+  // per 2048-row chunk, the rows its rows reference: [lo, hi), and the
+  // off-diagonals past the register kernel's slots
+  const int nch0 = (np + RED_CHUNK - 1) / RED_CHUNK;
+  std::vector<int> hrange(2 * (size_t)nch0), over1(nch0, 0), over2(nch0, 0);
+  for (int ch = 0; ch < nch0; ++ch) {
+    hrange[2 * ch] = ch * RED_CHUNK;
+    hrange[2 * ch + 1] = std::min(np, (ch + 1) * RED_CHUNK);
   }
   for (int i = 0; i < np; ++i) {
-    const int tl = i / (JCG_CPB * RED_CHUNK);
+    const int ch = i / RED_CHUNK;
     for (int j = 1; j < nneigh[i]; ++j) {
       const int v = col[(size_t)j * np + i];
-      hrange[2 * tl] = std::min(hrange[2 * tl], v);
-      hrange[2 * tl + 1] = std::max(hrange[2 * tl + 1], v + 1);
+      hrange[2 * ch] = std::min(hrange[2 * ch], v);
+      hrange[2 * ch + 1] = std::max(hrange[2 * ch + 1], v + 1);
     }
+    over1[ch] += std::max(0, nneigh[i] - 1 - JCG_REG_W1);
+    over2[ch] += std::max(0, nneigh[i] - 1 - JCG_REG_W2);
   }
   std::vector<int> csrpos(6 * (size_t)ne);
   for (int e = 0; e < ne; ++e)
@@ -682,16 +721,20 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   // staging needs the point-to-point halo wait (every staged row belongs to a
   // tile within jcg_halo)
   c->jcg_hrows = c->jcg_halo >= 0 ? jcg_stage_rows(bw) : -1;
-  // staged: each off-diagonal column as its position in the tile's staged
-  // rows (fewer than 2^16 by the LDS bound), two slots per word
+  c->jcg_bw = bw;
+  if (P->ilump == 0) {
+    c->jreg[0] = jcg_reg_plan(np, bw, 1, hrange, over1);
+    c->jreg[1] = jcg_reg_plan(np, bw, 2, hrange, over2);
+  }
+  // staged: each off-diagonal column as its position counted from (the first
+  // row of the row's chunk - bandwidth), 16 bits, two slots per word
   std::vector<uint32_t> lcol;
-  if (c->jcg_hrows >= 0) {
+  if (c->jcg_hrows >= 0 || c->jreg[0].ok || c->jreg[1].ok) {
     lcol.assign((size_t)std::max(mnei / 2, 1) * np, 0u);
     for (int i = 0; i < np; ++i) {
-      const int t0 = i / (JCG_CPB * RED_CHUNK) * (JCG_CPB * RED_CHUNK);
-      const int slo = std::max(0, t0 - c->jcg_hrows);
+      const int from = i / RED_CHUNK * RED_CHUNK - bw;
       for (int j = 1; j < nneigh[i]; ++j) {
-        const uint32_t v = (uint32_t)(col[(size_t)j * np + i] - slo);
+        const uint32_t v = (uint32_t)(col[(size_t)j * np + i] - from);
         lcol[(size_t)((j - 1) / 2) * np + i] |= v << (16 * ((j - 1) & 1));
       }
     }
@@ -746,8 +789,13 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   double** nodal[] = {&c->eta1, &c->eta2, &c->etas, &c->uu1, &c->vv1, &c->uu2, &c->vv2,
                       &c->qx1, &c->qy1, &c->qx2, &c->qy2, &c->h1, &c->h2, &c->tk,
                       &c->etamax, &c->totalarea, &c->wsx1, &c->wsy1, &c->wsx2, &c->wsy2,
-                      &c->pr1, &c->pr2, &c->gwce_lv, &c->jd, &c->jw};
+                      &c->pr1, &c->pr2, &c->gwce_lv, &c->jw};
   for (auto p : nodal) A(p, np);
+  // the solver's published vectors, padded to whole tiles
+  const size_t npad = (size_t)nblk(np, 2 * RED_CHUNK) * 2 * RED_CHUNK;
+  A(&c->jd, npad); A(&c->jndv, npad);
+  A(&c->jhprev, std::max((size_t)c->jreg[0].hmem * nblk(np, RED_CHUNK),
+                         (size_t)c->jreg[1].hmem * nblk(np, 2 * RED_CHUNK)));
   A(&c->alphal, ne); A(&c->coef, (size_t)mnei * np); A(&c->cs, (size_t)mnei * np);
   A(&c->obc, (size_t)std::max(neta, 1) * mnei);
   A(&c->nodecode, np); A(&c->nnodecode, np); A(&c->noff, ne); A(&c->noffold, ne);
@@ -780,7 +828,7 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     A(&c->wd.xcnt, nwb);
     A(&c->wd.xval, nwb * WD_XMAX);
   }
-  A(&c->flags, F_COUNT); A(&c->jpart, 2 * (size_t)c->nch * 4); A(&c->jsaved, 12);
+  A(&c->flags, F_COUNT); A(&c->jpart, jcg_part_doubles(c->nch)); A(&c->jsaved, 12);
   A(&c->jbar, JCG_BAR_WORDS);
   if (!rc) {
     hipError_t e = hipStreamCreate(&c->stream);
@@ -1143,7 +1191,6 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, GwceStep* g) {
   const int np = c->np, ne = c->ne;
   const bool lumped = c->prm.ilump != 0;
   const size_t rows_lds = (size_t)c->mnei * RED_THREADS * sizeof(double);
-  const double* rcs = c->coef_scaled ? (const double*)c->cs : nullptr;
   const double* rw = c->coef_scaled ? (const double*)c->jw : nullptr;
   // a rebuild multiplies the cached terms by each element's NCEle, which the
   // momentum element pass left unless the flags changed since
@@ -1162,17 +1209,17 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, GwceStep* g) {
   if (c->mixed) {
     if (lumped)
       hipLaunchKernelGGL((k_lhs_rows<true, float>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rcs, rw);
+                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
     else
       hipLaunchKernelGGL((k_lhs_rows<false, float>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rcs, rw);
+                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
   } else {
     if (lumped)
       hipLaunchKernelGGL((k_lhs_rows<true, double>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rcs, rw);
+                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
     else
       hipLaunchKernelGGL((k_lhs_rows<false, double>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rcs, rw);
+                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
   }
   if (c->lhs_pairs) {
     // the cached rebuild (k_lhs_rows above only restored or left at once)
@@ -1215,7 +1262,9 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, GwceStep* g) {
       hipLaunchKernelGGL(k_ml_collect, dim3(nblk(c->ml_collect, 128)), dim3(256), 0, c->stream,
                          in, c->smp, slot0, c->ml_collect, c->cur_it);
   }
-  JcgPre pre{c->jw, c->jbar, jcg_barrier_words(c), c->flags, c->etas_prev, c->prm.warm_start,
+  JcgPre pre{c->jw, c->jbar, jcg_barrier_words(c),
+             reinterpret_cast<unsigned long long*>(c->jpart), jcg_part_doubles(c->nch),
+             c->flags, c->etas_prev, c->prm.warm_start,
              (c->prm.warm_start != 0 || c->ml_ready) ? 1 : 0, c->ml_corr, c->ml_u};
   const dim3 ng(nblk(np, 256)), nbk(256);
   // with ILump = 1 the explicit solve of the lumped GWCE ends the node pass; no JCG
@@ -1242,10 +1291,10 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, GwceStep* g) {
 }
 
 // The arguments of the step's JCG launch (prescaled rows, ETA2 written at the end).
-static JcgArgs gwce_jcg_args(adcgpu_ctx* c, const GwceStep& g, bool deferred) {
+static JcgArgs gwce_jcg_args(adcgpu_ctx* c, const GwceStep& g, bool deferred, int cpb) {
   return make_jcg_args(c, c->coef, c->col, c->nneigh, c->gwce_lv, c->etas, c->np, c->prm.itmax,
                        c->prm.convcr, c->eta2, c->eta1, c->nodecode, true, deferred,
-                       g.learned ? c->ml_u : nullptr);
+                       g.learned ? c->ml_u : nullptr, cpb);
 }
 
 // After the solve: the off-diagonals left scaled (deferred) and the training
@@ -1275,7 +1324,7 @@ static int gwce_device(adcgpu_ctx* c, const double* d_eta_bc, bool deferred) {
 static int restore_coef(adcgpu_ctx* c) {
   if (!c->coef_scaled) return 0;
   hipLaunchKernelGGL(k_coef_restore, dim3(nblk(c->np, 256)), dim3(256), 0, c->stream, c->mesh(),
-                     c->state(), (const double*)c->cs, (const double*)c->jw);
+                     c->state(), (const double*)c->jw);
   c->coef_scaled = false;
   return check_launch("coef restore");
 }
@@ -1515,6 +1564,7 @@ struct adcgpu_batch {
   // members `sm`, launched with first-block offsets dfirst[gf[g] ..]
   std::vector<int> sm, gm, gf;
   std::vector<bool> gdual;
+  std::vector<int> gcpb;     // chunks per block of the register kernel (0: k_jcg_batch)
   int* dfirst = nullptr;
   JcgArgs* dargs = nullptr;  // [2][n]: the launch arguments by step parity
   JcgArgs* hargs = nullptr;  // pinned host copy of what dargs holds
@@ -1559,22 +1609,44 @@ int adcgpu_batch_create(adcgpu_ctx* const* members, int n, adcgpu_batch** out) {
     if (members[k]->prm.ilump == 0) b->sm.push_back(k);
   int sum = 0;
   bool dual = false;
-  std::vector<int> first;
   for (size_t q = 0; q < b->sm.size(); ++q) {
     adcgpu_ctx* c = members[b->sm[q]];
     const bool d = c->prm.warm_start == 2;
     if (q == 0 || sum + c->jcg_grid > cap || d != dual) {
       b->gm.push_back((int)q);
-      b->gf.push_back((int)first.size());
       b->gdual.push_back(d);
-      first.push_back(0);
       sum = 0;
       dual = d;
     }
     sum += c->jcg_grid;
-    first.push_back(sum);
   }
   b->gm.push_back((int)b->sm.size());
+  // per group the register kernel with one chunk per block if all its members'
+  // blocks are then resident together, else with two; k_jcg_batch when some
+  // member cannot run it
+  std::vector<int> first;
+  for (size_t gi = 0; gi + 1 < b->gm.size(); ++gi) {
+    int cpb = 0;
+    for (int k = 2; k >= 1; --k) {
+      int blocks = 0;
+      bool ok = true;
+      for (int q = b->gm[gi]; q < b->gm[gi + 1]; ++q) {
+        const adcgpu_ctx* c = members[b->sm[q]];
+        ok = ok && c->jreg[k - 1].ok;
+        blocks += jcg_reg_grid(c->np, k);
+      }
+      if (ok && blocks <= cap) cpb = k;
+    }
+    b->gcpb.push_back(cpb);
+    b->gf.push_back((int)first.size());
+    int at = 0;
+    first.push_back(0);
+    for (int q = b->gm[gi]; q < b->gm[gi + 1]; ++q) {
+      const adcgpu_ctx* c = members[b->sm[q]];
+      at += cpb > 0 ? jcg_reg_grid(c->np, cpb) : c->jcg_grid;
+      first.push_back(at);
+    }
+  }
   int rc = 0;
   if (!first.empty()) rc = upload(&b->dfirst, first);
   if (!rc && !b->sm.empty()) rc = dmalloc(&b->dargs, 2 * b->sm.size());
@@ -1627,11 +1699,11 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
     if (!rc && ns) {
       JcgArgs* h = b->hargs + par * ns;
       std::vector<JcgArgs> cur(ns);
-      for (size_t q = 0; q < ns; ++q) {
-        adcgpu_ctx* c = b->m[b->sm[q]];
-        cur[q] = gwce_jcg_args(c, g[b->sm[q]], true);
-      }
+      for (size_t gi = 0; gi + 1 < b->gm.size(); ++gi)
+        for (int q = b->gm[gi]; q < b->gm[gi + 1]; ++q)
+          cur[q] = gwce_jcg_args(b->m[b->sm[q]], g[b->sm[q]], true, b->gcpb[gi]);
       for (size_t gi = 0; gi + 1 < b->gm.size(); ++gi) {
+        if (b->gcpb[gi] > 0) continue;
         // a group runs staged only if all its members can
         bool st = true;
         for (int q = b->gm[gi]; q < b->gm[gi + 1]; ++q) st = st && cur[q].hrows >= 0;
@@ -1647,22 +1719,31 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
       }
       for (size_t gi = 0; gi + 1 < b->gm.size() && !rc; ++gi) {
         const int q0 = b->gm[gi], q1 = b->gm[gi + 1];
-        int grid = 0, hmax = -1;
+        const int cpb = b->gcpb[gi];
+        int grid = 0, hmax = -1, lds_doubles = 0;
         for (int q = q0; q < q1; ++q) {
-          grid += b->m[b->sm[q]]->jcg_grid;
+          const adcgpu_ctx* c = b->m[b->sm[q]];
+          grid += cpb > 0 ? jcg_reg_grid(c->np, cpb) : c->jcg_grid;
           hmax = std::max(hmax, cur[q].hrows);
+          lds_doubles = std::max(lds_doubles, cur[q].lds_doubles);
         }
-        const bool st = cur[q0].hrows >= 0;
-        const void* fn = b->gdual[gi] ? (st ? (const void*)k_jcg_batch<true, true>
-                                            : (const void*)k_jcg_batch<true, false>)
-                                      : (st ? (const void*)k_jcg_batch<false, true>
-                                            : (const void*)k_jcg_batch<false, false>);
+        const bool st = cur[q0].hrows >= 0, d = b->gdual[gi];
+        const void* fn =
+            cpb == 1   ? (d ? (const void*)k_jcg_reg_batch<true, 1>
+                            : (const void*)k_jcg_reg_batch<false, 1>)
+            : cpb == 2 ? (d ? (const void*)k_jcg_reg_batch<true, 2>
+                            : (const void*)k_jcg_reg_batch<false, 2>)
+            : d        ? (st ? (const void*)k_jcg_batch<true, true>
+                             : (const void*)k_jcg_batch<true, false>)
+                       : (st ? (const void*)k_jcg_batch<false, true>
+                             : (const void*)k_jcg_batch<false, false>);
+        const size_t lds = cpb > 0 ? (size_t)lds_doubles * 8 : jcg_stage_bytes(st ? hmax : -1);
         const JcgArgs* pa = b->dargs + par * ns + q0;
         const int* pf = b->dfirst + b->gf[gi];
         int nsys = q1 - q0;
         void* args[] = {(void*)&pa, (void*)&pf, (void*)&nsys};
         const hipError_t e = hipLaunchCooperativeKernel(
-            fn, dim3(grid), dim3(JCG_BLOCK), args, (unsigned)jcg_stage_bytes(st ? hmax : -1),
+            fn, dim3(grid), dim3(cpb > 0 ? RED_THREADS : JCG_BLOCK), args, (unsigned)lds,
             b->stream);
         if (e != hipSuccess) rc = fail(ADCGPU_E_HIP, std::string("batched JCG: ") +
                                                          hipGetErrorString(e));

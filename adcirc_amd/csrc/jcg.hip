@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "jcg_device.h"
 #include "kernels.h"
 #include "reduce.h"
 
@@ -155,24 +156,6 @@ __device__ __forceinline__ bool halo_sync(unsigned* hflags, int tile, int lo, in
   return failed == 0;
 }
 
-// Element access through a 32-bit byte offset from a uniform base: the
-// addresses then take the scalar-base + 32-bit-offset form of the vector
-// memory instructions instead of one 64-bit VGPR pair per row.  Arrays here
-// stay below 4 GiB (checked on the host).
-template <class T>
-__device__ __forceinline__ T& at(T* base, unsigned i) {
-  return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + i * (unsigned)sizeof(T));
-}
-template <class T>
-__device__ __forceinline__ const T& at(const T* base, unsigned i) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + i * (unsigned)sizeof(T));
-}
-
-// Agent-scope load of a value another block wrote (coherent across XCDs).
-__device__ __forceinline__ double ld_agent(const double* p) {
-  return __hip_atomic_load(const_cast<double*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // The neighbouring tiles' rows lo .. t0-1 and t1 .. hi-1 of v into the staged
 // rows (dsh holds rows slo ..); a thread's loads are all issued before their
 // LDS stores.
@@ -193,184 +176,6 @@ __device__ __forceinline__ void stage_halo(double* dsh, const double* v, int slo
     for (int m = 0; m < K; ++m)
       if (k0 + m * JCG_BLOCK < nh) dsh[row[m] - slo] = x[m];
   }
-}
-
-struct ItLocal {
-  int in, adapt, halt, q1, maxfn, nsig, itmax, stop;
-  double zeta, cme, gamma, rho, delnnm, delsnm, udnm, stptst, gamold, rhoold, cmold;
-  double c1, c2, c3, c4, tz;
-};
-
-// determ (src/itpackv.F:1029-1068): the backward three-term recurrence with
-// the two running values kept in registers (same operations, same order).
-__device__ double jcg_determ(int n, const double* tri1, const double* tri2, double x) {
-  double a2 = tri1[n - 1] - x;                            // wk2(n)
-  double a1 = (tri1[n - 2] - x) * a2 + tri2[n - 1];       // wk2(n-1)
-  for (int l = n - 3; l >= 0; --l) {
-    const double w = (tri1[l] - x) * a1 + tri2[l + 1] * a2;  // wk2(l)
-    a2 = a1;
-    a1 = w;
-  }
-  return a1;
-}
-
-// zbrent (src/itpackv.F:2521-2781) with eps = 0; returns ier, result in *pb.
-__device__ int jcg_zbrent(int n, const double* tri1, const double* tri2, double t, int maxfn,
-                          double a, double* pb) {
-  double b = 1.0, c = 0, d = 0, e = 0, p, qq, r, ss, fa, fb, fc = 0, tol, rm, rone, temp;
-  int ic = 2;
-  const double eps = 0.0;
-  fa = jcg_determ(n, tri1, tri2, a);
-  fb = jcg_determ(n, tri1, tri2, b);
-  if ((fa > 0.0 && fb > 0.0) || (fa < 0.0 && fb < 0.0)) {
-    *pb = b;
-    return 502;
-  }
-  bool reset = true;
-  while (true) {
-    if (reset) {
-      c = a; fc = fa; d = b - c; e = d;
-    }
-    if (!(fabs(fc) >= fabs(fb))) {
-      a = b; b = c; c = a; fa = fb; fb = fc; fc = fa;
-    }
-    tol = t * fmax(fabs(b), 0.1);
-    rm = (c - b) * 0.5;
-    if (fabs(fb) <= eps || fabs(c - b) <= tol) { *pb = b; return 0; }
-    if (ic >= maxfn) { *pb = b; return 501; }
-    bool bisect = (fabs(e) < tol) || (fabs(fa) <= fabs(fb));
-    if (!bisect) {
-      ss = fb / fa;
-      if (a == c) {
-        p = (c - b) * ss;
-        qq = 1.0 - ss;
-      } else {
-        qq = fa / fc;
-        r = fb / fc;
-        rone = r - 1.0;
-        p = ss * ((c - b) * qq * (qq - r) - (b - a) * rone);
-        qq = (qq - 1.0) * rone * (ss - 1.0);
-      }
-      if (p > 0.0) qq = -qq;
-      if (p < 0.0) p = -p;
-      ss = e;
-      e = d;
-      if (p + p >= 3.0 * rm * qq || p + p >= fabs(ss * qq)) {
-        bisect = true;
-      } else {
-        d = p / qq;
-      }
-    }
-    if (bisect) { e = rm; d = e; }
-    a = b;
-    fa = fb;
-    temp = d;
-    if (fabs(temp) <= 0.5 * tol) temp = copysign(0.5 * tol, rm);
-    b = b + temp;
-    fb = jcg_determ(n, tri1, tri2, b);
-    ic = ic + 1;
-    if (fb == 0.0 || fc == 0.0) { reset = false; continue; }
-    if ((fb > 0.0 && fc < 0.0) || (fb < 0.0 && fc > 0.0)) { reset = false; continue; }
-    reset = true;
-  }
-}
-
-// chgcon(ibmth=1) (src/itpackv.F:893-1027); tri1/tri2 are the two columns.
-__device__ void jcg_chgcon(ItLocal& L, double* tri1, double* tri2) {
-  const int ip = L.in;
-  double start = L.cme, end1;
-  if (ip == 0) {
-    end1 = 0.0;
-    L.cmold = 0.0;
-  } else if (ip == 1) {
-    end1 = 1.0 - 1.0 / L.gamma;
-    tri1[0] = end1;
-    tri2[0] = 0.0;
-  } else {
-    if (fabs(start - L.cmold) <= L.zeta * start) {
-      L.adapt = 0;
-      return;
-    }
-    L.cmold = start;
-    tri1[ip - 1] = 1.0 - 1.0 / L.gamma;
-    tri2[ip - 1] = (1.0 - L.rho) / (L.rho * L.rhoold * L.gamma * L.gamold);
-    double b;
-    int ier = jcg_zbrent(ip, tri1, tri2, L.tz, L.maxfn, start, &b);
-    if (ier != 0) {
-      L.adapt = 0;
-      return;
-    }
-    end1 = b;
-  }
-  L.cme = end1;
-}
-
-// pstop_nrms(iflag=1) (src/itpackv.F:809-890)
-__device__ void jcg_pstop(ItLocal& L, double unrm, double dnrm) {
-  const double con = L.cme;
-  double uold, tr, tl;
-  L.halt = 0;
-  if (L.in < 1) {
-    L.q1 = 0;
-    L.udnm = 1.0;
-    L.stptst = 1000.0;
-  }
-  if (!(L.q1 || (L.in > 5 && (L.in % 5) != 0))) {
-    uold = L.udnm;
-    L.udnm = unrm;
-    if (L.udnm == 0.0) L.udnm = 1.0;
-    if (L.in > 5 && fabs(L.udnm - uold) <= L.udnm * L.zeta) L.q1 = 1;
-  }
-  tr = __builtin_sqrt(L.udnm);
-  tl = 1.0;
-  if (con != 1.0) {
-    tl = __builtin_sqrt(dnrm);
-    tr = tr * (1.0 - con);
-  }
-  L.stptst = tl / tr;
-  if (tl >= tr * L.zeta) return;
-  L.halt = 1;
-}
-
-// parcon(ibmth=1) (src/itpackv.F:1774-1851)
-__device__ void jcg_parcon(ItLocal& L, double dtnrm) {
-  const int ip = L.in;
-  const double rhoold = L.rho;
-  L.gamold = L.gamma;
-  L.gamma = 1.0 / (1.0 - dtnrm / L.delnnm);
-  L.rho = 1.0;
-  if (ip != 0) L.rho = 1.0 / (1.0 - L.gamma * L.delnnm / (L.gamold * L.delsnm * rhoold));
-  L.delsnm = L.delnnm;
-  L.rhoold = rhoold;
-  L.c1 = L.rho * L.gamma;
-  L.c2 = L.rho;
-  L.c3 = 1.0 - L.rho;
-  L.c4 = L.rho * (1.0 - L.gamma);
-}
-
-
-// The solve's scalar state at the start of a launch: ITPACK's SAVEd values
-// from the last solve, the rest cleared (thread 0).
-__device__ __forceinline__ void jcg_init_state(ItLocal& L, const JcgArgs& a) {
-  L.in = 0;
-  L.adapt = 1;
-  L.halt = 0;
-  L.q1 = a.saved[0] != 0.0;
-  L.gamold = a.saved[1];
-  L.rhoold = a.saved[2];
-  L.cmold = a.saved[3];
-  L.itmax = a.itmax;
-  L.zeta = a.zeta;
-  L.cme = 0.0;
-  L.gamma = 0.0;
-  L.rho = 0.0;
-  L.delnnm = 0.0;
-  L.delsnm = 0.0;
-  L.udnm = 0.0;
-  L.stptst = 0.0;
-  L.maxfn = a.maxfn;
-  L.tz = a.tz;
-  L.stop = 0;
 }
 
 // After iteration in's grid barrier: the chunk partials reduced by every
@@ -423,27 +228,13 @@ __device__ __forceinline__ void jcg_scalars(ItLocal& L, const JcgArgs& a, double
 // iteration's pair).
 __device__ __forceinline__ void jcg_eig_step(ItLocal& L, const JcgArgs& a, double* tri1,
                                              double* tri2, int in) {
-  if (threadIdx.x == 0) {
-    L.in = in;
-    if (L.adapt) jcg_chgcon(L, tri1, tri2);
-    a.saved[6 + 2 * (in & 1)] = L.cme;
-    a.saved[7 + 2 * (in & 1)] = L.cmold;
+  if (threadIdx.x < 64) {
+    jcg_eig_wave(L, tri1, tri2, in);
+    if (threadIdx.x == 0) {
+      a.saved[6 + 2 * (in & 1)] = L.cme;
+      a.saved[7 + 2 * (in & 1)] = L.cmold;
+    }
   }
-}
-
-// The solve's outcome and SAVEd state (block 0, thread 0).
-__device__ __forceinline__ void jcg_finish(const ItLocal& L, const JcgArgs& a, bool halted) {
-  const int in_final = halted ? L.in : a.itmax;
-  a.flags[F_NUMITR] = in_final;
-  a.flags[F_IER] = halted ? 0 : 13;
-  a.saved[0] = L.q1 ? 1.0 : 0.0;
-  a.saved[1] = L.gamold;
-  a.saved[2] = L.rhoold;
-  a.saved[3] = L.cmold;
-  a.saved[4] = L.cme;
-  a.saved[5] = L.stptst;
-  a.flags[F_ITSUM] += in_final;
-  if (!halted) a.flags[F_NITMAX] += 1;
 }
 
 // The per-row partials of one 2048-row chunk (threads g*512 .. g*512+511 of
@@ -500,14 +291,21 @@ __device__ __forceinline__ void jcg_solve(const JcgArgs& a, int bid, int nblocks
   const int base = c * RED_CHUNK + t % RED_THREADS;
   unsigned gen = 0;
   int* err = a.flags + F_ERROR;
-  // the staged rows: the tile's own rows t0 .. t1-1 and hrows each side
+  // the staged rows: the tile's own rows t0 .. t1-1 and hrows each side (the
+  // first position stands for row t0 - hrows, which may lie before row 0)
   const bool staged = STAGED && !eig_block;
   const int t0 = tile * JCG_CPB * RED_CHUNK;
   const int t1 = t0 + JCG_CPB * RED_CHUNK < np ? t0 + JCG_CPB * RED_CHUNK : np;
-  const int slo = staged ? (t0 - a.hrows > 0 ? t0 - a.hrows : 0) : 0;
+  const int slo = staged ? t0 - a.hrows : 0;
   // the rows the tile's rows reference, within slo .. t1 + hrows - 1
-  const int hlo_row = staged ? a.hrange[2 * tile] : 0;
-  const int hhi_row = staged ? a.hrange[2 * tile + 1] : 0;
+  int hlo_row = t0, hhi_row = t1;
+  if (staged)
+    for (int k = tile * JCG_CPB; k < tile * JCG_CPB + JCG_CPB && k < nch; ++k) {
+      hlo_row = a.hrange[2 * k] < hlo_row ? a.hrange[2 * k] : hlo_row;
+      hhi_row = a.hrange[2 * k + 1] > hhi_row ? a.hrange[2 * k + 1] : hhi_row;
+    }
+  // positions count from the chunk's first row less hrows
+  const double* dst = dsh + (t / RED_THREADS) * RED_CHUNK;
 
   if (t == 0) jcg_init_state(L, a);
   __syncthreads();
@@ -754,7 +552,7 @@ __device__ __forceinline__ void jcg_solve(const JcgArgs& a, int bid, int nblocks
 #pragma unroll
           for (int r = h; r < h + 4; ++r)
             if (j < NN(r))
-              nd[r] = nd[r] - sc[r - h] * (STAGED ? dsh[cc[r - h]] : at(dv, cc[r - h]));
+              nd[r] = nd[r] - sc[r - h] * (STAGED ? dst[cc[r - h]] : at(dv, cc[r - h]));
         }
       }
       double add = 0.0, adt = 0.0, auu = 0.0;

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "kernels.h"
 
@@ -40,36 +41,44 @@ inline int jcg_barrier_words_for(int grid) {
 // passes its first grid barrier, so the smaller of the two counts is used.
 // The device's capacity is that per-CU count times the CUs, and at most what
 // the barrier words hold.
-inline hipError_t jcg_resident_cap_of(const void* fn, int* per_cu_out) {
+inline hipError_t jcg_resident_cap_of(const void* fn, int threads, int lds, int* per_cu_out) {
   int per_cu = 0;
-  // the largest staged pseudo-residual a launch may ask for
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     JCG_STAGE_MAX_BYTES);
+  // the most dynamic LDS a launch may ask for
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return e;
-  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, JCG_BLOCK, JCG_STAGE_MAX_BYTES);
+  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds);
   if (e != hipSuccess) return e;
   hipFuncAttributes fa;
   if ((e = hipFuncGetAttributes(&fa, fn)) != hipSuccess) return e;
   const int vgpr = std::max((fa.numRegs + 7) & ~7, 8);  // allocation granule 8
   const int per_simd = std::min(8, 512 / vgpr);
-  const int waves = (JCG_BLOCK + 63) / 64;
+  const int waves = (threads + 63) / 64;
   *per_cu_out = std::min(per_cu, per_simd / ((waves + 3) / 4));
   return hipSuccess;
 }
 
-// Every variant of the kernel that is launched must fit: one start or two,
-// and one start with the staged pseudo-residual; single and batched.
+// Every variant of the kernel that is launched must fit.
 inline hipError_t jcg_resident_cap(int device, int* cap) {
   const void* fns[] = {(const void*)k_jcg<false, false>,      (const void*)k_jcg<true, false>,
                        (const void*)k_jcg<false, true>,       (const void*)k_jcg<true, true>,
                        (const void*)k_jcg_batch<false, false>, (const void*)k_jcg_batch<true, false>,
                        (const void*)k_jcg_batch<false, true>, (const void*)k_jcg_batch<true, true>,
                        (const void*)k_jcg_mem};
+  const void* regs[] = {
+      (const void*)k_jcg_reg<false, 1>,       (const void*)k_jcg_reg<false, 2>,
+      (const void*)k_jcg_reg<true, 1>,        (const void*)k_jcg_reg<true, 2>,
+      (const void*)k_jcg_reg_batch<false, 1>, (const void*)k_jcg_reg_batch<false, 2>,
+      (const void*)k_jcg_reg_batch<true, 1>,  (const void*)k_jcg_reg_batch<true, 2>};
   int per_cu = 1 << 30;
   hipError_t e = hipSuccess;
   for (const void* fn : fns) {
     int p = 0;
-    if ((e = jcg_resident_cap_of(fn, &p)) != hipSuccess) return e;
+    if ((e = jcg_resident_cap_of(fn, JCG_BLOCK, JCG_STAGE_MAX_BYTES, &p)) != hipSuccess) return e;
+    per_cu = std::min(per_cu, p);
+  }
+  for (const void* fn : regs) {
+    int p = 0;
+    if ((e = jcg_resident_cap_of(fn, RED_THREADS, JCG_REG_LDS_BYTES, &p)) != hipSuccess) return e;
     per_cu = std::min(per_cu, p);
   }
   int cus = 0;
@@ -87,6 +96,58 @@ inline hipError_t jcg_resident_cap(int device, int* cap) {
 inline int jcg_grid_for(int n) {
   const int nch = (n + RED_CHUNK - 1) / RED_CHUNK;
   return (nch + JCG_CPB - 1) / JCG_CPB + 1;
+}
+
+// The register kernel's launch for one system, with `cpb` chunks per block:
+// whether it can run, and its LDS.  hrange: per chunk the first and one past the
+// last row its rows reference; over[c]: off-diagonals past the register slots
+// of chunk c's rows.  A block keeps the rows it references (and one zero), the
+// entries past the slots, and as much of its neighbouring rows' previous d as
+// the LDS still takes; `hmem` rows of it per block go to memory.
+struct JcgRegPlan {
+  bool ok = false;
+  int lds_doubles = 0, ovf = 0, hmem = 0;
+};
+inline JcgRegPlan jcg_reg_plan(int n, int bw, int cpb, const std::vector<int>& hrange,
+                               const std::vector<int>& over) {
+  JcgRegPlan p;
+  const int nch = (n + RED_CHUNK - 1) / RED_CHUNK;
+  // 16-bit positions: of the packed columns and of the window
+  if (RED_CHUNK + 2 * (long long)bw > 65535) return p;
+  int base = 0, all = 0;
+  for (int c0 = 0; c0 < nch; c0 += cpb) {
+    const int t0 = c0 * RED_CHUNK, t1 = std::min(n, t0 + cpb * RED_CHUNK);
+    int lo = t0, hi = t1, ov = 0;
+    for (int c = c0; c < std::min(nch, c0 + cpb); ++c) {
+      lo = std::min(lo, hrange[2 * c]);
+      hi = std::max(hi, hrange[2 * c + 1]);
+      ov += over[c];
+    }
+    const int nh = (t0 - lo) + (hi - t1), win = nh + cpb * RED_CHUNK;
+    p.ovf = std::max(p.ovf, ov);
+    base = std::max(base, win + 1);
+    all = std::max(all, win + 1 + nh);
+  }
+  const int ovd = p.ovf + (p.ovf + 3) / 4;
+  const int most = JCG_REG_LDS_BYTES / 8;
+  if (base + ovd > most || base > 65535) return p;
+  p.lds_doubles = std::min(all + ovd, most);
+  for (int c0 = 0; c0 < nch; c0 += cpb) {
+    const int t0 = c0 * RED_CHUNK, t1 = std::min(n, t0 + cpb * RED_CHUNK);
+    int lo = t0, hi = t1;
+    for (int c = c0; c < std::min(nch, c0 + cpb); ++c) {
+      lo = std::min(lo, hrange[2 * c]);
+      hi = std::max(hi, hrange[2 * c + 1]);
+    }
+    const int nh = (t0 - lo) + (hi - t1), win = nh + cpb * RED_CHUNK;
+    p.hmem = std::max(p.hmem, nh - (p.lds_doubles - (win + 1) - ovd));
+  }
+  p.ok = true;
+  return p;
+}
+inline int jcg_reg_grid(int n, int cpb) {
+  const int nch = (n + RED_CHUNK - 1) / RED_CHUNK;
+  return (nch + cpb - 1) / cpb + 1;
 }
 
 // ITPACK's tolerances of one solve: zeta raised to 512*srelpr when smaller

@@ -22,6 +22,13 @@ constexpr int JCG_BAR_WORDS = 10240;     // barrier words: (groups + 2) * JCG_BA
 constexpr int JCG_HALO_STRIDE = 16;      // words between per-tile halo flags (64 B)
 constexpr int JCG_HALO_MAX = 2;          // widest halo (tiles each side) waited on by flags
 constexpr int JCG_MAX_ITMAX = 256;       // tridiagonal history length (itmax)
+// k_jcg_reg: 2048-row chunks per 512-thread block, matrix entries per row in
+// registers (by chunks per block), LDS it may use in all
+constexpr int JCG_REG_W1 = 8, JCG_REG_W2 = 6;
+constexpr int JCG_REG_LDS_BYTES = 152 * 1024;
+// an empty partial slot: a quiet NaN no computation produces
+constexpr unsigned long long JCG_EMPTY = 0xfff8badc0ffee000ull;
+__host__ __device__ constexpr int jcg_part_doubles(int nch) { return 4 * 4 * (nch + 1); }
 // dynamic LDS for the staged pseudo-residual of a k_jcg block (JcgArgs.hrows),
 // at most: the block's rows and 5,632 rows each side
 constexpr int JCG_STAGE_MAX_BYTES = 120 * 1024;
@@ -249,22 +256,24 @@ struct JcgArgs {
   double* u;          // initial guess in (scaled in place), ETAS out
   double* d;          // pseudo-residual of the current iteration
   double* w;          // 1/sqrt(diag)
-  double* part;       // [2][nch*4] chunk partials (d.d, d.Nd, u.u), by iteration parity
+  double* part;       // chunk partials (d.d, d.Nd, u.u): [2][nch*4] by iteration parity;
+                      // k_jcg_reg: [4][(nch+1)*4] slots (jcg_part_doubles)
   double* saved;      // [12] ITPACK SAVE state q1, gamold, rhoold, cmold, cme,
                       // stptst; [6..9] = cme, cmold of the running iteration, by parity
   int prescaled;      // rows already scaled (w, u, rhs) by k_rhs_node
-  int defer_unscal;   // leave the off-diagonals scaled (k_lhs_rows restores them)
+  int defer_unscal;   // leave the off-diagonals unscaled (k_lhs_rows scales and
+                      // unscales them if they are needed again)
   unsigned* barrier;  // [JCG_BAR_WORDS] grid barrier counters, then per-tile halo flags
   int hrows;          // >= 0: the pseudo-residual of the tile's rows and of hrows
                       // rows each side (at least the matrix bandwidth) is kept
                       // in LDS for the products (dynamic shared memory of
                       // 8 (JCG_CPB RED_CHUNK + 2 hrows) bytes); -1: gathered
                       // from memory
-  const int* hrange;  // staged: per row tile, the first and one past the last row
-                      // its rows reference (within hrows of the tile)
+  const int* hrange;  // staged: per 2048-row chunk, the first and one past the last
+                      // row its rows reference (within hrows of the chunk)
   const unsigned* lcol;  // staged: [(mnei/2)][n] per row, off-diagonal slots 2p+1
-                         // and 2p+2 as positions in the tile's staged rows, 16
-                         // bits each (low half first)
+                         // and 2p+2 as positions counted from row (chunk's first
+                         // row - hrows), 16 bits each (low half first)
   int halo;           // row tiles each side whose pseudo-residual a tile's rows read;
                       // -1: wait for all tiles (a grid barrier) after each update
   long long barrier_ticks;  // longest grid-barrier wait, in wall-clock ticks
@@ -275,6 +284,11 @@ struct JcgArgs {
   double* uo;         // k_jcg_mem: [n] the previous u
   double* dpv;        //             [n] the previous d
   double* ndv;        //             [n] N d
+  int lds_doubles;    // k_jcg_reg: doubles of dynamic LDS of a block
+  int ovf;            //            of which for entries past the register slots
+                      //            (coefficient and 16-bit position of each)
+  int hmem;           //            neighbouring rows of a block whose previous d
+  double* hprev;      //            does not fit the LDS: [row blocks][hmem]
   const double* u2;   // k_jcg<true>: the second (learned) start, scaled like u
   double* d2;         //              and its initial pseudo-residual
 };
@@ -299,7 +313,7 @@ __global__ void k_lhs_elem(DevMesh m, DevState s, const int* flags, double* sd, 
 template <bool LUMPED, typename CT>
 __global__ void k_lhs_rows(DevMesh m, DevState s, const int* flags, const double* sd,
                            const double* sa, const double* sb, LhsTerms lt, double* ep_part,
-                           const double* restore_cs, const double* restore_w);
+                           const double* restore_w);
 // the cached terms (once per context): k_lhs_elem's terms with NCEle = 1 and
 // ALPHAL = 1, and their FP32 roundings when td32 != null
 template <bool LUMPED>
@@ -319,7 +333,7 @@ __global__ void k_lhs_pair_setup(DevMesh m, LhsTerms lt, const int* c1, const in
 template <typename CT>
 __global__ void k_lhs_pairs(DevMesh m, DevState s, const int* flags, LhsTerms lt, LhsPairs lp);
 __global__ void k_lhs_ep(DevMesh m, DevState s, const int* flags, double* ep_part);
-__global__ void k_coef_restore(DevMesh m, DevState s, const double* cs, const double* w);
+__global__ void k_coef_restore(DevMesh m, DevState s, const double* w);
 // one block more than the elements need: the last finishes the GWCE matrix
 __global__ void k_rhs_elem(DevMesh m, DevState s, RhsPrm q, int* flags, double* contrib, int nch,
                            const double* ep_part, double* scal);
@@ -331,6 +345,8 @@ struct JcgPre {
   double* w;          // 1/sqrt(diag)
   unsigned* barrier;  // grid barrier words of the coming k_jcg launch, cleared here
   int barrier_words;
+  unsigned long long* part;  // k_jcg_reg's partial slots, marked empty here
+  int part_words;
   int* flags;
   double* etas_prev;  // the previous step's ETAS (kept when keep_prev != 0)
   int warm;           // 1: start JCG from 2*ETAS - ETAS_prev instead of ETAS;
@@ -351,6 +367,12 @@ __global__ void k_jcg(JcgArgs a);
 // nsys systems in one launch: blocks first[m] .. first[m+1]-1 solve args[m]
 template <bool DUAL, bool STAGED>
 __global__ void k_jcg_batch(const JcgArgs* args, const int* first, int nsys);
+// the matrix in registers, one exchange per iteration (jcg_reg.hip): CPB
+// 2048-row chunks per 512-thread block
+template <bool DUAL, int CPB>
+__global__ void k_jcg_reg(JcgArgs a);
+template <bool DUAL, int CPB>
+__global__ void k_jcg_reg_batch(const JcgArgs* args, const int* first, int nsys);
 // more row tiles than blocks: the iterates in memory (a.uo, a.dpv, a.ndv)
 __global__ void k_jcg_mem(JcgArgs a);
 __global__ void k_wd_d1(DevMesh m, DevState s, int* flags, double h0, double habsmin);

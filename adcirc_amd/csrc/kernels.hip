@@ -248,7 +248,6 @@ __global__ __launch_bounds__(RED_THREADS) void k_lhs_rows(DevMesh m, DevState s,
                                                           const double* __restrict__ sb,
                                                           LhsTerms lt,
                                                           double* __restrict__ ep_part,
-                                                          const double* __restrict__ restore_cs,
                                                           const double* __restrict__ restore_w) {
   constexpr bool MIXED = sizeof(CT) == 4;
   __shared__ double lds[8];
@@ -261,17 +260,19 @@ __global__ __launch_bounds__(RED_THREADS) void k_lhs_rows(DevMesh m, DevState s,
   const int chunk = xcd_tile(blockIdx.x, gridDim.x);
   const int base = chunk * RED_CHUNK + t;
   if (flags[F_NCCHANGE] == 0) {
-    // no rebuild: the previous solve left the off-diagonals scaled; restore
-    // them as unscal does (src/itpackv.F:2460-2479), same operations
-    if (restore_cs)
+    // no rebuild: the previous solve left the off-diagonals as they were before
+    // its scaling; scale and unscale them as scal and unscal do
+    // (src/itpackv.F:2394-2400, 2460-2479), same operations
+    if (restore_w)
       for (int r = 0; r < RED_PER_THREAD; ++r) {
         const int i = base + RED_THREADS * r;
         if (i >= np) break;
         const int nn = m.nneigh[i];
-        const double ri = 1.0 / restore_w[i];
+        const double wi = restore_w[i], ri = 1.0 / wi;
         for (int j = 1; j < nn; ++j) {
           const size_t q = (size_t)j * np + i;
-          s.coef[q] = restore_cs[q] * ri * (1.0 / restore_w[m.col[q]]);
+          const double wj = restore_w[m.col[q]];
+          s.coef[q] = (s.coef[q] * wi * wj) * ri * (1.0 / wj);
         }
       }
     return;
@@ -365,10 +366,10 @@ __global__ __launch_bounds__(RED_THREADS) void k_lhs_rows(DevMesh m, DevState s,
   double tot = chunk_tree(acc, lds);
   if (t == 0) ep_part[chunk] = tot;
 }
-template __global__ void k_lhs_rows<false, double>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*, const double*);
-template __global__ void k_lhs_rows<true, double>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*, const double*);
-template __global__ void k_lhs_rows<false, float>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*, const double*);
-template __global__ void k_lhs_rows<true, float>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*, const double*);
+template __global__ void k_lhs_rows<false, double>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*);
+template __global__ void k_lhs_rows<true, double>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*);
+template __global__ void k_lhs_rows<false, float>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*);
+template __global__ void k_lhs_rows<true, float>(DevMesh, DevState, const int*, const double*, const double*, const double*, LhsTerms, double*, const double*);
 
 __global__ __launch_bounds__(256) void k_lhs_pair_setup(DevMesh m, LhsTerms lt,
                                                         const int* __restrict__ c1,
@@ -490,18 +491,18 @@ __device__ void lhs_bc_block(const DevMesh& m, DevState s, int nch,
   }
 }
 
-// The off-diagonals of a solve whose unscaling was deferred, restored as
-// unscal does (src/itpackv.F:2460-2479).
+// The off-diagonals of a solve whose unscaling was deferred, scaled and
+// unscaled as scal and unscal do (src/itpackv.F:2394-2400, 2460-2479).
 __global__ __launch_bounds__(256) void k_coef_restore(DevMesh m, DevState s,
-                                                      const double* __restrict__ cs,
                                                       const double* __restrict__ w) {
   const int i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (i >= m.np) return;
   const int np = m.np, nn = m.nneigh[i];
-  const double ri = 1.0 / w[i];
+  const double wi = w[i], ri = 1.0 / wi;
   for (int j = 1; j < nn; ++j) {
     const size_t q = (size_t)j * np + i;
-    s.coef[q] = cs[q] * ri * (1.0 / w[m.col[q]]);
+    const double wj = w[m.col[q]];
+    s.coef[q] = (s.coef[q] * wi * wj) * ri * (1.0 / wj);
   }
 }
 
@@ -870,6 +871,7 @@ __global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s, const C
   const int r0 = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x;
   const int i = r0 + threadIdx.x;
   if (i < pre.barrier_words) pre.barrier[i] = 0u;
+  if (i < pre.part_words) pre.part[i] = JCG_EMPTY;
   const int p0 = m.inc_ptr[r0];
   const int n_st = m.inc_ptr[min(r0 + (int)blockDim.x, m.np)] - p0;
   const bool staged = n_st <= NODE_STAGE;

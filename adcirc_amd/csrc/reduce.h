@@ -10,9 +10,39 @@
 
 namespace adcgpu {
 
+// A 64-bit value through a data-parallel-primitive lane permutation within
+// rows of 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// The xor butterfly over the 64 lanes (offsets 32, 16, 8, 4, 2, 1; every lane
+// active), in registers: permlane32/16_swap give the two halves of the first
+// two levels to both sides, then row rotations by 8 and 4 and quad
+// permutations (after the level of offset 8 a lane's value depends on its index
+// mod 8 only, so a rotation by 4 reads the partner of offset 4).  A lane adds
+// the same two values as the butterfly, so the result has the same bits.
+// Through LDS (ds_bpermute) the six levels cost about 0.35 us of the JCG
+// iteration's critical path, twice per iteration.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off, 64);
+  long long b = __double_as_longlong(v);
+  auto l32 = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+  auto h32 = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  v = __longlong_as_double(((long long)h32[0] << 32) | l32[0]) +
+      __longlong_as_double(((long long)h32[1] << 32) | l32[1]);
+  b = __double_as_longlong(v);
+  auto l16 = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+  auto h16 = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  v = __longlong_as_double(((long long)h16[0] << 32) | l16[0]) +
+      __longlong_as_double(((long long)h16[1] << 32) | l16[1]);
+  v = v + dpp_move<0x128>(v);  // row_ror:8
+  v = v + dpp_move<0x124>(v);  // row_ror:4
+  v = v + dpp_move<0x4e>(v);   // quad_perm:[2,3,0,1]
+  v = v + dpp_move<0xb1>(v);   // quad_perm:[1,0,3,2]
   return v;
 }
 
