@@ -14,6 +14,7 @@
 #include "jcg_host.h"
 #include "kernels.h"
 #include "mlp.h"
+#include "patch.h"
 
 using namespace adcgpu;
 
@@ -71,9 +72,8 @@ struct adcgpu_ctx {
   // mesh
   int *nm = nullptr, *inc_ptr = nullptr, *inc = nullptr, *slot = nullptr, *nneigh = nullptr;
   int *col = nullptr, *slot_cols = nullptr;
-  int *csrpos = nullptr, *bnd_index = nullptr, *nbd = nullptr, *obc_q = nullptr, *obc_s = nullptr;
-  int nobc = 0;
-  int *obcg_ptr = nullptr, *obcg = nullptr, *vbc_ptr = nullptr, *vbc = nullptr, *lbcodei = nullptr;
+  int *csrpos = nullptr, *bnd_index = nullptr, *nbd = nullptr;
+  int *obcg_ptr = nullptr, *obcg = nullptr, *obcg_q = nullptr, *vbc_ptr = nullptr, *vbc = nullptr, *lbcodei = nullptr;
   double *fdx = nullptr, *fdy = nullptr, *areas = nullptr, *x = nullptr, *y = nullptr, *dp = nullptr;
   double *tau0 = nullptr, *evm = nullptr, *corif = nullptr, *csii = nullptr, *siii = nullptr;
   // state (pointers rotate between time levels)
@@ -83,7 +83,7 @@ struct adcgpu_ctx {
   int *nodecode, *nnodecode, *noff, *noffold, *mju, *etamax_it, *umax_it;
   int cur_it = 0;  // step opened by adcgpu_begin_step
   // work
-  double *contrib = nullptr, *cx = nullptr, *cy = nullptr, *ep_part = nullptr, *scal = nullptr;
+  double *wd_area = nullptr, *ep_part = nullptr, *scal = nullptr;
   double *eta_bc = nullptr, *eta_bc_table = nullptr;
   int eta_bc_table_steps = 0;
   WdWork wd{};
@@ -128,22 +128,13 @@ struct adcgpu_ctx {
   int qn_table_steps = 0, qn_table_cap = 0;
   int64_t run_iters = 0, run_rebuilds = 0, run_itmax = 0, run_errstep = 0, run_mlused = 0;
   bool coef_scaled = false;  // off-diagonals of COEF left scaled by a deferred solve
-  // the GWCE matrix's unchanging terms per incidence slot, and each element's
-  // NCEle as the next rebuild sees it (written by the momentum element pass;
+  // the patches of the GWCE and momentum passes, and each patch element's
+  // NCEle as the next GWCE pass sees it (written by the momentum pass;
   // recomputed when the flags were changed otherwise)
-  double *lhs_td = nullptr, *lhs_ta = nullptr, *lhs_tb = nullptr;
+  DevPatch patch{};
   unsigned char* ncele = nullptr;
   bool ncele_fresh = false;
-  // mixed precision (ADCGPU_MIXED): FP32 element geometry and cached matrix
-  // terms; contrib, cx and cy then hold floats
-  bool mixed = false;
-  float *fdx32 = nullptr, *fdy32 = nullptr, *areas32 = nullptr;
-  float *lhs_td32 = nullptr, *lhs_ta32 = nullptr, *lhs_tb32 = nullptr;
-  // the cached terms per off-diagonal entry (k_lhs_pairs; ILump = 0)
-  bool lhs_pairs = false;
-  double *lp_t1 = nullptr, *lp_t2 = nullptr;
-  float *lp_t1f = nullptr, *lp_t2f = nullptr;
-  int *lp_e1 = nullptr, *lp_e2 = nullptr;
+  bool mixed = false;  // ADCGPU_MIXED
   // learned JCG start (set up on first use): FP32 master parameters and Adam
   // moments, the kernels' weight layouts, the per-step correction and second
   // start, training samples and the training work arrays
@@ -177,11 +168,10 @@ struct adcgpu_ctx {
     m.tau0 = tau0; m.evm = evm; m.corif = corif; m.inc_ptr = inc_ptr; m.inc = inc;
     m.slot = slot; m.slot_cols = slot_cols;
     m.nneigh = nneigh; m.col = col; m.csrpos = csrpos; m.bnd_index = bnd_index; m.nbd = nbd;
-    m.obc_q = obc_q; m.obc_s = obc_s; m.nobc = nobc; m.obcg_ptr = obcg_ptr; m.obcg = obcg; m.vbc_ptr = vbc_ptr;
+    m.obcg_ptr = obcg_ptr; m.obcg = obcg; m.obcg_q = obcg_q; m.vbc_ptr = vbc_ptr;
     m.vbc = vbc; m.lbcodei = lbcodei; m.csii = csii; m.siii = siii;
     m.fb_ptr = nfluxf ? fb_ptr : nullptr; m.fb_ent = nfluxf ? fb_ent : nullptr;
     m.nbv = nfluxf ? nbv0 : nullptr; m.bndlen = nfluxf ? bndlen : nullptr;
-    m.fdx32 = fdx32; m.fdy32 = fdy32; m.areas32 = areas32;
     return m;
   }
   DevState state() const {
@@ -385,6 +375,36 @@ int launch_jcg(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh, d
   HIPCHK(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(threads), args, (unsigned)lds, c->stream));
   if (c->profile) HIPCHK(hipEventRecord(c->jcg_events[c->ev_used++].second, c->stream));
   return 0;
+}
+
+// The device's part of the patch plan: each own row's edge codes (left out if
+// some edge has more than two elements), and the element geometry where the
+// coordinates do not give it bit for bit.
+int patch_setup(adcgpu_ctx* c) {
+  DevPatch& pp = c->patch;
+  unsigned* pair = nullptr;
+  double* geo = nullptr;
+  if (c->prm.ilump == 0) {
+    if (int rc = dmalloc(&pair, (size_t)pp.n * (c->mnei - 1) * PATCH_NODES)) return rc;
+    c->allocs.push_back(pair);
+  }
+  // two words of the flags serve as the answers
+  hipLaunchKernelGGL(k_patch_check, dim3(nblk(std::max(pp.n * PATCH_NODES, c->ne), 256)),
+                     dim3(256), 0, c->stream, c->mesh(), pp, pair, c->flags + F_NUMITR);
+  int f[2] = {0, 0};
+  HIPCHK(hipMemcpyAsync(f, c->flags + F_NUMITR, sizeof(f), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  if (f[0] == 0) pp.pair = pair;
+  if (f[1] != 0) {
+    if (int rc = dmalloc(&geo, 7 * (size_t)pp.nq)) return rc;
+    c->allocs.push_back(geo);
+    hipLaunchKernelGGL(k_patch_geo, dim3(nblk(pp.nq, 256)), dim3(256), 0, c->stream, c->mesh(), pp,
+                       geo);
+    pp.geo = geo;
+  }
+  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_NUMITR, 0, 2);
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return check_launch("patch set-up");
 }
 
 // ---------------------------------------------------------------- learned start
@@ -648,8 +668,9 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     bnd_index[b] = I;
     nbd0[I] = b;
   }
-  std::vector<int> obc_slot((size_t)mnei * np, -1);
-  std::vector<std::vector<int>> obcl(np);
+  // the COEF positions that couple row i to an elevation-boundary node, with
+  // their OBCCOEF slots I*mnei+(J-2)
+  std::vector<std::vector<std::pair<int, int>>> obcl(np);
   for (int I = 0; I < neta; ++I) {
     int b = nbd0[I];
     for (int J = 2; J <= nneigh[b]; ++J) {
@@ -657,31 +678,19 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
       int found = 0;
       for (int IJ = 2; IJ <= nneigh[nb]; ++IJ)
         if (col[(size_t)(IJ - 1) * np + nb] == b) {
-          obc_slot[(size_t)(IJ - 1) * np + nb] = I * mnei + (J - 2);
+          obcl[nb].emplace_back(I * mnei + (J - 2), (IJ - 1) * np + nb);
           ++found;
         }
       if (found != 1) return fail(ADCGPU_E_ARG, "asymmetric neighbour table at a boundary");
-      obcl[nb].push_back(I * mnei + (J - 2));
     }
   }
-  // the COEF positions that involve a boundary node, for the matrix's boundary pass
-  std::vector<int> obc_q, obc_s;
-  for (int j = 1; j < mnei; ++j)
-    for (int i = 0; i < np; ++i) {
-      const int sl = obc_slot[(size_t)j * np + i];
-      if (sl < 0) continue;
-      obc_q.push_back(j * np + i);
-      obc_s.push_back(bnd_index[i] >= 0 ? -1 - sl : sl);
-    }
-  const int nobc = (int)obc_q.size();
-  if (obc_q.empty()) {  // device arrays of at least one element
-    obc_q.push_back(0);
-    obc_s.push_back(0);
-  }
-  std::vector<int> obcg_ptr(np + 1, 0), obcg;
+  std::vector<int> obcg_ptr(np + 1, 0), obcg, obcg_q;
   for (int i = 0; i < np; ++i) {
     obcg_ptr[i + 1] = obcg_ptr[i] + (int)obcl[i].size();
-    obcg.insert(obcg.end(), obcl[i].begin(), obcl[i].end());
+    for (const auto& o : obcl[i]) {
+      obcg.push_back(o.first);
+      obcg_q.push_back(o.second);
+    }
   }
   std::vector<std::vector<int>> vbl(np);
   std::vector<int> lbc(std::max(M->nvel, 1), 0);
@@ -713,6 +722,10 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     if (!(M->areas[e] > 0.0))
       return fail(ADCGPU_E_ARG, "element " + std::to_string(e + 1) + " has a non-positive AREAS");
 
+  const PatchPlan plan = patch_plan(np, ne, nm0, cnt, inc, M->x, M->y);
+  if (!plan.ok)
+    return fail(ADCGPU_E_UNSUPPORTED, "a node with more than " + std::to_string(PATCH_ELEMS) +
+                                          " elements");
   adcgpu_ctx* c = new adcgpu_ctx();
   c->device = device;
   c->np = np; c->ne = ne; c->mnei = mnei; c->neta = neta;
@@ -773,8 +786,7 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   U(&c->nm, nm0); U(&c->inc_ptr, cnt); U(&c->inc, inc); U(&c->slot, slot); U(&c->slot_cols, slot_cols); U(&c->nneigh, nneigh); U(&c->col, col);
   U(&c->jhrange, hrange);
   if (!lcol.empty()) U(&c->jlcol, lcol);
-  U(&c->csrpos, csrpos); U(&c->bnd_index, bnd_index); U(&c->nbd, nbd0); U(&c->obc_q, obc_q);
-  U(&c->obc_s, obc_s); c->nobc = nobc;
+  U(&c->csrpos, csrpos); U(&c->bnd_index, bnd_index); U(&c->nbd, nbd0);
   c->nvel = M->nvel;
   for (int I = 0; I < M->nvel; ++I) {
     c->has_rad = c->has_rad || lbc[I] == 30 || lbc[I] == 52;
@@ -782,7 +794,7 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   }
   c->h_nbv = h_nbv;
   c->h_bnd_index = bnd_index;
-  U(&c->obcg_ptr, obcg_ptr); U(&c->obcg, obcg); U(&c->vbc_ptr, vbc_ptr); U(&c->vbc, vbc);
+  U(&c->obcg_ptr, obcg_ptr); U(&c->obcg, obcg); U(&c->obcg_q, obcg_q); U(&c->vbc_ptr, vbc_ptr); U(&c->vbc, vbc);
   U(&c->lbcodei, lbc); U(&c->fdx, fdx); U(&c->fdy, fdy); U(&c->areas, var); U(&c->x, vx);
   U(&c->y, vy); U(&c->dp, vdp); U(&c->tau0, vt); U(&c->evm, ve); U(&c->corif, vcor);
   U(&c->csii, csii); U(&c->siii, siii); U(&c->fric, vfric);
@@ -801,21 +813,21 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   A(&c->nodecode, np); A(&c->nnodecode, np); A(&c->noff, ne); A(&c->noffold, ne);
   A(&c->mju, np); A(&c->etamax_it, np); A(&c->etas_prev, np);
   A(&c->umax, np); A(&c->umax_it, np);
-  A(&c->contrib, 3 * (size_t)ne); A(&c->cx, 3 * (size_t)ne); A(&c->cy, 3 * (size_t)ne);
-  A(&c->lhs_td, 3 * (size_t)ne); A(&c->lhs_ta, 3 * (size_t)ne); A(&c->lhs_tb, 3 * (size_t)ne);
-  A(&c->ncele, ne);
+  A(&c->wd_area, 3 * (size_t)ne);
   c->mixed = P->precision == ADCGPU_MIXED;
-  if (c->mixed) {
-    std::vector<float> f32(3 * (size_t)ne);
-    for (size_t k = 0; k < f32.size(); ++k) f32[k] = (float)fdx[k];
-    U(&c->fdx32, f32);
-    for (size_t k = 0; k < f32.size(); ++k) f32[k] = (float)fdy[k];
-    U(&c->fdy32, f32);
-    f32.resize(ne);
-    for (int e = 0; e < ne; ++e) f32[e] = (float)var[e];
-    U(&c->areas32, f32);
-    A(&c->lhs_td32, 3 * (size_t)ne); A(&c->lhs_ta32, 3 * (size_t)ne);
-    A(&c->lhs_tb32, 3 * (size_t)ne);
+  {
+    DevPatch& pp = c->patch;
+    pp.n = plan.n;
+    pp.nq = (int)plan.el.size();
+    pp.wmax = plan.wmax;
+    auto UP = [&](auto& dst, const auto& v) {  // into a const member
+      std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(dst)>>>* d = nullptr;
+      U(&d, v);
+      dst = d;
+    };
+    UP(pp.win, plan.win); UP(pp.el, plan.el); UP(pp.lv, plan.lv);
+    UP(pp.cspan, plan.cspan); UP(pp.code, plan.code);
+    A(&c->ncele, (size_t)pp.nq);
   }
   A(&c->ep_part, c->nch); A(&c->scal, S_COUNT); A(&c->eta_bc, std::max(neta, 1));
   {
@@ -836,17 +848,21 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   }
   if (!rc) rc = setup_jcg_grid(c);
   if (!rc) {
-    // the LHS row kernel keeps MNEI x 512 doubles of LDS per block; the
-    // wetting propagation stages candidates through LDS
+    // the patch passes' windows; the wetting propagation stages candidates
+    // through LDS
     hipError_t e = hipSuccess;
-    const void* rows_fns[] = {(const void*)k_lhs_rows<false, double>,
-                              (const void*)k_lhs_rows<true, double>,
-                              (const void*)k_lhs_rows<false, float>,
-                              (const void*)k_lhs_rows<true, float>};
-    for (const void* fn : rows_fns)
+    const void* gwce_fns[] = {(const void*)k_gwce<false, double>, (const void*)k_gwce<true, double>,
+                              (const void*)k_gwce<false, float>, (const void*)k_gwce<true, float>};
+    const void* mom_fns[] = {(const void*)k_mom<false, double>, (const void*)k_mom<true, double>,
+                             (const void*)k_mom<false, float>, (const void*)k_mom<true, float>};
+    for (const void* fn : gwce_fns)
       if (e == hipSuccess)
         e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                mnei * RED_THREADS * (int)sizeof(double));
+                                patch_lds_bytes(PATCH_GWCE_FIELDS, PATCH_GWCE_TERMS, PATCH_WIN));
+    for (const void* fn : mom_fns)
+      if (e == hipSuccess)
+        e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                patch_lds_bytes(PATCH_MOM_FIELDS, PATCH_MOM_TERMS, PATCH_WIN));
     if (e == hipSuccess)
       e = hipFuncSetAttribute((const void*)k_wd_link, hipFuncAttributeMaxDynamicSharedMemorySize,
                               WD_LINK_LDS);
@@ -869,63 +885,11 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     int f[F_COUNT] = {0};
     f[F_NCCHANGE] = 1;
     (void)hipMemcpy(c->flags, f, sizeof(f), hipMemcpyHostToDevice);
-    // the GWCE matrix's unchanging terms, once
-    if (P->ilump != 0)
-      hipLaunchKernelGGL(k_lhs_terms<true>, dim3(nblk(ne, 256)), dim3(256), 0, c->stream,
-                         c->mesh(), c->lhs_td, c->lhs_ta, c->lhs_tb, c->lhs_td32, c->lhs_ta32,
-                         c->lhs_tb32);
-    else
-      hipLaunchKernelGGL(k_lhs_terms<false>, dim3(nblk(ne, 256)), dim3(256), 0, c->stream,
-                         c->mesh(), c->lhs_td, c->lhs_ta, c->lhs_tb, c->lhs_td32, c->lhs_ta32,
-                         c->lhs_tb32);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) rc = fail(ADCGPU_E_HIP, hipGetErrorString(e));
   }
-  if (!rc && P->ilump == 0) {
-    // the terms per off-diagonal entry: slot p's ta term goes to column ja,
-    // its tb term to jb, in ascending element order; more than two
-    // contributions to one entry (a non-manifold edge) keep the row pass
-    const size_t nq = (size_t)(mnei - 1) * np;
-    std::vector<int> pc1(nq, -1), pc2(nq, -1);
-    bool ok = true;
-    for (int i = 0; i < np && ok; ++i)
-      for (int p = cnt[i]; p < cnt[i + 1] && ok; ++p) {
-        const int jj[2] = {slot_cols[p] & 0xffff, slot_cols[p] >> 16};
-        for (int w = 0; w < 2; ++w) {
-          const size_t q = (size_t)(jj[w] - 1) * np + i;
-          const int code = 2 * p + w;
-          if (pc1[q] < 0) pc1[q] = code;
-          else if (pc2[q] < 0) pc2[q] = code;
-          else ok = false;
-        }
-      }
-    if (ok) {
-      // the codes are needed only here: uploaded outside the context's list
-      // of allocations and freed below
-      int *d1 = nullptr, *d2 = nullptr;
-      if (!rc) rc = upload(&d1, pc1);
-      if (!rc) rc = upload(&d2, pc2);
-      if (c->mixed) {
-        A(&c->lp_t1f, nq); A(&c->lp_t2f, nq);
-      } else {
-        A(&c->lp_t1, nq); A(&c->lp_t2, nq);
-      }
-      A(&c->lp_e1, nq); A(&c->lp_e2, nq);
-      if (!rc) {
-        const LhsTerms lt{c->lhs_td, c->lhs_ta, c->lhs_tb, c->lhs_td32, c->lhs_ta32, c->lhs_tb32, 0};
-        hipLaunchKernelGGL(k_lhs_pair_setup, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0,
-                           c->stream, c->mesh(), lt, (const int*)d1, (const int*)d2, c->lp_t1,
-                           c->lp_t2, c->lp_t1f, c->lp_t2f, c->lp_e1, c->lp_e2);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e != hipSuccess) rc = fail(ADCGPU_E_HIP, hipGetErrorString(e));
-        c->lhs_pairs = rc == 0;
-      }
-      if (d1) (void)hipFree(d1);
-      if (d2) (void)hipFree(d2);
-    }
-  }
+  if (!rc) rc = patch_setup(c);
   if (!rc && P->warm_start == 2) rc = ml_setup(c);
   if (rc) {
     adcgpu_destroy(c);
@@ -1187,66 +1151,28 @@ struct GwceStep {
 // The GWCE assembly up to the solve: matrix, right-hand side, time-level
 // rotation, the learned start's inputs, and the node pass that scales the
 // rows for JCG (or, with ILump = 1, solves).
-static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, GwceStep* g) {
-  const int np = c->np, ne = c->ne;
+static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceStep* g) {
+  const int np = c->np;
   const bool lumped = c->prm.ilump != 0;
-  const size_t rows_lds = (size_t)c->mnei * RED_THREADS * sizeof(double);
   const double* rw = c->coef_scaled ? (const double*)c->jw : nullptr;
-  // a rebuild multiplies the cached terms by each element's NCEle, which the
-  // momentum element pass left unless the flags changed since
+  // the passes multiply each element's terms by its NCEle, which the momentum
+  // pass left unless the flags changed since
   if (!c->ncele_fresh) {
-    hipLaunchKernelGGL(k_ncele, dim3(nblk(ne, 256)), dim3(256), 0, c->stream, c->mesh(),
-                       c->state());
+    hipLaunchKernelGGL(k_ncele, dim3(nblk(c->patch.nq, 256)), dim3(256), 0, c->stream, c->mesh(),
+                       c->state(), c->patch);
     c->ncele_fresh = true;
   }
-  const LhsTerms lt{c->lhs_td,   c->lhs_ta,   c->lhs_tb,       c->lhs_td32,
-                    c->lhs_ta32, c->lhs_tb32, c->lhs_pairs ? 1 : 0};
-  // contrib, cx and cy are free until the GWCE right-hand side
-  if (!lumped)  // the element pass only runs while some ALPHAL differs from 1
-    hipLaunchKernelGGL(k_lhs_elem<false>, dim3(nblk(ne, 256)), dim3(256), 0, c->stream,
-                       c->mesh(), c->state(), c->flags, c->contrib, c->cx, c->cy);
-  const dim3 rg(c->nch), rb(RED_THREADS);
-  if (c->mixed) {
-    if (lumped)
-      hipLaunchKernelGGL((k_lhs_rows<true, float>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
-    else
-      hipLaunchKernelGGL((k_lhs_rows<false, float>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
-  } else {
-    if (lumped)
-      hipLaunchKernelGGL((k_lhs_rows<true, double>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
-    else
-      hipLaunchKernelGGL((k_lhs_rows<false, double>), rg, rb, rows_lds, c->stream, c->mesh(),
-                         c->state(), c->flags, c->contrib, c->cx, c->cy, lt, c->ep_part, rw);
-  }
-  if (c->lhs_pairs) {
-    // the cached rebuild (k_lhs_rows above only restored or left at once)
-    const LhsPairs lp{c->lp_t1, c->lp_t2, c->lp_t1f, c->lp_t2f, c->lp_e1, c->lp_e2};
-    const dim3 pg(nblk(np, 256), c->mnei);
-    if (c->mixed)
-      hipLaunchKernelGGL(k_lhs_pairs<float>, pg, dim3(256), 0, c->stream, c->mesh(), c->state(),
-                         (const int*)c->flags, lt, lp);
-    else
-      hipLaunchKernelGGL(k_lhs_pairs<double>, pg, dim3(256), 0, c->stream, c->mesh(), c->state(),
-                         (const int*)c->flags, lt, lp);
-    hipLaunchKernelGGL(k_lhs_ep, rg, rb, 0, c->stream, c->mesh(), c->state(),
-                       (const int*)c->flags, c->ep_part);
-  }
+  const RhsPrm q{c->ifnlfa, c->ifnlct, c->ifnlcat, lumped ? 4.0 : 2.0, lumped ? 0.0 : 1.0,
+                 fric ? 1 : 0, c->prm.nws};
+  const dim3 pg(c->patch.n), pb(PATCH_THREADS);
+  const size_t lds = patch_lds_bytes(PATCH_GWCE_FIELDS, PATCH_GWCE_TERMS, c->patch.wmax);
+  auto gwce = lumped ? (c->mixed ? k_gwce<true, float> : k_gwce<true, double>)
+                     : (c->mixed ? k_gwce<false, float> : k_gwce<false, double>);
+  hipLaunchKernelGGL(gwce, pg, pb, lds, c->stream, c->mesh(), c->state(), c->patch, q, fric_prm(c),
+                     (const int*)c->flags, rw);
   c->coef_scaled = false;
-  RhsPrm q{c->ifnlfa, c->ifnlct, c->ifnlcat, lumped ? 4.0 : 2.0, lumped ? 0.0 : 1.0,
-           lumped ? 1 : 0, c->prm.nws};
-  // its last block finishes the matrix (EP, elevation-boundary rows) and
-  // clears NCChange
-  static_assert(RED_XTHREADS == 256, "the matrix-finishing block is a 256-thread block");
-  float* contrib32 = reinterpret_cast<float*>(c->contrib);
-  if (c->mixed)
-    hipLaunchKernelGGL(k_rhs_elem32, dim3(nblk(ne, 256) + 1), dim3(256), 0, c->stream, c->mesh(),
-                       c->state(), q, c->flags, contrib32, c->nch, c->ep_part, c->scal);
-  else
-    hipLaunchKernelGGL(k_rhs_elem, dim3(nblk(ne, 256) + 1), dim3(256), 0, c->stream, c->mesh(),
-                       c->state(), q, c->flags, c->contrib, c->nch, c->ep_part, c->scal);
+  hipLaunchKernelGGL(k_lhs_ep, dim3(c->nch), dim3(RED_THREADS), 0, c->stream, c->mesh(),
+                     c->state(), c->flags, c->ep_part);
   // ETA1 <- ETA2, H1 <- H2 (src/gwce.F:1622-1631) by rotation
   std::swap(c->eta1, c->eta2);
   std::swap(c->h1, c->h2);
@@ -1266,23 +1192,11 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, GwceStep* g) {
              reinterpret_cast<unsigned long long*>(c->jpart), jcg_part_doubles(c->nch),
              c->flags, c->etas_prev, c->prm.warm_start,
              (c->prm.warm_start != 0 || c->ml_ready) ? 1 : 0, c->ml_corr, c->ml_u};
-  const dim3 ng(nblk(np, 256)), nbk(256);
   // with ILump = 1 the explicit solve of the lumped GWCE ends the node pass; no JCG
-  if (c->mixed) {
-    if (lumped)
-      hipLaunchKernelGGL((k_rhs_node<true, float>), ng, nbk, 0, c->stream, c->mesh(), c->state(),
-                         (const float*)contrib32, d_eta_bc, c->scal, pre);
-    else
-      hipLaunchKernelGGL((k_rhs_node<false, float>), ng, nbk, 0, c->stream, c->mesh(), c->state(),
-                         (const float*)contrib32, d_eta_bc, c->scal, pre);
-  } else {
-    if (lumped)
-      hipLaunchKernelGGL((k_rhs_node<true, double>), ng, nbk, 0, c->stream, c->mesh(), c->state(),
-                         (const double*)c->contrib, d_eta_bc, c->scal, pre);
-    else
-      hipLaunchKernelGGL((k_rhs_node<false, double>), ng, nbk, 0, c->stream, c->mesh(),
-                         c->state(), (const double*)c->contrib, d_eta_bc, c->scal, pre);
-  }
+  static_assert(RED_XTHREADS == 256, "the node pass forms EP with its 256 threads");
+  hipLaunchKernelGGL(lumped ? k_rhs_node<true> : k_rhs_node<false>, dim3(nblk(np, 256)), dim3(256),
+                     0, c->stream, c->mesh(), c->state(), d_eta_bc, c->nch,
+                     (const double*)c->ep_part, c->scal, pre);
   g->solve = !lumped;
   g->learned = learned;
   g->collect = collect;
@@ -1309,9 +1223,9 @@ static int gwce_finish(adcgpu_ctx* c, const GwceStep& g, bool deferred) {
   return check_launch("training samples");
 }
 
-static int gwce_device(adcgpu_ctx* c, const double* d_eta_bc, bool deferred) {
+static int gwce_device(adcgpu_ctx* c, const double* d_eta_bc, bool deferred, bool fric) {
   GwceStep g;
-  int rc = gwce_assemble(c, d_eta_bc, &g);
+  int rc = gwce_assemble(c, d_eta_bc, fric, &g);
   if (!rc && g.solve)
     rc = launch_jcg(c, c->coef, c->col, c->nneigh, c->gwce_lv, c->etas, c->np, c->prm.itmax,
                     c->prm.convcr, c->eta2, c->eta1, c->nodecode, true, deferred,
@@ -1329,15 +1243,19 @@ static int restore_coef(adcgpu_ctx* c) {
   return check_launch("coef restore");
 }
 
-int adcgpu_solve_gwce(adcgpu_ctx* c, int it, const double* eta_bc) {
-  (void)it;
-  if (!c) return fail(ADCGPU_E_ARG, "null context");
+static int solve_gwce(adcgpu_ctx* c, const double* eta_bc, bool fric) {
   if (c->neta > 0) {
     if (!eta_bc) return fail(ADCGPU_E_ARG, "eta_bc required");
     HIPCHK(hipMemcpyAsync(c->eta_bc, eta_bc, c->neta * sizeof(double), hipMemcpyHostToDevice,
                           c->stream));
   }
-  return gwce_device(c, c->eta_bc, false);
+  return gwce_device(c, c->eta_bc, false, fric);
+}
+
+int adcgpu_solve_gwce(adcgpu_ctx* c, int it, const double* eta_bc) {
+  (void)it;
+  if (!c) return fail(ADCGPU_E_ARG, "null context");
+  return solve_gwce(c, eta_bc, false);
 }
 
 // Wet/dry; without `alpha_pass` the ALPHAL pass is left to the momentum
@@ -1356,7 +1274,7 @@ static int wetdry_device(adcgpu_ctx* c, bool alpha_pass) {
   WdPrm q{c->hoff, c->prm.velmin, c->iflinbf, c->ifnlbf, c->tkmax, c->hyb};
   const int nb = nblk(ne, 256);
   hipLaunchKernelGGL(k_wd_elem, dim3(nb), dim3(256), 0, c->stream, c->mesh(), c->state(), q,
-                     c->wd);
+                     c->wd, c->flags);
   hipLaunchKernelGGL(k_wd_index, dim3(1), dim3(1024), 0, c->stream, c->wd.bcnt, nb, c->wd.bofs,
                      c->flags);
   hipLaunchKernelGGL(k_wd_pred, dim3(nb), dim3(256), 0, c->stream, c->mesh(), c->state(), c->wd);
@@ -1365,11 +1283,11 @@ static int wetdry_device(adcgpu_ctx* c, bool alpha_pass) {
                      c->flags);
   hipLaunchKernelGGL(k_wd_link, dim3(1), dim3(256), WD_LINK_LDS, c->stream, c->wd, c->flags,
                      c->tk);
-  // cx is free until the momentum step: it holds NCEle*AREAS/2 per incidence slot
+  // NCEle*AREAS/2 per incidence slot
   hipLaunchKernelGGL(k_wd_final_area, dim3(nblk(ne, 256)), dim3(256), 0, c->stream, c->mesh(),
-                     c->state(), c->wd, c->flags, c->tk, c->cx);
+                     c->state(), c->wd, c->flags, c->tk, c->wd_area);
   hipLaunchKernelGGL(k_wd_d2, dim3(nblk(np, 256)), dim3(256), 0, c->stream, c->mesh(),
-                     c->state(), c->cx, c->flags, c->ifnlfa);
+                     c->state(), c->wd_area, c->flags, c->ifnlfa);
   if (alpha_pass)
     hipLaunchKernelGGL(k_wd_alpha, dim3(nblk(ne, 256)), dim3(256), 0, c->stream, c->mesh(),
                        c->state(), c->flags, 1.0e9);
@@ -1382,31 +1300,14 @@ int adcgpu_wetdry(adcgpu_ctx* c, int it) {
   return wetdry_device(c, true);
 }
 
-// Momentum; with `alpha` the element pass forms ALPHAL first.
+// Momentum; with `alpha` the pass forms ALPHAL first.
 static int momentum_device(adcgpu_ctx* c, bool alpha) {
   MomPrm q{c->ifnlct, c->prm.nws, c->cur_it, c->errorelev, c->flags};
-  const dim3 eg(nblk(c->ne, 256)), ng(nblk(c->np, 256)), bk(256);
-  if (c->mixed) {
-    float* cx32 = reinterpret_cast<float*>(c->cx);
-    float* cy32 = reinterpret_cast<float*>(c->cy);
-    if (alpha)
-      hipLaunchKernelGGL(k_mom_elem32<true>, eg, bk, 0, c->stream, c->mesh(), c->state(), q, cx32,
-                         cy32, c->flags);
-    else
-      hipLaunchKernelGGL(k_mom_elem32<false>, eg, bk, 0, c->stream, c->mesh(), c->state(), q,
-                         cx32, cy32, c->flags);
-    hipLaunchKernelGGL(k_mom_node<float>, ng, bk, 0, c->stream, c->mesh(), c->state(), q,
-                       (const float*)cx32, (const float*)cy32);
-  } else {
-    if (alpha)
-      hipLaunchKernelGGL(k_mom_elem<true>, eg, bk, 0, c->stream, c->mesh(), c->state(), q, c->cx,
-                         c->cy, c->flags);
-    else
-      hipLaunchKernelGGL(k_mom_elem<false>, eg, bk, 0, c->stream, c->mesh(), c->state(), q,
-                         c->cx, c->cy, c->flags);
-    hipLaunchKernelGGL(k_mom_node<double>, ng, bk, 0, c->stream, c->mesh(), c->state(), q,
-                       (const double*)c->cx, (const double*)c->cy);
-  }
+  auto mom = alpha ? (c->mixed ? k_mom<true, float> : k_mom<true, double>)
+                   : (c->mixed ? k_mom<false, float> : k_mom<false, double>);
+  hipLaunchKernelGGL(mom, dim3(c->patch.n), dim3(PATCH_THREADS),
+                     patch_lds_bytes(PATCH_MOM_FIELDS, PATCH_MOM_TERMS, c->patch.wmax), c->stream,
+                     c->mesh(), c->state(), c->patch, q);
   c->ncele_fresh = true;
   return check_launch("momentum");
 }
@@ -1418,12 +1319,13 @@ int adcgpu_momentum(adcgpu_ctx* c) {
 
 int adcgpu_timestep(adcgpu_ctx* c, int it, const double* eta_bc, const double* wsx2,
                     const double* wsy2, const double* pr2) {
+  // friction in the GWCE pass, ALPHAL in the momentum pass
+  const bool wd = c && c->prm.nolifa == 2;
   int rc = adcgpu_begin_step(c, it);
-  if (!rc) rc = adcgpu_friction(c);
   if (!rc && c->prm.nws != 0) rc = adcgpu_set_forcing(c, wsx2, wsy2, pr2);
-  if (!rc) rc = adcgpu_solve_gwce(c, it, eta_bc);
-  if (!rc) rc = adcgpu_wetdry(c, it);
-  if (!rc) rc = adcgpu_momentum(c);
+  if (!rc) rc = solve_gwce(c, eta_bc, true);
+  if (!rc) rc = wetdry_device(c, !wd);
+  if (!rc) rc = momentum_device(c, wd);
   return rc;
 }
 
@@ -1478,26 +1380,22 @@ static int run_prepare(adcgpu_ctx* c, int nsteps, const double* eta_bc_table,
   return check_launch("run set-up");
 }
 
-// A resident step up to the GWCE solve: begin, friction (with this step's
-// Holland forcing in the same pass), the assembly.
+// A resident step up to the GWCE solve: begin, this step's Holland forcing, the
+// assembly (with friction).
 static int run_step_assemble(adcgpu_ctx* c, int it, int s, const double* holland, GwceStep* g) {
   const bool rows = c->nfluxf && c->qn_table_steps > s;
   int rc = begin_step(c, it, rows ? c->qn_table + (size_t)s * c->nvel : nullptr);
-  if (!rc) {
-    if (holland) {
-      // friction and this step's forcing in one pass
-      HollandPrm hp;
-      for (int k = 0; k < 13; ++k) hp.v[k] = holland[k];
-      hp.t = it * c->prm.dtdp;
-      hipLaunchKernelGGL(k_friction_holland, dim3(nblk(c->np, 256)), dim3(256), 0, c->stream,
-                         c->np, fric_prm(c), c->tk, c->x, c->y, hp, c->wsx2, c->wsy2, c->pr2);
-      rc = check_launch("friction and forcing");
-    } else {
-      rc = adcgpu_friction(c);
-    }
+  if (!rc && holland) {
+    HollandPrm hp;
+    for (int k = 0; k < 13; ++k) hp.v[k] = holland[k];
+    hp.t = it * c->prm.dtdp;
+    hipLaunchKernelGGL(k_holland, dim3(nblk(c->np, 256)), dim3(256), 0, c->stream, c->np, c->x,
+                       c->y, hp, c->wsx2, c->wsy2, c->pr2);
+    rc = check_launch("forcing");
   }
   if (!rc)
-    rc = gwce_assemble(c, c->neta > 0 ? c->eta_bc_table + (size_t)s * c->neta : c->eta_bc, g);
+    rc = gwce_assemble(c, c->neta > 0 ? c->eta_bc_table + (size_t)s * c->neta : c->eta_bc,
+                       true, g);
   return rc;
 }
 

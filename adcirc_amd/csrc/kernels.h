@@ -34,6 +34,16 @@ __host__ __device__ constexpr int jcg_part_doubles(int nch) { return 4 * 4 * (nc
 constexpr int JCG_STAGE_MAX_BYTES = 120 * 1024;
 static_assert(JCG_STAGE_MAX_BYTES / 8 <= 65536, "staged positions are 16-bit");
 constexpr int NODE_STAGE = 2048;   // incidence slots a 256-node block stages in LDS
+// patches: a block's threads, and at most so many elements (one per thread),
+// window nodes, and own nodes.  About 10 x 10 nodes have 235 elements: one per
+// thread, and a sixth more element evaluations than the mesh has elements.
+constexpr int PATCH_THREADS = 256, PATCH_ELEMS = 256, PATCH_WIN = 192, PATCH_NODES = 96;
+static_assert(PATCH_NODES <= PATCH_THREADS / 2 && PATCH_WIN <= PATCH_THREADS, "patch shape");
+constexpr int PATCH_GWCE_FIELDS = 18, PATCH_MOM_FIELDS = 13;
+constexpr int patch_lds_bytes(int fields, int terms, int wmax) {
+  return 8 * (fields * wmax > terms ? fields * wmax : terms);
+}
+constexpr int PATCH_GWCE_TERMS = 9 * PATCH_ELEMS + 1, PATCH_MOM_TERMS = 6 * PATCH_ELEMS;
 constexpr int LHS_MAXW = 32;         // widest COEF row (MNEI): LDS of the row kernel
 // ordered wetting updates: candidates are closed in blocks of WD_BLOCK, each
 // block naming at most WD_XMAX earlier candidates it depends on
@@ -56,9 +66,11 @@ constexpr int WD_LINK_LDS = WD_LINK_BLOCKS * WD_XMAX * 8 > WD_SERIAL_LDS
 enum { F_NCCHANGE = 0, F_NUMITR = 2, F_IER, F_ERROR, F_NCAND, F_ITSUM, F_NREBUILD, F_WDSERIAL,
        F_ERRSTEP,  // first step that raised ERR_ELEV or ERR_NONFINITE (0: none)
        F_NITMAX,   // solves that reached ITMAX (ier = 13)
-       F_ALPHA,    // some element's ALPHAL differs from 1 (the cached matrix
-                   // terms assume ALPHAL = 1; the element pass recomputes them)
+       F_ALPHA,    // some element's ALPHAL differs from 1 (otherwise the passes
+                   // that use it do not read it)
        F_MLUSED,   // solves that started from the learned guess
+       F_REBUILT,  // this step's GWCE matrix was rebuilt (k_lhs_ep)
+       F_ALPHA0,   // F_ALPHA as the last step left it
        F_COUNT = 16 };
 enum { ERR_DIAG = 1, ERR_BARRIER = 4, ERR_ELEV = 8, ERR_NONFINITE = 16 };
 // device scalar slots
@@ -87,12 +99,9 @@ struct DevMesh {
   const int* bnd_index; // [np] elevation-boundary index, -1, or -2-k for the
                         //      k-th node that takes specified-flux edge terms
   const int* nbd;       // [neta] 0-based
-  const int* obc_q;     // [nobc] COEF positions j*np+i that couple row i to an
-  const int* obc_s;     //        elevation-boundary node, and their OBCCOEF slot
-                        //        I*mnei+(J-2); -1-slot when row i is itself a boundary row
-  int nobc;
   const int* obcg_ptr;  // [np+1] node -> boundary-column slots, (I,J) order
   const int* obcg;
+  const int* obcg_q;    //        and the COEF position j*np+i of each
   const int* vbc_ptr;   // [np+1] node -> flow-boundary entries in ME2GW order
   const int* vbc;
   const int* lbcodei;
@@ -106,10 +115,6 @@ struct DevMesh {
   const int* fb_ent;
   const int* nbv;       // [nvel] 0-based
   const double* bndlen; // [nvel] BNDLEN2O3
-  // mixed precision: FP32 copies of the element geometry (null in FP64 runs)
-  const float* fdx32;
-  const float* fdy32;
-  const float* areas32;
 };
 
 struct DevState {
@@ -120,7 +125,7 @@ struct DevState {
   int *etamax_it;  // step of the last ETAMAX rise (0: never)
   double *umax;    // peak depth-averaged speed at wet nodes
   int *umax_it;    // step of the last UMAX rise (0: never)
-  unsigned char* ncele;  // [ne] NCEle of each element for the next GWCE matrix
+  unsigned char* ncele;  // [nq] NCEle of each patch element (DevPatch) for the next GWCE
   double *tip1, *tip2;   // tidal potential at time levels s and s+1 (null: none)
   double *qn0, *qn1, *qn2;  // normal flux per flow-boundary entry at three time
                             // levels (null: no flux boundaries)
@@ -142,26 +147,40 @@ struct TipPrm {
   double argt[TIP_MAX], tpmul[TIP_MAX];
 };
 
-// The GWCE matrix terms of every (element, vertex) slot that do not change
-// from step to step (geometry, depth, Tau0, ALPHAL = 1), kept in slot order;
-// a rebuild multiplies them by the element's NCEle.
-struct LhsTerms {
-  const double *td, *ta, *tb;  // [3 ne] diagonal and the two off-diagonal terms
-  const float *td32, *ta32, *tb32;  // the same rounded to FP32 (mixed precision)
-  int pairs;  // 1: a cached rebuild is k_lhs_pairs' and k_lhs_ep's (LhsPairs)
+// Patches (patch.h): per patch its own nodes, the elements at them and all nodes
+// of those elements (the window), each list padded to its longest length.
+struct DevPatch {
+  int n, nq;            // patches; element slots over all patches, n PATCH_ELEMS
+  int wmax;             // the largest window
+  const int* win;       // [n][PATCH_WIN] window nodes: the patch's own, ascending, then the
+                        //   others; -1: none
+  const int* el;        // [nq] elements, ascending
+  const ushort4* lv;    // [nq] window positions of an element's vertices; w: 1 if the first
+                        //   is the patch's own (each element in exactly one patch), 2: none
+  const ushort2* cspan; // [n][PATCH_NODES] per own node the span of its codes; y < x: none
+  const unsigned short* code;  // [n][3 PATCH_ELEMS] k PATCH_ELEMS + element for vertex k of
+                        //   the patch's element, in ascending element order per node
+  const unsigned* pair; // [n][mnei-1][PATCH_NODES] per own node and column j >= 1 the two
+                        //   codes of the edge terms it sums (3 PATCH_ELEMS: no term), low half
+                        //   first; ~0: no such column; null when some edge has more than
+                        //   two elements
+  const double* geo;    // [7][nq] FDXE, FDYE, AREAS; null: formed from the coordinates
 };
 
-// The same terms gathered per off-diagonal entry: entry (i, j >= 1) of COEF
-// receives, in ascending element order, the terms of the (at most two)
-// elements that hold the edge i-j, so a rebuild is
-// COEF(i, j) = (0 + t1 NCEle(e1)) + t2 NCEle(e2), one thread per entry with
-// no accumulation in between.  Index (j - 1) NP + i; an absent second term is
-// a zero term of element 0.
-struct LhsPairs {
-  const double *t1, *t2;
-  const float *t1f, *t2f;  // mixed precision: the FP32 terms
-  const int *e1, *e2;
-};
+// FDXE, FDYE and AREAS of an element from its vertices' coordinates, as a
+// reader of the grid forms them (src/mesh.F): the operations of prep.py's tables.
+__host__ __device__ __forceinline__ void elem_geometry(double X1, double X2, double X3, double Y1,
+                                                       double Y2, double Y3, double& fx1,
+                                                       double& fx2, double& fx3, double& fy1,
+                                                       double& fy2, double& fy3, double& area) {
+  fx1 = -(Y3 - Y2);
+  fx2 = -(Y1 - Y3);
+  fx3 = -(Y2 - Y1);
+  fy1 = X3 - X2;
+  fy2 = X1 - X3;
+  fy3 = X2 - X1;
+  area = fy2 * fx1 + fy1 * (Y1 - Y3);
+}
 
 // Compensated (Kahan 1965) summation in FP32: the node sums of FP32
 // element contributions in the mixed-precision path.  The result carries the
@@ -180,7 +199,7 @@ struct Kahan32 {
 struct RhsPrm {
   double ifnlfa, ifnlct, ifnlcat;
   double ondiag, offdiag;  // (1+ILump)*2 and 1-ILump (src/gwce.F:419-420)
-  int lumped;              // ILump = 1: no ETA1 gradient term (src/gwce.F:1233-1238)
+  int fric;                // TK formed by the pass itself
   int nws;
 };
 
@@ -245,6 +264,17 @@ struct FricPrm {
   Hybrid hyb;
 };
 
+// Apply2DBottomFriction (src/nodalattr.F:2400-2411), and the TKM = (TK, TK, 0)
+// of Apply2DInternalWaveDrag without wave drag; TKM is represented by TK alone.
+__device__ __forceinline__ double friction(const FricPrm& f, int i, double u, double v, double dp,
+                                           double eta2) {
+  const double uv1 = __builtin_sqrt(u * u + v * v);
+  const double h1 = dp + f.ifnlfa * eta2;
+  const double hyb = hybrid_term(f.hyb, h1);
+  const double a = f.fric[i] * (f.iflinbf + (uv1 / h1) * (f.ifnlbf + hyb));
+  return fmin(a, f.tkmax);
+}
+
 struct JcgArgs {
   int n, itmax, maxfn;
   double zeta, tz;
@@ -301,45 +331,19 @@ __global__ void k_tide_pot(int np, TipPrm p, const double* ln, const double* sla
 __global__ void k_friction(int np, FricPrm f, double* tk);
 __global__ void k_holland(int np, const double* x, const double* y, HollandPrm p, double* wsx,
                           double* wsy, double* pr);
-__global__ void k_friction_holland(int np, FricPrm f, double* tk, const double* x, const double* y,
-                                   HollandPrm p, double* wsx, double* wsy, double* pr);
 // LUMPED: the lumped GWCE (ILump = 1), whose LHS is the diagonal COEFD only
-// (kept in COEF's diagonal column) and whose solve is explicit
-template <bool LUMPED>
-__global__ void k_lhs_elem(DevMesh m, DevState s, const int* flags, double* sd, double* sa,
-                           double* sb);
-// CT: the type of the matrix terms summed per row (double; float in the
-// mixed path, which sums FP32 terms with compensation)
+// (kept in COEF's diagonal column) and whose solve is explicit.  CT: the type of
+// the element terms (float: the mixed path).
 template <bool LUMPED, typename CT>
-__global__ void k_lhs_rows(DevMesh m, DevState s, const int* flags, const double* sd,
-                           const double* sa, const double* sb, LhsTerms lt, double* ep_part,
-                           const double* restore_w);
-// the cached terms (once per context): k_lhs_elem's terms with NCEle = 1 and
-// ALPHAL = 1, and their FP32 roundings when td32 != null
-template <bool LUMPED>
-__global__ void k_lhs_terms(DevMesh m, double* td, double* ta, double* tb, float* td32,
-                            float* ta32, float* tb32);
-// NCEle of every element from the current NODECODE and NOFF
-__global__ void k_ncele(DevMesh m, DevState s);
-// per-entry terms (once per context) from the cached terms and the host's
-// entry codes (2 p + 0/1 for slot p's ta/tb term, -1 for none)
-__global__ void k_lhs_pair_setup(DevMesh m, LhsTerms lt, const int* c1, const int* c2,
-                                 double* t1, double* t2, float* t1f, float* t2f, int* e1,
-                                 int* e2);
-// A rebuild of the consistent GWCE matrix from the cached terms (the common
-// case: NCChange set, every ALPHAL 1): grid (row blocks, MNEI), column j of
-// COEF by blockIdx.y; then the EP chunk partials of the diagonal in the
-// fixed blocked tree.  Both leave at once otherwise (k_lhs_rows does it).
-template <typename CT>
-__global__ void k_lhs_pairs(DevMesh m, DevState s, const int* flags, LhsTerms lt, LhsPairs lp);
-__global__ void k_lhs_ep(DevMesh m, DevState s, const int* flags, double* ep_part);
+__global__ void k_gwce(DevMesh m, DevState s, DevPatch pp, RhsPrm q, FricPrm f, const int* flags,
+                       const double* restore_w);
+// bad[0]: some edge has more than two elements, bad[1]: the coordinates do not
+// give the geometry (both set, never cleared)
+__global__ void k_patch_check(DevMesh m, DevPatch pp, unsigned* pair, int* bad);
+__global__ void k_patch_geo(DevMesh m, DevPatch pp, double* geo);
+__global__ void k_ncele(DevMesh m, DevState s, DevPatch pp);
+__global__ void k_lhs_ep(DevMesh m, DevState s, int* flags, double* ep_part);
 __global__ void k_coef_restore(DevMesh m, DevState s, const double* w);
-// one block more than the elements need: the last finishes the GWCE matrix
-__global__ void k_rhs_elem(DevMesh m, DevState s, RhsPrm q, int* flags, double* contrib, int nch,
-                           const double* ep_part, double* scal);
-// the same in FP32 (the mixed path): FP32 contributions
-__global__ void k_rhs_elem32(DevMesh m, DevState s, RhsPrm q, int* flags, float* contrib,
-                             int nch, const double* ep_part, double* scal);
 // Jacobi scaling of the GWCE rows ahead of k_jcg (its first scaling pass)
 struct JcgPre {
   double* w;          // 1/sqrt(diag)
@@ -355,10 +359,9 @@ struct JcgPre {
   const double* ml_corr;  // warm == 2: the network's correction per node
   double* ml_u;           // warm == 2: the learned start, scaled
 };
-// CT: the type of the element contributions (float: compensated FP32 sums)
-template <bool LUMPED, typename CT>
-__global__ void k_rhs_node(DevMesh m, DevState s, const CT* contrib, const double* eta_bc,
-                           const double* scal, JcgPre pre);
+template <bool LUMPED>
+__global__ void k_rhs_node(DevMesh m, DevState s, const double* eta_bc, int nch,
+                           const double* ep_part, double* scal, JcgPre pre);
 // DUAL: start from the better (smaller initial pseudo-residual) of a.u and a.u2;
 // STAGED: the products read the pseudo-residual from LDS (a.hrows >= 0).
 // Instantiated for all four combinations.
@@ -376,7 +379,7 @@ __global__ void k_jcg_reg_batch(const JcgArgs* args, const int* first, int nsys)
 // more row tiles than blocks: the iterates in memory (a.uo, a.dpv, a.ndv)
 __global__ void k_jcg_mem(JcgArgs a);
 __global__ void k_wd_d1(DevMesh m, DevState s, int* flags, double h0, double habsmin);
-__global__ void k_wd_elem(DevMesh m, DevState s, WdPrm q, WdWork w);
+__global__ void k_wd_elem(DevMesh m, DevState s, WdPrm q, WdWork w, int* flags);
 __global__ void k_wd_index(const int* bcnt, int nb, int* bofs, int* flags);
 __global__ void k_wd_pred(DevMesh m, DevState s, WdWork w);
 __global__ void k_wd_close(WdWork w, int* flags);
@@ -386,13 +389,8 @@ __global__ void k_wd_final_area(DevMesh m, DevState s, WdWork w, const int* flag
 __global__ void k_wd_d2(DevMesh m, DevState s, const double* area_slot, int* flags, double ifnlfa);
 __global__ void k_wd_alpha(DevMesh m, DevState s, int* flags, double slim);
 __global__ void k_h2(int np, const double* dp, const double* eta2, double ifnlfa, double* h2);
-template <bool ALPHA>
-__global__ void k_mom_elem(DevMesh m, DevState s, MomPrm q, double* cx, double* cy, int* flags);
-// the same in FP32 (the mixed path)
-template <bool ALPHA>
-__global__ void k_mom_elem32(DevMesh m, DevState s, MomPrm q, float* cx, float* cy, int* flags);
-template <typename CT>
-__global__ void k_mom_node(DevMesh m, DevState s, MomPrm q, const CT* cx, const CT* cy);
+template <bool ALPHA, typename CT>
+__global__ void k_mom(DevMesh m, DevState s, DevPatch pp, MomPrm q);
 __global__ void k_fill_u32(unsigned* p, unsigned v, int n);
 __global__ void k_fill_i32(int* p, int v, int n);
 __global__ void k_total_area(DevMesh m, DevState s);
