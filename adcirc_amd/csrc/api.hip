@@ -83,7 +83,7 @@ struct adcgpu_ctx {
   int *nodecode, *nnodecode, *noff, *noffold, *mju, *etamax_it, *umax_it;
   int cur_it = 0;  // step opened by adcgpu_begin_step
   // work
-  double *wd_area = nullptr, *ep_part = nullptr, *scal = nullptr;
+  double *ep_part = nullptr, *scal = nullptr;
   double *eta_bc = nullptr, *eta_bc_table = nullptr;
   int eta_bc_table_steps = 0;
   WdWork wd{};
@@ -813,7 +813,6 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   A(&c->nodecode, np); A(&c->nnodecode, np); A(&c->noff, ne); A(&c->noffold, ne);
   A(&c->mju, np); A(&c->etamax_it, np); A(&c->etas_prev, np);
   A(&c->umax, np); A(&c->umax_it, np);
-  A(&c->wd_area, 3 * (size_t)ne);
   c->mixed = P->precision == ADCGPU_MIXED;
   {
     DevPatch& pp = c->patch;
@@ -832,8 +831,10 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   A(&c->ep_part, c->nch); A(&c->scal, S_COUNT); A(&c->eta_bc, std::max(neta, 1));
   {
     const size_t nb = (size_t)(ne + 255) / 256;
-    A(&c->wd.mask, nb * 4); A(&c->wd.bcnt, nb); A(&c->wd.bofs, nb);
-    A(&c->wd.tkc, ne); A(&c->wd.lc, ne); A(&c->wd.m0, ne); A(&c->wd.pred, ne);
+    A(&c->wd.mask, nb * 4); A(&c->wd.cid, ne); A(&c->wd.bcnt, nb);
+    A(&c->wd.tkc, ne); A(&c->wd.lc, ne);
+    if (!rc) (void)hipMemset(c->wd.lc, 0xff, (size_t)ne * sizeof(int2));
+    A(&c->wd.m0, ne); A(&c->wd.pred, ne);
     A(&c->wd.wnode, ne); A(&c->wd.M, ne);
     const size_t nwb = (size_t)(ne + WD_BLOCK - 1) / WD_BLOCK;
     A(&c->wd.cv, ne); A(&c->wd.cE, (size_t)ne * WD_XW); A(&c->wd.xtab, nwb * WD_XMAX);
@@ -864,11 +865,8 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
         e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 patch_lds_bytes(PATCH_MOM_FIELDS, PATCH_MOM_TERMS, PATCH_WIN));
     if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)k_wd_link, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              WD_LINK_LDS);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)k_wd_close, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              WD_CLOSE_LDS);
+      e = hipFuncSetAttribute((const void*)k_wd_chain, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              WD_CHAIN_LDS);
     if (e != hipSuccess) rc = fail(ADCGPU_E_UNSUPPORTED, std::string("LDS request: ") +
                                                          hipGetErrorString(e));
   }
@@ -1269,25 +1267,16 @@ static int wetdry_device(adcgpu_ctx* c, bool alpha_pass) {
                        c->ifnlfa, c->h2);
     return check_launch("h2");
   }
-  hipLaunchKernelGGL(k_wd_d1, dim3(nblk(np, 256)), dim3(256), 0, c->stream, c->mesh(),
-                     c->state(), c->flags, c->prm.h0, c->habsmin);
-  WdPrm q{c->hoff, c->prm.velmin, c->iflinbf, c->ifnlbf, c->tkmax, c->hyb};
-  const int nb = nblk(ne, 256);
-  hipLaunchKernelGGL(k_wd_elem, dim3(nb), dim3(256), 0, c->stream, c->mesh(), c->state(), q,
-                     c->wd, c->flags);
-  hipLaunchKernelGGL(k_wd_index, dim3(1), dim3(1024), 0, c->stream, c->wd.bcnt, nb, c->wd.bofs,
-                     c->flags);
-  hipLaunchKernelGGL(k_wd_pred, dim3(nb), dim3(256), 0, c->stream, c->mesh(), c->state(), c->wd);
-  const int nwb = std::min((ne + WD_BLOCK - 1) / WD_BLOCK, 256);
-  hipLaunchKernelGGL(k_wd_close, dim3(nwb), dim3(WD_BLOCK), WD_CLOSE_LDS, c->stream, c->wd,
-                     c->flags);
-  hipLaunchKernelGGL(k_wd_link, dim3(1), dim3(256), WD_LINK_LDS, c->stream, c->wd, c->flags,
-                     c->tk);
-  // NCEle*AREAS/2 per incidence slot
-  hipLaunchKernelGGL(k_wd_final_area, dim3(nblk(ne, 256)), dim3(256), 0, c->stream, c->mesh(),
-                     c->state(), c->wd, c->flags, c->tk, c->wd_area);
-  hipLaunchKernelGGL(k_wd_d2, dim3(nblk(np, 256)), dim3(256), 0, c->stream, c->mesh(),
-                     c->state(), c->wd_area, c->flags, c->ifnlfa);
+  const WdPrm q{c->prm.h0, c->habsmin, c->hoff, c->prm.velmin, c->iflinbf, c->ifnlbf, c->tkmax,
+                c->hyb};
+  const DevPatch& pp = c->patch;
+  hipLaunchKernelGGL(k_wd_elem, dim3(pp.n), dim3(PATCH_THREADS), 0, c->stream, c->mesh(),
+                     c->state(), pp, q, c->wd, c->flags);
+  hipLaunchKernelGGL(k_wd_d2, dim3(pp.n + nblk(nblk(ne, 256), WD_TILES)), dim3(PATCH_THREADS), 0, c->stream, c->mesh(),
+                     c->state(), pp, q, c->wd, c->flags, c->ifnlfa);
+  const int nwb = std::min((ne + WD_BLOCK - 1) / WD_BLOCK, WD_CHAIN_BLOCKS);
+  hipLaunchKernelGGL(k_wd_chain, dim3(nwb), dim3(WD_BLOCK), WD_CHAIN_LDS, c->stream, c->mesh(),
+                     c->state(), c->wd, c->flags);
   if (alpha_pass)
     hipLaunchKernelGGL(k_wd_alpha, dim3(nblk(ne, 256)), dim3(256), 0, c->stream, c->mesh(),
                        c->state(), c->flags, 1.0e9);

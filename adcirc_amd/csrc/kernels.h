@@ -33,7 +33,6 @@ __host__ __device__ constexpr int jcg_part_doubles(int nch) { return 4 * 4 * (nc
 // at most: the block's rows and 5,632 rows each side
 constexpr int JCG_STAGE_MAX_BYTES = 120 * 1024;
 static_assert(JCG_STAGE_MAX_BYTES / 8 <= 65536, "staged positions are 16-bit");
-constexpr int NODE_STAGE = 2048;   // incidence slots a 256-node block stages in LDS
 // patches: a block's threads, and at most so many elements (one per thread),
 // window nodes, and own nodes.  About 10 x 10 nodes have 235 elements: one per
 // thread, and a sixth more element evaluations than the mesh has elements.
@@ -53,14 +52,17 @@ constexpr int WD_XW = WD_XMAX / 64;
 constexpr int WD_HASH = 2 * WD_XMAX;         // LDS hash slots for a block's external names
 constexpr int WD_INC_MAX = 12;               // incidence lists a wetting candidate scans at once
 constexpr int WD_CLOSE_LDS = 2 * WD_BLOCK * (8 + 8 * WD_XW + 4) + 2 * WD_HASH * 4;
-constexpr int WD_LINK_BLOCKS = 64;           // blocks whose link values fit the LDS of k_wd_link
-// serial fallback of k_wd_link: candidates staged through LDS in chunks, the
+constexpr int WD_LINK_BLOCKS = 64;           // blocks whose link values fit the LDS of k_wd_chain
+// serial fallback of k_wd_chain: candidates staged through LDS in chunks, the
 // running maxima of the most recent WD_RING candidates kept in an LDS ring
 constexpr int WD_CHUNK = 2048;
 constexpr int WD_RING = 8192;   // power of two
 constexpr int WD_SERIAL_LDS = WD_RING * 8 + WD_CHUNK * (8 + 8 + 8);
 constexpr int WD_LINK_LDS = WD_LINK_BLOCKS * WD_XMAX * 8 > WD_SERIAL_LDS
                                 ? WD_LINK_BLOCKS * WD_XMAX * 8 : WD_SERIAL_LDS;
+constexpr int WD_CHAIN_LDS = WD_LINK_LDS > WD_CLOSE_LDS ? WD_LINK_LDS : WD_CLOSE_LDS;
+constexpr int WD_TILES = 1024;        // 256-element tiles a block lists
+constexpr int WD_CHAIN_BLOCKS = 32;  // blocks of k_wd_chain at most
 
 // device flag slots
 enum { F_NCCHANGE = 0, F_NUMITR = 2, F_IER, F_ERROR, F_NCAND, F_ITSUM, F_NREBUILD, F_WDSERIAL,
@@ -71,6 +73,7 @@ enum { F_NCCHANGE = 0, F_NUMITR = 2, F_IER, F_ERROR, F_NCAND, F_ITSUM, F_NREBUIL
        F_MLUSED,   // solves that started from the learned guess
        F_REBUILT,  // this step's GWCE matrix was rebuilt (k_lhs_ep)
        F_ALPHA0,   // F_ALPHA as the last step left it
+       F_WDDONE,   // k_wd_chain's blocks that have ended
        F_COUNT = 16 };
 enum { ERR_DIAG = 1, ERR_BARRIER = 4, ERR_ELEV = 8, ERR_NONFINITE = 16 };
 // device scalar slots
@@ -226,7 +229,7 @@ __device__ __forceinline__ double hybrid_term(const Hybrid& h, double H) {
 }
 
 struct WdPrm {
-  double hoff, velmin, iflinbf, ifnlbf, tkmax;
+  double h0, habsmin, hoff, velmin, iflinbf, ifnlbf, tkmax;
   Hybrid hyb;
 };
 
@@ -234,16 +237,18 @@ struct WdPrm {
 // Candidate k is the k-th candidate element in element order; every array is
 // sized for the worst case of one candidate per element.
 struct WdWork {
-  unsigned long long* mask;  // [ceil(ne/64)] bit e%64 of word e/64: element e is a candidate
-  int* bcnt;                 // [ceil(ne/256)] candidates per 256-element tile
-  int* bofs;                 // [ceil(ne/256)] candidates in earlier tiles
+  unsigned long long* mask;  // [4 ceil(ne/256)] bit e%64 of word e/64: element e is a
+                             // candidate (clear between steps)
+  int* bcnt;                 // [ceil(ne/256)] candidates per 256-element tile (clear between steps)
+  int* cid;                  // [ne] candidate k: its element
   double* tkc;               // [ne] TK_TMP(NM123) of candidate element e
-  int* lc;                   // [ne] local vertex of NM123 | local vertex of the partner << 2
-  double* m0;                // [ne] candidate k: TK_TMP and the entry TK of nodes it opens
-  int2* pred;                // [ne] candidate k: previous candidate on NM123 / partner, or -1
-  int2* wnode;               // [ne] candidate k: NM123 / partner if k is its last candidate, or -1
+  int2* lc;                  // [ne] candidate element: local vertex of NM123 | local vertex of
+                             // the partner << 2, and its candidate index; -1 otherwise
+  double* m0;                // [ne] candidate element: TK_TMP and the entry TK of nodes it opens
+  int2* pred;                // [ne] candidate element: the previous one on NM123 / partner, or -1
+  int2* wnode;               // [ne] candidate element: NM123 / partner if it is the node's last, or -1
   double* M;                 // [ne] candidate k: TK of both nodes after k (serial fallback)
-  // block closure (k_wd_close): candidate k's value is
+  // block closure (wd_close): candidate k's value is
   // max(cv[k], X values of the bits of cE[k]), the X values being those of the
   // earlier candidates xtab[b*WD_XMAX + i] of its block b = k / WD_BLOCK
   double* cv;                // [ne] maximum over k's ancestors inside its block
@@ -378,15 +383,11 @@ template <bool DUAL, int CPB>
 __global__ void k_jcg_reg_batch(const JcgArgs* args, const int* first, int nsys);
 // more row tiles than blocks: the iterates in memory (a.uo, a.dpv, a.ndv)
 __global__ void k_jcg_mem(JcgArgs a);
-__global__ void k_wd_d1(DevMesh m, DevState s, int* flags, double h0, double habsmin);
-__global__ void k_wd_elem(DevMesh m, DevState s, WdPrm q, WdWork w, int* flags);
-__global__ void k_wd_index(const int* bcnt, int nb, int* bofs, int* flags);
-__global__ void k_wd_pred(DevMesh m, DevState s, WdWork w);
-__global__ void k_wd_close(WdWork w, int* flags);
-__global__ void k_wd_link(WdWork w, int* flags, double* tk);
-__global__ void k_wd_final_area(DevMesh m, DevState s, WdWork w, const int* flags, double* tk,
-                                double* area_slot);
-__global__ void k_wd_d2(DevMesh m, DevState s, const double* area_slot, int* flags, double ifnlfa);
+__global__ void k_wd_elem(DevMesh m, DevState s, DevPatch pp, WdPrm q, WdWork w, int* flags);
+// the first ceil(ceil(NE/256) / WD_TILES) blocks list the candidates, then one per patch
+__global__ void k_wd_d2(DevMesh m, DevState s, DevPatch pp, WdPrm q, WdWork w, int* flags,
+                        double ifnlfa);
+__global__ void k_wd_chain(DevMesh m, DevState s, WdWork w, int* flags);
 __global__ void k_wd_alpha(DevMesh m, DevState s, int* flags, double slim);
 __global__ void k_h2(int np, const double* dp, const double* eta2, double ifnlfa, double* h2);
 template <bool ALPHA, typename CT>

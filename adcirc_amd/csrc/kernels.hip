@@ -316,228 +316,26 @@ template __global__ void k_rhs_node<false>(DevMesh, DevState, const double*, int
 template __global__ void k_rhs_node<true>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre);
 
 // ---------------------------------------------------------------- wet/dry
-// D1 (src/wetdry.F:234-285); also NNODECODE := NODECODE for the W1 writes.
-__global__ __launch_bounds__(256) void k_wd_d1(DevMesh m, DevState s, int* flags, double h0, double habsmin) {
-  int i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  // this step's ALPHAL pass sets F_ALPHA again where needed; it rewrites ALPHAL
-  // while the last pass (or the host) left some value other than 1
-  if (i == 0) {
-    flags[F_ALPHA0] = flags[F_ALPHA];
-    flags[F_ALPHA] = 0;
-  }
-  if (i >= m.np) return;
-  int nc = s.nodecode[i];
-  if (nc == 1) {
-    const double htot = m.dp[i] + s.eta2[i];
-    if (htot <= h0) {
-      if (htot < habsmin) s.eta2[i] = habsmin - m.dp[i];
-      nc = 0;
-      s.nodecode[i] = 0;
-      atomicOr(&flags[F_NCCHANGE], 1);
-    }
-  }
-  s.nnodecode[i] = nc;
+// Values that another block of the launch reads: written through, and read past
+// the caches.
+__device__ __forceinline__ void wd_put(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void wd_put(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void wd_put(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ T wd_get(const T* p) {
+  return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// W1 candidates (src/wetdry.F:332-818) and DE1 (src/wetdry.F:1110-1233).
-// Candidate elements whose steady-flow velocity exceeds VELMIN wet their dry
-// node here (an idempotent store).  Their friction updates depend on element
-// order: each candidate leaves its TK_TMP value and local vertices at its
-// element and sets its bit in the candidate mask (one word per wave), and the
-// block's candidate count goes to bcnt[tile] for the compaction below.
-__global__ __launch_bounds__(256) void k_wd_elem(DevMesh m, DevState s, WdPrm q, WdWork w, int* flags) {
-  __shared__ int wcount[4];
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int e = tile * 256 + threadIdx.x;
-  bool cand = false;
-  if (e < m.ne) {
-    const int n[3] = {m.nm[3 * e], m.nm[3 * e + 1], m.nm[3 * e + 2]};
-    const int old = s.noff[e];
-    int noff = 1;
-    const double e1 = s.eta2[n[0]], e2 = s.eta2[n[1]], e3 = s.eta2[n[2]];
-    const double h1 = m.dp[n[0]] + e1, h2 = m.dp[n[1]] + e2, h3 = m.dp[n[2]] + e3;
-    const int c0 = s.nodecode[n[0]], c1 = s.nodecode[n[1]], c2 = s.nodecode[n[2]];
-    if (c0 + c1 + c2 == 2) {
-      int a = -1, b = -1, c = -1;
-      if (c0 == 1 && c1 == 1) { a = 0; b = 1; c = 2; }
-      else if (c1 == 1 && c2 == 1) { a = 1; b = 2; c = 0; }
-      else if (c2 == 1 && c0 == 1) { a = 2; b = 0; c = 1; }
-      const double ht[3] = {h1, h2, h3};
-      if (a >= 0 && ht[a] >= q.hoff && ht[b] >= q.hoff) {
-        const int na = n[a], nb = n[b], nc = n[c];
-        int l123 = a;
-        if (s.eta2[nb] > s.eta2[na]) l123 = b;
-        const int nm123 = n[l123];
-        const double dy = m.y[nc] - m.y[nm123], dx = m.x[nc] - m.x[nm123];
-        const double deldist = __builtin_sqrt(dy * dy + dx * dx);
-        double deleta = s.eta2[nm123] - s.eta2[nc];
-        if (deleta < 0.0) deleta = 0.0;
-        const double H1 = s.eta2[nm123] + m.dp[nm123];
-        const double fr = s.fric[nm123];
-        const double hyb = hybrid_term(q.hyb, H1);
-        const double tkwet = fmax(fr * (q.iflinbf + (q.velmin / H1) * (q.ifnlbf + hyb)), 0.0001);
-        const double vel = m.g * (deleta / deldist) / tkwet;
-        if (vel > q.velmin) {
-          s.nnodecode[nc] = 1;
-          w.tkc[e] = fmin(fr * (q.iflinbf + (1.0 * vel / H1) * (q.ifnlbf + hyb)), q.tkmax);
-          w.lc[e] = l123 | ((l123 == b ? a : b) << 2);
-          cand = true;
-        }
-      }
-    }
-    const double HOFF = q.hoff;
-    if ((e1 >= e2) && (e2 > e3)) if ((h1 < HOFF) || (h2 < HOFF)) noff = 0;
-    if ((e2 >= e3) && (e3 > e1)) if ((h2 < HOFF) || (h3 < HOFF)) noff = 0;
-    if ((e3 >= e1) && (e1 > e2)) if ((h3 < HOFF) || (h1 < HOFF)) noff = 0;
-    if ((e1 >= e3) && (e3 > e2)) if ((h1 < HOFF) || (h3 < HOFF)) noff = 0;
-    if ((e2 >= e1) && (e1 > e3)) if ((h2 < HOFF) || (h1 < HOFF)) noff = 0;
-    if ((e3 >= e2) && (e2 > e1)) if ((h3 < HOFF) || (h2 < HOFF)) noff = 0;
-    // NOFF changes count toward NCCHANGE (src/wetdry.F:1428-1430)
-    if (noff != old) {
-      s.noff[e] = noff;
-      atomicOr(&flags[F_NCCHANGE], 1);
-    }
-  }
-  // every lane of the block reaches the ballot; a wave covers elements
-  // 64*word .. 64*word+63
-  const unsigned long long bits = __ballot(cand);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    if (tile * 256 + wave * 64 < m.ne) w.mask[tile * 4 + wave] = bits;
-    wcount[wave] = __popcll(bits);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) w.bcnt[tile] = (wcount[0] + wcount[1]) + (wcount[2] + wcount[3]);
-}
-
-// Exclusive prefix of the per-tile candidate counts (one block of 1024) and
-// the step's candidate count.
-__global__ __launch_bounds__(1024) void k_wd_index(const int* __restrict__ bcnt, int nb,
-                                                   int* __restrict__ bofs, int* flags) {
-  __shared__ int wtot[16];
-  const int t = threadIdx.x;
-  const int per = (nb + 1023) / 1024;
-  const int lo = min(t * per, nb), hi = min(lo + per, nb);
-  int sum = 0;
-#pragma unroll 8
-  for (int i = lo; i < hi; ++i) sum += bcnt[i];
-  int incl = sum;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(incl, off, 64);
-    if ((t & 63) >= off) incl += v;
-  }
-  if ((t & 63) == 63) wtot[t >> 6] = incl;
-  __syncthreads();
-  int base = 0;
-  for (int i = 0; i < (t >> 6); ++i) base += wtot[i];
-  int run = base + incl - sum;
-#pragma unroll 8
-  for (int i = lo; i < hi; ++i) {
-    bofs[i] = run;
-    run += bcnt[i];
-  }
-  if (t == 1023) {
-    flags[F_NCAND] = base + incl;
-    flags[F_WDSERIAL] = 0;
-  }
-}
-
-// Candidate index of candidate element e (element order); `word` = mask[e/64].
-__device__ __forceinline__ int wd_index(const WdWork& w, int e, unsigned long long word) {
-  const int tile = e >> 8, wi = (e >> 6) & 3;
-  int k = w.bofs[tile];
-  for (int j = 0; j < wi; ++j) k += __popcll(w.mask[tile * 4 + j]);
-  return k + __popcll(word & ((1ull << (e & 63)) - 1ull));
-}
-
-// Does candidate code 3*e2+k2 (element e2, local vertex k2) update the TK of
-// that vertex, i.e. is e2 a candidate and the vertex one of its two wet nodes?
-__device__ __forceinline__ bool wd_touches(const WdWork& w, int e2, int k2) {
-  if (!((w.mask[e2 >> 6] >> (e2 & 63)) & 1ull)) return false;
-  const int lc = w.lc[e2];
-  return k2 == (lc & 3) || k2 == ((lc >> 2) & 3);
-}
-
-// Ordered W1 friction updates (src/wetdry.F:447-472), links.  The reference
-// visits the candidates in ascending element order; candidate k sets
-// TK(NM123) = MAX(TK_TMP, TK(NM123)), gives the partner the larger of the two
-// and takes it back if the partner was larger, so afterwards both of its
-// nodes hold M_k = max(TK_TMP_k, their values before k).  A node's value
-// before k is M_j of the nearest earlier candidate j on that node, or its
-// value on entry.  The node incidence lists are sorted by element, so j and
-// "k is the node's last candidate" are found by walking the node's list
-// backward and forward from k's own slot.  Entry values fold into m0.
-__global__ __launch_bounds__(256) void k_wd_pred(DevMesh m, DevState s, WdWork w) {
-  const int e = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (e >= m.ne) return;
-  const unsigned long long word = w.mask[e >> 6];
-  if (!((word >> (e & 63)) & 1ull)) return;
-  const int k = wd_index(w, e, word);
-  const int lc = w.lc[e];
-  double v = w.tkc[e];
-  int pred[2], wn[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int l = (lc >> (2 * j)) & 3;
-    const int x = m.nm[3 * e + l];
-    const int pos = m.slot[3 * e + l];
-    const int p0 = m.inc_ptr[x], p1 = m.inc_ptr[x + 1];
-    int pk = -1;
-    bool last = true;
-    if (p1 - p0 <= WD_INC_MAX) {
-      // the node's whole list at once: its codes, then their mask words,
-      // then the candidates' vertex codes, each round of loads independent
-      int code[WD_INC_MAX];
-#pragma unroll
-      for (int q = 0; q < WD_INC_MAX; ++q) code[q] = p0 + q < p1 ? m.inc[p0 + q] : -1;
-      unsigned long long mw[WD_INC_MAX];
-#pragma unroll
-      for (int q = 0; q < WD_INC_MAX; ++q) mw[q] = code[q] >= 0 ? w.mask[(code[q] / 3) >> 6] : 0ull;
-      unsigned tch = 0;  // bit q: entry q's element is a candidate that updates node x
-      int lq[WD_INC_MAX];
-#pragma unroll
-      for (int q = 0; q < WD_INC_MAX; ++q) {
-        const int e2 = code[q] / 3;
-        const bool cand = code[q] >= 0 && ((mw[q] >> (e2 & 63)) & 1ull);
-        lq[q] = cand ? w.lc[e2] : -1;
-      }
-#pragma unroll
-      for (int q = 0; q < WD_INC_MAX; ++q) {
-        const int k2 = code[q] - 3 * (code[q] / 3);
-        if (lq[q] >= 0 && (k2 == (lq[q] & 3) || k2 == ((lq[q] >> 2) & 3))) tch |= 1u << q;
-      }
-      const int me = pos - p0;
-      const unsigned before = tch & ((1u << me) - 1u), after = tch >> (me + 1);
-      if (before) {
-        const int q = 31 - __clz((int)before);  // the nearest earlier candidate
-        const int e2 = m.inc[p0 + q] / 3;
-        pk = wd_index(w, e2, w.mask[e2 >> 6]);
-      }
-      last = after == 0u;
-    } else {
-      for (int r = pos - 1; r >= p0; --r) {
-        const int code = m.inc[r], e2 = code / 3;
-        if (wd_touches(w, e2, code - 3 * e2)) {
-          pk = wd_index(w, e2, w.mask[e2 >> 6]);
-          break;
-        }
-      }
-      for (int r = pos + 1; r < p1; ++r) {
-        const int code = m.inc[r], e2 = code / 3;
-        if (wd_touches(w, e2, code - 3 * e2)) {
-          last = false;
-          break;
-        }
-      }
-    }
-    if (pk < 0) v = fmax(v, s.tk[x]);
-    pred[j] = pk;
-    wn[j] = last ? x : -1;
-  }
-  w.m0[k] = v;
-  w.pred[k] = make_int2(pred[0], pred[1]);
-  w.wnode[k] = make_int2(wn[0], wn[1]);
+// The candidate indices of candidate element e's predecessors, or -1.
+__device__ __forceinline__ int2 wd_pred_index(const WdWork& w, int e) {
+  const int2 p = w.pred[e];
+  return make_int2(p.x >= 0 ? w.lc[p.x].y : -1, p.y >= 0 ? w.lc[p.y].y : -1);
 }
 
 // Ordered W1 friction updates, values: M_k = max(m0_k, M of k's predecessors)
@@ -558,7 +356,7 @@ __global__ __launch_bounds__(256) void k_wd_pred(DevMesh m, DevState s, WdWork w
 // can always expand it, so the rounds end; along a wetting front, where
 // candidates chain through shared nodes, they take about log2 of the chain
 // length.  A block naming more than WD_XMAX external candidates sets
-// F_WDSERIAL, and k_wd_link then forms every value serially instead.
+// F_WDSERIAL, and every value is formed serially instead.
 __device__ __forceinline__ void wd_add(int* u, int& nu, int f) {
   if (f == 0xffff) return;
   for (int i = 0; i < nu; ++i)
@@ -566,8 +364,8 @@ __device__ __forceinline__ void wd_add(int* u, int& nu, int f) {
   u[nu++] = f;
 }
 
-__global__ __launch_bounds__(1024) void k_wd_close(WdWork w, int* flags) {
-  extern __shared__ double wc_lds[];
+__device__ __forceinline__ void wd_close(const DevMesh& m, const DevState& s, const WdWork& w,
+                                         int* flags, double* wc_lds) {
   double* sv = wc_lds;                                                       // [2][WD_BLOCK]
   unsigned long long* sE = reinterpret_cast<unsigned long long*>(sv + 2 * WD_BLOCK);  // [2][WD_XW][WD_BLOCK]
   int* sF = reinterpret_cast<int*>(sE + 2 * WD_XW * WD_BLOCK);               // [2][WD_BLOCK]
@@ -582,13 +380,16 @@ __global__ __launch_bounds__(1024) void k_wd_close(WdWork w, int* flags) {
     for (int i = l; i < WD_HASH; i += WD_BLOCK) hkey[i] = -1;
     if (l == 0) xn = 0;
     __syncthreads();
-    int qq[2] = {-1, -1};
+    int qq[2] = {-1, -1}, wn[2] = {-1, -1};
     double v = 0.0;
     if (k < n) {
-      const int2 q = w.pred[k];
+      const int e = w.cid[k];
+      const int2 q = wd_pred_index(w, e), x = w.wnode[e];
+      v = w.m0[e];
       qq[0] = q.x;
       qq[1] = q.y;
-      v = w.m0[k];
+      wn[0] = x.x;
+      wn[1] = x.y;
     }
     // the block's external names: one hash slot per distinct candidate
     int slot[2] = {-1, -1};
@@ -614,7 +415,7 @@ __global__ __launch_bounds__(1024) void k_wd_close(WdWork w, int* flags) {
       if (won[j]) {
         const int i = atomicAdd(&xn, 1);
         hidx[slot[j]] = i;
-        if (i < WD_XMAX) w.xtab[b * WD_XMAX + i] = qq[j];
+        if (i < WD_XMAX) wd_put(&w.xtab[b * WD_XMAX + i], qq[j]);
       }
     __syncthreads();
     unsigned long long E[WD_XW] = {};
@@ -636,7 +437,7 @@ __global__ __launch_bounds__(1024) void k_wd_close(WdWork w, int* flags) {
       if (l == 0) atomicOr(&flags[F_WDSERIAL], 1);
       continue;
     }
-    if (l == 0) w.xcnt[b] = xn;
+    if (l == 0) wd_put(&w.xcnt[b], xn);
     int cur = 0;
     sv[l] = v;
 #pragma unroll
@@ -703,10 +504,13 @@ __global__ __launch_bounds__(1024) void k_wd_close(WdWork w, int* flags) {
       cur = nx;
       if (!__syncthreads_or((F & 0xffff) != 0xffff)) break;
     }
-    if (k < n) {
-      w.cv[k] = v;
+    if (nblk == 1) {  // no candidates outside the block: the values are final
+      for (int j = 0; j < 2; ++j)
+        if (wn[j] >= 0) s.tk[wn[j]] = v;
+    } else if (k < n) {
+      wd_put(&w.cv[k], v);
 #pragma unroll
-      for (int i = 0; i < WD_XW; ++i) w.cE[(size_t)k * WD_XW + i] = E[i];
+      for (int i = 0; i < WD_XW; ++i) wd_put(&w.cE[(size_t)k * WD_XW + i], E[i]);
     }
   }
 }
@@ -726,9 +530,10 @@ __device__ void wd_serial(const WdWork& w, int n, double* __restrict__ tk, doubl
   for (int base = 0; base < n; base += WD_CHUNK) {
     const int cn = min(WD_CHUNK, n - base);
     for (int i = t; i < cn; i += blockDim.x) {
-      cm0[i] = w.m0[base + i];
-      cpred[i] = w.pred[base + i];
-      cwn[i] = w.wnode[base + i];
+      const int e = w.cid[base + i];
+      cm0[i] = w.m0[e];
+      cpred[i] = wd_pred_index(w, e);
+      cwn[i] = w.wnode[e];
     }
     __syncthreads();
     if (t == 0) {
@@ -760,117 +565,74 @@ __device__ void wd_serial(const WdWork& w, int n, double* __restrict__ tk, doubl
 
 // Values of the external names, block after block: name i of block c is an
 // earlier candidate x of block b < c, so its value is max(cv[x], values of
-// the names of block b set in cE[x]), all known by then.  One block of 256
-// (one lane per name); dynamic LDS of WD_LINK_LDS bytes (the name values of
-// up to WD_LINK_BLOCKS blocks; beyond that they stay in w.xval).
-__global__ __launch_bounds__(256) void k_wd_link(WdWork w, int* flags, double* __restrict__ tk) {
-  extern __shared__ double lk_lds[];
-  const int n = flags[F_NCAND];
-  if (n == 0) return;
-  if (flags[F_WDSERIAL]) {
-    wd_serial(w, n, tk, lk_lds);
-    return;
-  }
+// the names of block b set in cE[x]), all known by then.  One block, one lane
+// per name; LDS of WD_LINK_LDS bytes (the name values of up to WD_LINK_BLOCKS
+// blocks; beyond that they are kept in w.xval).  Then each candidate's M_k,
+// written as TK of the nodes it is the last candidate of.
+__device__ __forceinline__ void wd_link(const WdWork& w, int n, double* __restrict__ tk,
+                                        double* lk_lds) {
   const int nblk = (n + WD_BLOCK - 1) / WD_BLOCK;
   double* X = nblk <= WD_LINK_BLOCKS ? lk_lds : w.xval;
   const int t = threadIdx.x;
-  for (int c = 1; c < nblk; ++c) {
-    if (t < w.xcnt[c]) {
-      const int x = w.xtab[c * WD_XMAX + t];
-      double v = w.cv[x];
-      const double* Xb = X + (x / WD_BLOCK) * WD_XMAX;
+  auto value = [&](int x) {
+    double v = wd_get(&w.cv[x]);
+    unsigned long long E[WD_XW];
 #pragma unroll
-      for (int i = 0; i < WD_XW; ++i) {
-        unsigned long long E = w.cE[(size_t)x * WD_XW + i];
-        while (E) {
-          v = fmax(v, Xb[64 * i + __ffsll((long long)E) - 1]);
-          E &= E - 1;
-        }
+    for (int i = 0; i < WD_XW; ++i) E[i] = wd_get(&w.cE[(size_t)x * WD_XW + i]);
+    const double* Xb = X + (x / WD_BLOCK) * WD_XMAX;
+#pragma unroll
+    for (int i = 0; i < WD_XW; ++i)
+      while (E[i]) {
+        v = fmax(v, Xb[64 * i + __ffsll((long long)E[i]) - 1]);
+        E[i] &= E[i] - 1;
       }
-      X[c * WD_XMAX + t] = v;
-    }
+    return v;
+  };
+  for (int c = 1; c < nblk; ++c) {
+    if (t < wd_get(&w.xcnt[c])) X[c * WD_XMAX + t] = value(wd_get(&w.xtab[c * WD_XMAX + t]));
     __syncthreads();
   }
-  if (X != w.xval)
-    for (int i = t; i < nblk * WD_XMAX; i += blockDim.x) w.xval[i] = X[i];
+  for (int k = t; k < n; k += blockDim.x) {
+    const int2 x = w.wnode[w.cid[k]];
+    const double v = value(k);
+    if (x.x >= 0) tk[x.x] = v;
+    if (x.y >= 0) tk[x.y] = v;
+  }
 }
 
-// Final values and the TK of each node from its last candidate.
-__global__ __launch_bounds__(256) void k_wd_final_area(DevMesh m, DevState s, WdWork w,
-                                                       const int* flags,
-                                                       double* __restrict__ tk,
-                                                       double* __restrict__ area_slot) {
-  // (1) each candidate's M_k, written as TK of its two wet nodes (skipped
-  // when the serial pass already did it)
+// The ordered friction updates of the step's candidates (linked and listed by the
+// pass before): block closure by as many blocks as have candidates; the block
+// that ends last joins the blocks' values and writes TK, so that no block waits
+// for another.  Dynamic LDS: WD_CHAIN_LDS bytes.
+__global__ __launch_bounds__(WD_BLOCK) void k_wd_chain(DevMesh m, DevState s, WdWork w, int* flags) {
+  extern __shared__ double ch_lds[];
+  __shared__ int last;
   const int n = flags[F_NCAND];
-  if (!flags[F_WDSERIAL]) {
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-      double v = w.cv[k];
-      const double* Xb = w.xval + (k / WD_BLOCK) * WD_XMAX;
-#pragma unroll
-      for (int i = 0; i < WD_XW; ++i) {
-        unsigned long long E = w.cE[(size_t)k * WD_XW + i];
-        while (E) {
-          v = fmax(v, Xb[64 * i + __ffsll((long long)E) - 1]);
-          E &= E - 1;
-        }
-      }
-      const int2 x = w.wnode[k];
-      if (x.x >= 0) tk[x.x] = v;
-      if (x.y >= 0) tk[x.y] = v;
-    }
+  const int nblk = (n + WD_BLOCK - 1) / WD_BLOCK;
+  const int active = min(nblk, (int)gridDim.x);
+  if ((int)blockIdx.x >= active) return;
+  wd_close(m, s, w, flags, ch_lds);
+  if (nblk > 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's values are written
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&flags[F_WDDONE], 1) == active - 1;
+    __syncthreads();
+    if (!last) return;
+    if (wd_get(&flags[F_WDSERIAL]))
+      wd_serial(w, n, s.tk, ch_lds);
+    else
+      wd_link(w, n, s.tk, ch_lds);
+    if (threadIdx.x == 0) flags[F_WDDONE] = 0;
   }
-  // (2) D2, element part: NCEle (NNODECODE of the three nodes times NOFF,
-  // both final since the candidate pass) and its area term NCEle*AREAS/2,
-  // written to the incidence slots of the element's three nodes
-  // (src/wetdry.F:1361-1380).  Independent of (1): one launch for both.
-  const int e = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (e >= m.ne) return;
-  const int ncele = s.nnodecode[m.nm[3 * e]] * s.nnodecode[m.nm[3 * e + 1]] *
-                    s.nnodecode[m.nm[3 * e + 2]] * s.noff[e];
-  const double a = (double)ncele * m.areas[e] / 2.0;
-  area_slot[m.slot[3 * e]] = a;
-  area_slot[m.slot[3 * e + 1]] = a;
-  area_slot[m.slot[3 * e + 2]] = a;
-}
-
-// D2: MJU, TotalArea, landlocked nodes, NODECODE update, NCCHANGE, and
-// H2 = DP + IFNLFA*ETA2 (src/wetdry.F:1361-1430, src/timestep.F:1097-1099).
-// MJU counts the wet incident elements: AREAS > 0, so NCEle = 1 exactly when
-// the slot's area term is non-zero.
-__global__ __launch_bounds__(256) void k_wd_d2(DevMesh m, DevState s,
-                                               const double* __restrict__ area_slot, int* flags,
-                                               double ifnlfa) {
-  // the block's slot range staged in LDS, as in k_mom_node
-  __shared__ double sa[NODE_STAGE];
-  const int r0 = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x;
-  const int i = r0 + threadIdx.x;
-  const int p0 = m.inc_ptr[r0];
-  const int n_st = m.inc_ptr[min(r0 + (int)blockDim.x, m.np)] - p0;
-  const bool staged = n_st <= NODE_STAGE;
-  if (staged)
-    for (int k = threadIdx.x; k < n_st; k += blockDim.x) sa[k] = area_slot[p0 + k];
+  // the candidate marks are clear between steps (every block has followed its
+  // links by now)
   __syncthreads();
-  if (i >= m.np) return;
-  int mju = 0;
-  double ta = 0.0;
-  const int q0 = staged ? p0 : 0;
-  const double* src = staged ? sa : area_slot;
-  for (int p = m.inc_ptr[i]; p < m.inc_ptr[i + 1]; ++p) {
-    const double a = src[p - q0];
-    mju += a != 0.0 ? 1 : 0;
-    ta = ta + a;
+  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    const int e = w.cid[k];
+    w.mask[e >> 6] = 0ull;
+    w.bcnt[e >> 8] = 0;
+    w.lc[e] = make_int2(-1, -1);
   }
-  int nn = s.nnodecode[i];
-  if (nn == 1 && mju == 0) nn = 0;
-  if (mju == 0) mju = 1;
-  s.mju[i] = mju;
-  s.totalarea[i] = ta;
-  if (nn != s.nodecode[i]) {
-    s.nodecode[i] = nn;
-    atomicOr(&flags[F_NCCHANGE], 1);
-  }
-  s.h2[i] = m.dp[i] + ifnlfa * s.eta2[i];
 }
 
 // computeAlpha (src/wetdry.F:1561-1652): ALPHAL of element e.

@@ -540,6 +540,311 @@ __global__ __launch_bounds__(256) void k_ncele(DevMesh m, DevState s, DevPatch p
                                s.nodecode[m.nm[3 * e + 2]] * s.noff[e]);
 }
 
+// ---------------------------------------------------------------- wet/dry
+// D1 (src/wetdry.F:234-285) of a node: its NODECODE, and ETA2 clipped.
+__device__ __forceinline__ int wd_dry(int nc, double dp, const WdPrm& q, double& eta2) {
+  if (nc == 1) {
+    const double htot = dp + eta2;
+    if (htot <= q.h0) {
+      if (htot < q.habsmin) eta2 = q.habsmin - dp;
+      nc = 0;
+    }
+  }
+  return nc;
+}
+
+// D1, W1 candidates (src/wetdry.F:332-818) and DE1 (src/wetdry.F:1110-1233).
+// NNODECODE of a node is its D1 code, or 1 if a candidate element, one whose
+// steady-flow velocity exceeds VELMIN, wets it: all elements of the patch's own
+// nodes are here.  ETA2 and NODECODE are left to the next pass, as other patches
+// read them here.  The candidates' friction updates depend on element order:
+// each leaves its TK_TMP value and local vertices at its element and sets its
+// bit in the candidate mask.
+__global__ __launch_bounds__(PATCH_THREADS) void k_wd_elem(DevMesh m, DevState s, DevPatch pp, WdPrm q,
+                                                           WdWork w, int* flags) {
+  __shared__ double se[PATCH_WIN], sp[PATCH_WIN];
+  __shared__ unsigned char sc[PATCH_WIN], sn[PATCH_WIN];
+  const int patch = xcd_tile(blockIdx.x, gridDim.x);
+  const int t = threadIdx.x;
+  const int i = t < PATCH_WIN ? pp.win[patch * PATCH_WIN + t] : -1;
+  const int ke = patch * PATCH_ELEMS + t;
+  const ushort4 lv = pp.lv[ke];
+  const int e = pp.el[ke];
+  const ushort2 c = t < PATCH_NODES ? pp.cspan[patch * PATCH_NODES + t] : make_ushort2(1, 0);
+  const int old = s.noff[e];
+  // this step's ALPHAL pass sets F_ALPHA again where needed; it rewrites ALPHAL
+  // while the last pass (or the host) left some value other than 1
+  if (blockIdx.x == 0 && t == 0) {
+    flags[F_ALPHA0] = flags[F_ALPHA];
+    flags[F_ALPHA] = 0;
+  }
+  if (i >= 0) {
+    double e2 = s.eta2[i];
+    const double dp = m.dp[i];
+    const int nc = wd_dry(s.nodecode[i], dp, q, e2);
+    se[t] = e2;
+    sp[t] = dp;
+    sc[t] = (unsigned char)nc;
+    sn[t] = (unsigned char)nc;
+  }
+  __syncthreads();
+  if (lv.w != 2) {
+    const int n[3] = {lv.x, lv.y, lv.z};
+    int noff = 1;
+    const double e1 = se[n[0]], e2 = se[n[1]], e3 = se[n[2]];
+    const double h1 = sp[n[0]] + e1, h2 = sp[n[1]] + e2, h3 = sp[n[2]] + e3;
+    const int c0 = sc[n[0]], c1 = sc[n[1]], c2 = sc[n[2]];
+    if (c0 + c1 + c2 == 2) {
+      int a = -1, b = -1, c = -1;
+      if (c0 == 1 && c1 == 1) { a = 0; b = 1; c = 2; }
+      else if (c1 == 1 && c2 == 1) { a = 1; b = 2; c = 0; }
+      else if (c2 == 1 && c0 == 1) { a = 2; b = 0; c = 1; }
+      const double ht[3] = {h1, h2, h3};
+      if (a >= 0 && ht[a] >= q.hoff && ht[b] >= q.hoff) {
+        const double et[3] = {e1, e2, e3};
+        int l123 = a;
+        if (et[b] > et[a]) l123 = b;
+        const int nm123 = m.nm[3 * (size_t)e + l123], nc = m.nm[3 * (size_t)e + c];
+        const double dy = m.y[nc] - m.y[nm123], dx = m.x[nc] - m.x[nm123];
+        const double deldist = __builtin_sqrt(dy * dy + dx * dx);
+        double deleta = et[l123] - et[c];
+        if (deleta < 0.0) deleta = 0.0;
+        const double H1 = et[l123] + sp[n[l123]];
+        const double fr = s.fric[nm123];
+        const double hyb = hybrid_term(q.hyb, H1);
+        const double tkwet = fmax(fr * (q.iflinbf + (q.velmin / H1) * (q.ifnlbf + hyb)), 0.0001);
+        const double vel = m.g * (deleta / deldist) / tkwet;
+        if (vel > q.velmin) {
+          sn[n[c]] = 1;
+          if (lv.w == 1) {
+            w.tkc[e] = fmin(fr * (q.iflinbf + (1.0 * vel / H1) * (q.ifnlbf + hyb)), q.tkmax);
+            w.lc[e].x = l123 | ((l123 == b ? a : b) << 2);
+            atomicOr(&w.mask[e >> 6], 1ull << (e & 63));
+            atomicAdd(&w.bcnt[e >> 8], 1);
+          }
+        }
+      }
+    }
+    const double HOFF = q.hoff;
+    if ((e1 >= e2) && (e2 > e3)) if ((h1 < HOFF) || (h2 < HOFF)) noff = 0;
+    if ((e2 >= e3) && (e3 > e1)) if ((h2 < HOFF) || (h3 < HOFF)) noff = 0;
+    if ((e3 >= e1) && (e1 > e2)) if ((h3 < HOFF) || (h1 < HOFF)) noff = 0;
+    if ((e1 >= e3) && (e3 > e2)) if ((h1 < HOFF) || (h3 < HOFF)) noff = 0;
+    if ((e2 >= e1) && (e1 > e3)) if ((h2 < HOFF) || (h1 < HOFF)) noff = 0;
+    if ((e3 >= e2) && (e2 > e1)) if ((h3 < HOFF) || (h2 < HOFF)) noff = 0;
+    // NOFF changes count toward NCCHANGE (src/wetdry.F:1428-1430)
+    if (lv.w == 1 && noff != old) {
+      s.noff[e] = noff;
+      atomicOr(&flags[F_NCCHANGE], 1);
+    }
+  }
+  __syncthreads();
+  if (c.y >= c.x) s.nnodecode[i] = sn[t];
+}
+
+// Does candidate code 3*e2+k2 (element e2, local vertex k2; lc = w.lc[e2].x)
+// update the TK of that vertex, i.e. is e2 a candidate and the vertex one of its
+// two wet nodes?
+__device__ __forceinline__ bool wd_touches(int lc, int k2) {
+  return lc >= 0 && (k2 == (lc & 3) || k2 == ((lc >> 2) & 3));
+}
+
+// Ordered W1 friction updates (src/wetdry.F:447-472), links of candidate element
+// e.  The reference visits the candidates in ascending element order; candidate
+// k sets TK(NM123) = MAX(TK_TMP, TK(NM123)), gives the partner the larger of the
+// two and takes it back if the partner was larger, so afterwards both of its
+// nodes hold M_k = max(TK_TMP_k, their values before k).  A node's value before k
+// is M_j of the nearest earlier candidate j on that node, or its value on entry.
+// The node incidence lists are sorted by element, so j and "k is the node's last
+// candidate" are found in the node's list.  Entry values fold into m0.  Done
+// here, by the elements' patches: by the few blocks of the ordered updates, the
+// scattered reads alone took 30 us at 4,000 candidates.
+__device__ __forceinline__ void wd_pred(const DevMesh& m, const DevState& s, const WdWork& w, int e,
+                                        int lc) {
+  double v = w.tkc[e];
+#pragma unroll 1
+  for (int j = 0; j < 2; ++j) {
+    const int l = (lc >> (2 * j)) & 3;
+    const int x = m.nm[3 * (size_t)e + l];
+    const int me = m.slot[3 * (size_t)e + l];
+    const int p0 = m.inc_ptr[x], p1 = m.inc_ptr[x + 1];
+    const double tk = s.tk[x];
+    int pe = -1;
+    bool last = true;
+    if (p1 - p0 <= WD_INC_MAX) {
+      // the node's whole list at once: its codes, then their marks
+      int code[WD_INC_MAX], c[WD_INC_MAX];
+#pragma unroll
+      for (int q = 0; q < WD_INC_MAX; ++q) code[q] = p0 + q < p1 ? m.inc[p0 + q] : -1;
+#pragma unroll
+      for (int q = 0; q < WD_INC_MAX; ++q) c[q] = code[q] >= 0 ? w.lc[code[q] / 3].x : -1;
+#pragma unroll
+      for (int q = 0; q < WD_INC_MAX; ++q)
+        if (wd_touches(c[q], code[q] % 3)) {
+          if (p0 + q < me) pe = code[q] / 3;  // the nearest earlier one is the last seen
+          if (p0 + q > me) last = false;
+        }
+    } else {
+      for (int q = me - 1; q >= p0; --q)
+        if (wd_touches(w.lc[m.inc[q] / 3].x, m.inc[q] % 3)) {
+          pe = m.inc[q] / 3;
+          break;
+        }
+      for (int q = me + 1; q < p1; ++q)
+        if (wd_touches(w.lc[m.inc[q] / 3].x, m.inc[q] % 3)) {
+          last = false;
+          break;
+        }
+    }
+    if (pe < 0) v = fmax(v, tk);
+    (&w.pred[e].x)[j] = pe;
+    (&w.wnode[e].x)[j] = last ? x : -1;
+  }
+  w.m0[e] = v;
+}
+
+// The candidates of tiles [WD_TILES r, WD_TILES (r+1)) in ascending element order
+// (w.cid, and their indices in w.lc); the last block also leaves their number.
+// Each block adds up the earlier tiles' counts itself.  A thread follows every
+// 256th tile, so that a front's candidates, which lie in consecutive tiles, are
+// spread over the block.
+__device__ __forceinline__ void wd_list(const DevMesh& m, const WdWork& w, int r, int nr, int* flags) {
+  __shared__ unsigned short cnt[WD_TILES];
+  __shared__ int ofs[WD_TILES];
+  __shared__ int wtot[PATCH_THREADS / 64], wbef[PATCH_THREADS / 64];
+  constexpr int PER = WD_TILES / PATCH_THREADS;
+  const int t = threadIdx.x;
+  const int nb = (m.ne + 255) / 256, b0 = WD_TILES * r;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int b = b0 + t + PATCH_THREADS * j;
+    cnt[t + PATCH_THREADS * j] = (unsigned short)(b < nb ? w.bcnt[b] : 0);
+  }
+  int bef = 0;
+#pragma unroll 8
+  for (int b = t; b < b0; b += PATCH_THREADS) bef += w.bcnt[b];
+  __syncthreads();
+  int sum = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) sum += cnt[PER * t + j];
+  int incl = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(incl, off, 64), u = __shfl_xor(bef, off, 64);
+    if ((t & 63) >= off) incl += v;
+    bef += u;
+  }
+  if ((t & 63) == 63) {
+    wtot[t >> 6] = incl;
+    wbef[t >> 6] = bef;
+  }
+  __syncthreads();
+  int k = incl - sum, all = 0;
+  for (int q = 0; q < PATCH_THREADS / 64; ++q) {
+    if (q < (t >> 6)) k += wtot[q];
+    k += wbef[q];
+    all += wtot[q] + wbef[q];
+  }
+  if (t == 0) {
+    if (r == 0) flags[F_WDSERIAL] = 0;
+    if (r == nr - 1) flags[F_NCAND] = all;
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    ofs[PER * t + j] = k;
+    k += cnt[PER * t + j];
+  }
+  __syncthreads();
+  ulonglong2 mk[PER][2];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int x = t + PATCH_THREADS * j;
+    if (cnt[x] == 0) continue;
+    const ulonglong2* p = reinterpret_cast<const ulonglong2*>(w.mask) + 2 * (size_t)(b0 + x);
+    mk[j][0] = p[0];
+    mk[j][1] = p[1];
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int x = t + PATCH_THREADS * j;
+    if (cnt[x] == 0) continue;
+    int at = ofs[x];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      for (unsigned long long y = q & 1 ? mk[j][q / 2].y : mk[j][q / 2].x; y; y &= y - 1) {
+        const int e = 256 * (b0 + x) + 64 * q + __ffsll((long long)y) - 1;
+        w.cid[at] = e;
+        w.lc[e].y = at++;
+      }
+  }
+}
+
+// D2: MJU, TotalArea, landlocked nodes, NODECODE update, NCCHANGE, and
+// H2 = DP + IFNLFA*ETA2 (src/wetdry.F:1361-1430, src/timestep.F:1097-1099), and
+// D1's ETA2; and the candidates' links and list.  MJU counts the wet elements of a node: AREAS > 0, so NCEle = 1
+// exactly when an element's term is non-zero.
+__global__ __launch_bounds__(PATCH_THREADS) void k_wd_d2(DevMesh m, DevState s, DevPatch pp, WdPrm q,
+                                                         WdWork w, int* flags, double ifnlfa) {
+  __shared__ double sa[PATCH_ELEMS];
+  __shared__ unsigned char sn[PATCH_WIN];
+  __shared__ __attribute__((aligned(4))) unsigned short code[3 * PATCH_ELEMS];
+  const int nlist = (int)gridDim.x - pp.n;
+  if ((int)blockIdx.x < nlist) {
+    wd_list(m, w, blockIdx.x, nlist, flags);
+    return;
+  }
+  const int patch = xcd_tile((int)blockIdx.x - nlist, pp.n);
+  const int t = threadIdx.x;
+  const int i = t < PATCH_WIN ? pp.win[patch * PATCH_WIN + t] : -1;
+  const int ke = patch * PATCH_ELEMS + t;
+  const ushort4 lv = pp.lv[ke];
+  const int e = pp.el[ke];
+  const ushort2 c = t < PATCH_NODES ? pp.cspan[patch * PATCH_NODES + t] : make_ushort2(1, 0);
+  const bool own = c.y >= c.x;
+  for (int k = t; k < 3 * PATCH_ELEMS / 2; k += PATCH_THREADS)
+    reinterpret_cast<unsigned*>(code)[k] =
+        reinterpret_cast<const unsigned*>(pp.code)[patch * (3 * PATCH_ELEMS / 2) + k];
+  const int noff = s.noff[e];
+  const double area = m.areas[e];
+  const int lc = lv.w == 1 ? w.lc[e].x : -1;
+  int nn = 0, old = 0;
+  double e2 = 0.0, dp = 0.0;
+  if (i >= 0) {
+    nn = s.nnodecode[i];
+    if (own) {
+      old = s.nodecode[i];
+      e2 = s.eta2[i];
+      dp = m.dp[i];
+    }
+    sn[t] = (unsigned char)nn;
+  }
+  __syncthreads();
+  if (lv.w != 2) {
+    const int ncele = sn[lv.x] * sn[lv.y] * sn[lv.z] * noff;
+    sa[t] = (double)ncele * area / 2.0;
+  }
+  __syncthreads();
+  if (lc >= 0) wd_pred(m, s, w, e, lc);
+  if (!own) return;
+  int mju = 0;
+  double ta = 0.0;
+  for (int p = c.x; p < c.y; ++p) {
+    const double a = sa[code[p] % PATCH_ELEMS];
+    mju += a != 0.0 ? 1 : 0;
+    ta = ta + a;
+  }
+  const double was = e2;
+  const int nc = wd_dry(old, dp, q, e2);  // D1
+  if (nn == 1 && mju == 0) nn = 0;
+  if (mju == 0) mju = 1;
+  s.mju[i] = mju;
+  s.totalarea[i] = ta;
+  if (nn != old) s.nodecode[i] = nn;
+  if (nn != nc || nc != old) atomicOr(&flags[F_NCCHANGE], 1);
+  if (e2 != was) s.eta2[i] = e2;
+  s.h2[i] = dp + ifnlfa * e2;
+}
+
 // --------------------------------------------------------------- momentum
 enum { MF_X, MF_Y, MF_U, MF_V, MF_H1, MF_EVM, MF_E1, MF_E2, MF_DP, MF_P1, MF_P2, MF_T1, MF_T2, MF_COUNT };
 static_assert(MF_COUNT == PATCH_MOM_FIELDS, "LDS of k_mom");

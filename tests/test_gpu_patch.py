@@ -105,3 +105,28 @@ def test_alphal_from_the_host(lumped):
         bad = compare(g, o, it)
         assert not bad, f"step {it}: " + "; ".join(bad)
     g.close()
+
+
+@pytest.mark.parametrize("shape", [(60, 40), (200, 160), (620, 230)])
+def test_many_wetting_candidates_bitexact(shape):
+    """Shallow water over a rough bed, wet and dry all over: thousands of wetting
+    candidates a step, in one block of the ordered friction updates and in many,
+    and in more than one list of element tiles (over 262,144 elements)."""
+    from adcirc_amd.model import cold_wetdry_state
+    case = _beach(*shape)
+    rng = np.random.default_rng(7)
+    m = case.mesh
+    dp = 0.15 + 0.25 * rng.standard_normal(m.x.shape[0])
+    case = dataclasses.replace(case, mesh=dataclasses.replace(m, dp=dp),
+                               run=dataclasses.replace(case.run, dtdp=0.5))
+    d = case_setup(case)
+    eta = 0.3 * np.sin(m.x / 700.0) * np.cos(m.y / 900.0)
+    e2, nc, nf = cold_wetdry_state(d, case.run, eta)
+    d["eta2_0"], d["nodecode0"], d["noff0"] = e2, nc, nf
+    g, o = build_pair(d, case.run)
+    log(f"rough bed {int(d['np'])} nodes, {int((nc == 0).sum())} dry: 6 steps bit-exact")
+    for it in range(1, 7):
+        step_pair(g, o, it)
+        bad = compare(g, o, it)
+        assert not bad, f"step {it}: " + "; ".join(bad)
+    g.close()
