@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -102,6 +103,8 @@ struct adcgpu_ctx {
   JcgRegPlan jreg[2];           // the register kernel with one and two chunks per block
   double* jhprev = nullptr;     // its neighbouring rows' previous d past the LDS
   unsigned* jlcol = nullptr;    // staged: the columns as 16-bit LDS positions, two slots a word
+  bool jcg_giveup = false;      // adcgpu_set_jcg_giveup
+  bool solving = false;         // solves enqueued since the stream was last waited for
   int jcg_limit = 0;            // caller's limit on JCG blocks per launch (0: the device's)
   bool jcg_mem = false;         // more row tiles than blocks: k_jcg_mem
   double *juo = nullptr, *jdpv = nullptr, *jndv = nullptr;  // k_jcg_mem's iterates
@@ -325,6 +328,27 @@ JcgArgs make_jcg_args(adcgpu_ctx* c, double* coef, const int* col, const int* nn
   return a;
 }
 
+// Contexts per device with solves enqueued that nobody has waited for yet.
+std::mutex g_solving_lock;
+int g_solving[64] = {0};
+
+// Counts the context in before a solve is enqueued; whether it is the only one.
+bool solve_begins(adcgpu_ctx* c) {
+  std::lock_guard<std::mutex> hold(g_solving_lock);
+  if (c->device >= 64) return false;
+  if (!c->solving) ++g_solving[c->device];
+  c->solving = true;
+  return g_solving[c->device] == 1;
+}
+
+// The context's stream has been waited for (or is about to be destroyed).
+void solves_done(adcgpu_ctx* c) {
+  if (!c->solving) return;
+  std::lock_guard<std::mutex> hold(g_solving_lock);
+  --g_solving[c->device];
+  c->solving = false;
+}
+
 // Chunks per block of the register kernel for the context's own launches; 0:
 // another kernel.  One chunk per block while the blocks are all resident: half
 // the rows per thread and twice the CUs; two beyond that.
@@ -372,7 +396,28 @@ int launch_jcg(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh, d
   } else {
     fn = u2 ? (const void*)k_jcg<true, false> : (const void*)k_jcg<false, false>;
   }
-  HIPCHK(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(threads), args, (unsigned)lds, c->stream));
+  // A cooperative launch waits for and is waited for through a queue of its own:
+  // 11 us idle before and 11 after, a tenth of a step at 20,000 nodes.  A small
+  // solve is launched like any kernel instead when nothing else of this process
+  // is solving: its blocks are all resident unless others hold the chip, and
+  // then it is given up after 2 ms and k_jcg_mem behind it (4 us when there is
+  // nothing to do) solves with two blocks.  Up to a quarter of the resident
+  // blocks, so that several processes' solves fit side by side; beyond, the gaps
+  // are a small part of the step, and two blocks would take too long.
+  const bool alone = solve_begins(c);
+  if (cpb > 0 && !u2 && alone && 4 * grid <= c->jcg_cap) {
+    JcgArgs f = make_jcg_args(c, coef, col, nneigh, rhs, u, n, itmax, zeta, eta2, eta1, nodecode,
+                              prescaled, defer_unscal, u2, 0);
+    f.hrows = f.halo = -1;
+    f.admit = a.admit = c->jbar + JCG_ADMIT_WORD;
+    a.admit_ticks = (long long)((double)c->clock_khz * 2.0);
+    HIPCHK(hipLaunchKernel(fn, dim3(grid), dim3(threads), args, lds, c->stream));
+    hipLaunchKernelGGL(k_jcg_mem, dim3(2), dim3(JCG_BLOCK), 0, c->stream, f);
+    if (int rc = check_launch("JCG")) return rc;
+  } else {
+    HIPCHK(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(threads), args, (unsigned)lds,
+                                      c->stream));
+  }
   if (c->profile) HIPCHK(hipEventRecord(c->jcg_events[c->ev_used++].second, c->stream));
   return 0;
 }
@@ -842,7 +887,9 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     A(&c->wd.xval, nwb * WD_XMAX);
   }
   A(&c->flags, F_COUNT); A(&c->jpart, jcg_part_doubles(c->nch)); A(&c->jsaved, 12);
-  A(&c->jbar, JCG_BAR_WORDS);
+  A(&c->jbar, JCG_BAR_WORDS + 1);
+  A(&c->juo, np); A(&c->jdpv, np);
+  c->jmem_n = np;
   if (!rc) {
     hipError_t e = hipStreamCreate(&c->stream);
     if (e != hipSuccess) rc = fail(ADCGPU_E_HIP, hipGetErrorString(e));
@@ -901,6 +948,7 @@ void adcgpu_destroy(adcgpu_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  solves_done(c);
   for (auto& ev : c->jcg_events) {
     (void)hipEventDestroy(ev.first);
     (void)hipEventDestroy(ev.second);
@@ -987,6 +1035,7 @@ int adcgpu_set_field(adcgpu_ctx* c, int f, const void* host, int64_t count) {
   if (f == ADCGPU_ALPHAL)
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_ALPHA, 1, 1);
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   return check_launch("set_field");
 }
 
@@ -1006,6 +1055,7 @@ int adcgpu_get_field(adcgpu_ctx* c, int f, void* host, int64_t count) {
     return fail(ADCGPU_E_ARG, "unknown field");
   }
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   return 0;
 }
 
@@ -1188,7 +1238,7 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceS
   }
   JcgPre pre{c->jw, c->jbar, jcg_barrier_words(c),
              reinterpret_cast<unsigned long long*>(c->jpart), jcg_part_doubles(c->nch),
-             c->flags, c->etas_prev, c->prm.warm_start,
+             c->flags, c->jcg_giveup ? JCG_ABORT : 0u, c->etas_prev, c->prm.warm_start,
              (c->prm.warm_start != 0 || c->ml_ready) ? 1 : 0, c->ml_corr, c->ml_u};
   // with ILump = 1 the explicit solve of the lumped GWCE ends the node pass; no JCG
   static_assert(RED_XTHREADS == 256, "the node pass forms EP with its 256 threads");
@@ -1323,6 +1373,7 @@ int adcgpu_last_numitr(adcgpu_ctx* c, int* numitr, int* ier) {
   int f[F_COUNT];
   HIPCHK(hipMemcpyAsync(f, c->flags, sizeof(f), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   if (numitr) *numitr = f[F_NUMITR];
   if (ier) *ier = f[F_IER];
   return flag_errors(f);
@@ -1331,6 +1382,7 @@ int adcgpu_last_numitr(adcgpu_ctx* c, int* numitr, int* ier) {
 int adcgpu_synchronize(adcgpu_ctx* c) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   return 0;
 }
 
@@ -1403,6 +1455,7 @@ static int run_read_flags(adcgpu_ctx* c, bool* error) {
   int f[F_COUNT];
   HIPCHK(hipMemcpyAsync(f, c->flags, sizeof(f), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   c->run_iters = f[F_ITSUM];
   c->run_rebuilds = f[F_NREBUILD];
   c->run_itmax = f[F_NITMAX];
@@ -1604,6 +1657,7 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
                               hipMemcpyHostToDevice, b->stream));
         b->hvalid[par] = true;
       }
+      for (int q : b->sm) (void)solve_begins(b->m[q]);
       for (size_t gi = 0; gi + 1 < b->gm.size() && !rc; ++gi) {
         const int q0 = b->gm[gi], q1 = b->gm[gi + 1];
         const int cpb = b->gcpb[gi];
@@ -1675,6 +1729,12 @@ int adcgpu_last_solve(adcgpu_ctx* c, double* out4) {
   const bool dual = c->prm.warm_start == 2 && c->prm.ilump == 0;
   out4[2] = dual ? s[10] : 0.0;
   out4[3] = dual ? s[11] : 0.0;
+  return 0;
+}
+
+int adcgpu_set_jcg_giveup(adcgpu_ctx* c, int on) {
+  if (!c) return fail(ADCGPU_E_ARG, "null context");
+  c->jcg_giveup = on != 0;
   return 0;
 }
 
@@ -2038,6 +2098,7 @@ int adcgpu_state_save(adcgpu_ctx* c, void* buf, int64_t bytes) {
     o += p.bytes;
   }
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   return 0;
 }
 
@@ -2056,6 +2117,7 @@ int adcgpu_state_load(adcgpu_ctx* c, const void* buf, int64_t bytes) {
     o += p.bytes;
   }
   HIPCHK(hipStreamSynchronize(c->stream));
+  solves_done(c);
   c->cur_it = hdr[3];
   c->coef_scaled = false;
   c->ncele_fresh = false;
@@ -2203,6 +2265,7 @@ int adcgpu_jcg(int n, int ndim, int maxnz, int32_t* jcoef, double* coef, double*
     double saved[8] = {0};
     if (c) {
       (void)hipMemcpy(saved, c->jsaved, sizeof(saved), hipMemcpyDeviceToHost);
+      solves_done(c);
       for (void* p : c->allocs) (void)hipFree(p);
       if (c->stream) (void)hipStreamDestroy(c->stream);
       delete c;
@@ -2251,6 +2314,7 @@ int adcgpu_jcg(int n, int ndim, int maxnz, int32_t* jcoef, double* coef, double*
     int fe[F_COUNT];
     HIPCHK(hipMemcpyAsync(fe, c->flags, sizeof(fe), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    solves_done(c);
     // the device copies are left as the failed launch left them; the
     // caller's arrays are untouched
     if (int erc = flag_errors(fe)) return erc;

@@ -809,6 +809,10 @@ __device__ void jcg_solve_mem(const JcgArgs& a, int bid, int nblocks) {
 }
 
 __global__ __launch_bounds__(JCG_BLOCK) void k_jcg_mem(JcgArgs a) {
+  // behind an ordinary launch of k_jcg_reg: only if that was given up
+  if (a.admit &&
+      !(__hip_atomic_load(a.admit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & JCG_ABORT))
+    return;
   jcg_solve_mem(a, (int)blockIdx.x, (int)gridDim.x);
 }
 

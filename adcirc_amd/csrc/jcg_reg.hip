@@ -44,19 +44,38 @@ namespace adcgpu {
 
 // A bounded wait: every 64th unsuccessful poll looks at the error flag and at
 // the clock; a wait that runs out sets the flag, so every block drains.
+//
+// An ordinary launch (JcgArgs::admit) may find part of the chip taken by blocks
+// that wait for it in turn.  Each block counts itself in when it starts; a wait
+// that lasts admit_ticks while some block has not started gives the launch up: the
+// abort bit is set (by an exchange on the count, so never once all have
+// started), every block leaves, and nothing but scratch has been written: no block
+// gets past the first iteration's partials before all have started.  k_jcg_mem,
+// enqueued behind, then solves the system with two blocks.
 struct BoundedWait {
+  const JcgArgs& a;
   int* err;
-  long long ticks;
+  unsigned blocks;
   long long t0 = 0;
   unsigned polls = 0;
-  __device__ BoundedWait(int* e, long long t) : err(e), ticks(t) {}
+  __device__ BoundedWait(const JcgArgs& a, int nblocks)
+      : a(a), err(a.flags + F_ERROR), blocks((unsigned)nblocks) {}
   __device__ __forceinline__ bool more() {
     if ((++polls & 63u) != 0) return true;
     if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_BARRIER)
       return false;
     const long long t = wall_clock64();
     if (t0 == 0) t0 = t;
-    if (t - t0 <= ticks) return true;
+    if (a.admit) {
+      unsigned v = __hip_atomic_load(a.admit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (v & JCG_ABORT) return false;
+      if (v != blocks) {
+        if (t - t0 <= a.admit_ticks) return true;
+        return !__hip_atomic_compare_exchange_strong(a.admit, &v, v | JCG_ABORT, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (t - t0 <= a.barrier_ticks) return true;
     atomicOr(err, ERR_BARRIER);
     return false;
   }
@@ -173,11 +192,11 @@ struct RegShared {
 // The eigenvalue block: the adaptive estimate of each iteration beside the
 // row blocks' products, then the same scalars as theirs.
 template <bool DUAL>
-__device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh) {
+__device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh, int nblocks) {
   __shared__ double tri1[JCG_MAX_ITMAX], tri2[JCG_MAX_ITMAX];
   const int t = threadIdx.x;
   const int nch = (a.n + RED_CHUNK - 1) / RED_CHUNK;
-  BoundedWait wait(a.flags + F_ERROR, a.barrier_ticks);
+  BoundedWait wait(a, nblocks);
   auto slot = [&](int k) { return a.part + (size_t)k * 4 * (nch + 1) + 4 * nch; };
   for (int in = 0; in <= a.itmax; ++in) {
     const bool need_u = reg_need_u(sh.L, in);
@@ -222,14 +241,17 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
     jcg_init_state(sh.L, a);
     sh.failed = 0;
     sh.ovn = 0;
+    // (a launch given up before this block started is left at once)
+    if (a.admit && (atomicAdd(a.admit, 1u) & JCG_ABORT)) sh.failed = 1;
   }
   if (bid == nrb) {  // the last block: no rows
     __syncthreads();
-    jcg_reg_eig<DUAL>(a, sh);
+    if (sh.failed) return;
+    jcg_reg_eig<DUAL>(a, sh, nblocks);
     return;
   }
   const int lane = t & 63, wave = t >> 6;
-  BoundedWait wait(a.flags + F_ERROR, a.barrier_ticks);
+  BoundedWait wait(a, nblocks);
   const int tile = xcd_tile(bid, nrb);
   const int c0 = tile * CPB;  // first chunk
   const int t0 = tile * TILE, t1 = t0 + TILE < np ? t0 + TILE : np;
@@ -283,6 +305,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
   };
   stage(a.w);
   __syncthreads();
+  if (sh.failed) return;
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int i = ROW(q);

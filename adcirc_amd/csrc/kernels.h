@@ -19,6 +19,8 @@ constexpr int JCG_BAR_GROUP = 16;        // blocks per first-level barrier count
 constexpr int JCG_BAR_STRIDE = 64;       // words between barrier counters (256 B)
 constexpr int JCG_BAR_WORDS = 10240;     // barrier words: (groups + 2) * JCG_BAR_STRIDE
                                           // + blocks * JCG_HALO_STRIDE
+constexpr int JCG_ADMIT_WORD = JCG_BAR_WORDS;  // admission word of an ordinary launch:
+constexpr unsigned JCG_ABORT = 0x80000000u;      // blocks started, or given up
 constexpr int JCG_HALO_STRIDE = 16;      // words between per-tile halo flags (64 B)
 constexpr int JCG_HALO_MAX = 2;          // widest halo (tiles each side) waited on by flags
 constexpr int JCG_MAX_ITMAX = 256;       // tridiagonal history length (itmax)
@@ -312,6 +314,9 @@ struct JcgArgs {
   int halo;           // row tiles each side whose pseudo-residual a tile's rows read;
                       // -1: wait for all tiles (a grid barrier) after each update
   long long barrier_ticks;  // longest grid-barrier wait, in wall-clock ticks
+  unsigned* admit;          // an ordinary launch of k_jcg_reg: the admission word
+                            // (JCG_ABORT); null: a cooperative launch
+  long long admit_ticks;    // the longest wait for blocks that have not started
   int* flags;
   double* eta2;       // optional: ETA2 = NODECODE*(ETAS+0)+ETA1
   const double* eta1;
@@ -357,6 +362,7 @@ struct JcgPre {
   unsigned long long* part;  // k_jcg_reg's partial slots, marked empty here
   int part_words;
   int* flags;
+  unsigned admit0;    // the admission word's first value (0, or JCG_ABORT: give up)
   double* etas_prev;  // the previous step's ETAS (kept when keep_prev != 0)
   int warm;           // 1: start JCG from 2*ETAS - ETAS_prev instead of ETAS;
                       // 2: also form the learned start ETAS + ml_corr into ml_u

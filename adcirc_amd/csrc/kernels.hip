@@ -216,6 +216,7 @@ __global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s,
   const int i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (i < pre.barrier_words) pre.barrier[i] = 0u;
   if (i < pre.part_words) pre.part[i] = JCG_EMPTY;
+  if (i == 0) pre.barrier[JCG_ADMIT_WORD] = pre.admit0;
   const bool rebuilt = pre.flags[F_REBUILT] != 0;
   const bool in = i < m.np;
   const int bi = in ? m.bnd_index[i] : -1;

@@ -394,6 +394,11 @@ int adcgpu_jcg_noalloc(int n, int ndim, int maxnz, int32_t *jcoef, double *coef,
  * failure-handling tests (a tiny bound forces the error path from the host). */
 int adcgpu_set_wait_limit(double seconds);
 
+/* For tests: with on != 0 the context's small solves, which are launched like
+ * any kernel, are given up as if the chip were taken, so that the two-block
+ * solver enqueued behind them does the work (same results). */
+int adcgpu_set_jcg_giveup(adcgpu_ctx* ctx, int on);
+
 /* ---- synthetic forcing ---- */
 /* Holland (1980) vortex wind stress / rho0 and pressure head at time t on
  * the context's nodes, written into WSX2, WSY2, PR2 on the device. */
