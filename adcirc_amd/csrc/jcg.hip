@@ -648,6 +648,7 @@ __device__ __forceinline__ void jcg_solve(const JcgArgs& a, int bid, int nblocks
 
 template <bool DUAL, bool STAGED>
 __global__ __launch_bounds__(JCG_BLOCK) void k_jcg(JcgArgs a) {
+  if (a.flags[F_ERROR] & ERR_INPUT) return;
   jcg_solve<DUAL, STAGED>(a, (int)blockIdx.x, (int)gridDim.x);
 }
 
@@ -809,6 +810,7 @@ __device__ void jcg_solve_mem(const JcgArgs& a, int bid, int nblocks) {
 }
 
 __global__ __launch_bounds__(JCG_BLOCK) void k_jcg_mem(JcgArgs a) {
+  if (a.flags[F_ERROR] & ERR_INPUT) return;
   // behind an ordinary launch of k_jcg_reg: only if that was given up
   if (a.admit &&
       !(__hip_atomic_load(a.admit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & JCG_ABORT))

@@ -77,7 +77,8 @@ enum { F_NCCHANGE = 0, F_NUMITR = 2, F_IER, F_ERROR, F_NCAND, F_ITSUM, F_NREBUIL
        F_ALPHA0,   // F_ALPHA as the last step left it
        F_WDDONE,   // k_wd_chain's blocks that have ended
        F_COUNT = 16 };
-enum { ERR_DIAG = 1, ERR_BARRIER = 4, ERR_ELEV = 8, ERR_NONFINITE = 16 };
+enum { ERR_DIAG = 1, ERR_BARRIER = 4, ERR_ELEV = 8, ERR_NONFINITE = 16,
+       ERR_INPUT = 32 };  // a system the drop-in refuses (k_na_compact): not solved
 // device scalar slots
 enum { S_EP = 0, S_COUNT = 8 };
 
@@ -398,6 +399,16 @@ __global__ void k_wd_alpha(DevMesh m, DevState s, int* flags, double slim);
 __global__ void k_h2(int np, const double* dp, const double* eta2, double ifnlfa, double* h2);
 template <bool ALPHA, typename CT>
 __global__ void k_mom(DevMesh m, DevState s, DevPatch pp, MomPrm q);
+// The drop-in's system: the caller's ELLPACK arrays (n rows, maxnz columns)
+// compacted to the solver's layout, and the solved rows back.  `check` holds the
+// smallest row*4 + kind of a row that is refused; ERR_INPUT is set with it.
+enum { NA_NODIAG = 0, NA_BADCOL = 1, NA_ZERODIAG = 2, NA_NEGDIAG = 3 };
+constexpr int NA_OK = 0x7fffffff;
+__global__ void k_na_compact(int n, int maxnz, const double* in_coef, const int* in_jcoef,
+                             double* coef, int* col, int* nneigh, int* check, int* flags);
+__global__ void k_na_scatter(int n, int maxnz, double* in_coef, const int* in_jcoef,
+                             const double* coef, const int* flags);
+__global__ void k_na_clear(int* flags, int* check, unsigned* bar, int bar_words);
 __global__ void k_fill_u32(unsigned* p, unsigned v, int n);
 __global__ void k_fill_i32(int* p, int v, int n);
 __global__ void k_total_area(DevMesh m, DevState s);

@@ -54,21 +54,24 @@ static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 // row by row: per row, no diagonal (402) before a column index above n
 // (argument error) before a zero diagonal (401) before a negative one
 // (unsupported).  `check` holds the smallest row*4 + kind seen.
-enum { NA_NODIAG = 0, NA_BADCOL = 1, NA_ZERODIAG = 2, NA_NEGDIAG = 3 };
 
 // One row per thread: the ELLPACK row of the caller's (n, maxnz) arrays,
 // copied with leading dimension n, compacted to the solver's layout with the
 // diagonal first and the padding (jcoef <= 0) dropped, columns 0-based.
 __global__ __launch_bounds__(256) void k_na_compact(int n, int maxnz, const double* in_coef,
                                                     const int* in_jcoef, double* coef, int* col,
-                                                    int* nneigh, int* check) {
+                                                    int* nneigh, int* check, int* flags) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  auto refuse = [&](int kind) {
+    atomicMin(check, i * 4 + kind);
+    atomicOr(&flags[F_ERROR], ERR_INPUT);
+  };
   int dj = -1;
   for (int j = 0; j < maxnz; ++j)
     if (in_jcoef[(size_t)j * n + i] == i + 1) dj = j;
   if (dj < 0) {
-    atomicMin(check, i * 4 + NA_NODIAG);
+    refuse(NA_NODIAG);
     return;
   }
   int k = 0;
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(256) void k_na_compact(int n, int maxnz, const doub
   for (int j = 0; j < maxnz; ++j) {
     const int v = in_jcoef[(size_t)j * n + i];
     if (v > n) {
-      atomicMin(check, i * 4 + NA_BADCOL);
+      refuse(NA_BADCOL);
       return;
     }
     if (j != dj && v > 0) {
@@ -89,15 +92,16 @@ __global__ __launch_bounds__(256) void k_na_compact(int n, int maxnz, const doub
   }
   nneigh[i] = k;
   const double d = coef[i];
-  if (d == 0.0) atomicMin(check, i * 4 + NA_ZERODIAG);
-  else if (d < 0.0) atomicMin(check, i * 4 + NA_NEGDIAG);
+  if (d == 0.0) refuse(NA_ZERODIAG);
+  else if (d < 0.0) refuse(NA_NEGDIAG);
 }
 
 // The solved (unscaled) rows back to the caller's positions.
 __global__ __launch_bounds__(256) void k_na_scatter(int n, int maxnz, double* in_coef,
-                                                    const int* in_jcoef, const double* coef) {
+                                                    const int* in_jcoef, const double* coef,
+                                                    const int* flags) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || flags[F_ERROR] != 0) return;
   int dj = -1;
   for (int j = 0; j < maxnz; ++j)
     if (in_jcoef[(size_t)j * n + i] == i + 1) dj = j;
@@ -111,7 +115,7 @@ __global__ __launch_bounds__(256) void k_na_scatter(int n, int maxnz, double* in
 
 __global__ void k_na_clear(int* flags, int* check, unsigned* bar, int bar_words) {
   for (int k = threadIdx.x; k < F_COUNT; k += blockDim.x) flags[k] = 0;
-  if (threadIdx.x == 0) *check = 0x7fffffff;
+  if (threadIdx.x == 0) *check = NA_OK;
   for (int k = threadIdx.x; k < bar_words; k += blockDim.x) bar[k] = 0u;
 }
 
@@ -200,27 +204,22 @@ int adcgpu_jcg_noalloc(int n, int ndim, int maxnz, int32_t* jcoef, double* coef,
   const int bar_words = jcg_barrier_words_for(grid);
   hipLaunchKernelGGL(k_na_clear, dim3(1), dim3(256), 0, st, dflags, dcheck, dbar, bar_words);
   // the caller's n rows of each column (leading dimension ndim)
-  NACHK(hipMemcpy2DAsync(in_coef, (size_t)n * 8, coef, (size_t)ndim * 8, (size_t)n * 8, maxnz,
-                         hipMemcpyHostToDevice, st));
-  NACHK(hipMemcpy2DAsync(in_jcoef, (size_t)n * 4, jcoef, (size_t)ndim * 4, (size_t)n * 4, maxnz,
-                         hipMemcpyHostToDevice, st));
+  auto columns = [&](void* dst, size_t dpitch, const void* src, size_t spitch, size_t bytes,
+                     hipMemcpyKind kind) {
+    return dpitch == spitch ? hipMemcpyAsync(dst, src, spitch * maxnz, kind, st)
+                            : hipMemcpy2DAsync(dst, dpitch, src, spitch, bytes, maxnz, kind, st);
+  };
+  NACHK(columns(in_coef, (size_t)n * 8, coef, (size_t)ndim * 8, (size_t)n * 8,
+                hipMemcpyHostToDevice));
+  NACHK(columns(in_jcoef, (size_t)n * 4, jcoef, (size_t)ndim * 4, (size_t)n * 4,
+                hipMemcpyHostToDevice));
   NACHK(hipMemcpyAsync(drhs, rhs, (size_t)n * 8, hipMemcpyHostToDevice, st));
   NACHK(hipMemcpyAsync(du, u, (size_t)n * 8, hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(k_na_compact, dim3((n + 255) / 256), dim3(256), 0, st, n, maxnz,
-                     (const double*)in_coef, (const int*)in_jcoef, dcoef, dcol, dnn, dcheck);
+                     (const double*)in_coef, (const int*)in_jcoef, dcoef, dcol, dnn, dcheck,
+                     dflags);
   NACHK(hipGetLastError());
-  int chk = 0;
-  NACHK(hipMemcpyAsync(&chk, dcheck, sizeof(int), hipMemcpyDeviceToHost, st));
-  NACHK(hipStreamSynchronize(st));
-  if (chk != 0x7fffffff) {
-    switch (chk & 3) {
-      case NA_NODIAG: return 402;
-      case NA_BADCOL: return na_fail(ADCGPU_E_ARG, "jcoef out of range");
-      case NA_ZERODIAG: return 401;
-      default: return na_fail(ADCGPU_E_UNSUPPORTED, "negative diagonal (nonsymmetric scaling)");
-    }
-  }
-  JcgArgs a;
+  JcgArgs a = {};
   a.n = n;
   jcg_tolerances(a, itmax, rparm[0]);
   a.coef = dcoef;
@@ -248,18 +247,29 @@ int adcgpu_jcg_noalloc(int n, int ndim, int maxnz, int32_t* jcoef, double* coef,
   void* args[] = {&a};
   NACHK(hipLaunchCooperativeKernel((const void*)k_jcg<false, false>, dim3(grid), dim3(JCG_BLOCK), args,
                                    0, st));
-  int f[F_COUNT];
+  hipLaunchKernelGGL(k_na_scatter, dim3((n + 255) / 256), dim3(256), 0, st, n, maxnz, in_coef,
+                     (const int*)in_jcoef, (const double*)dcoef, (const int*)dflags);
+  NACHK(hipGetLastError());
+  // the outcome: saved state, (barrier words,) flags and the input check
+  int f[F_COUNT], chk = NA_OK;
   double saved[8];
   NACHK(hipMemcpyAsync(f, dflags, sizeof(f), hipMemcpyDeviceToHost, st));
   NACHK(hipMemcpyAsync(saved, dsaved, sizeof(saved), hipMemcpyDeviceToHost, st));
   NACHK(hipStreamSynchronize(st));
+  if (f[F_ERROR] & ERR_INPUT) {
+    NACHK(hipMemcpyAsync(&chk, dcheck, sizeof(int), hipMemcpyDeviceToHost, st));
+    NACHK(hipStreamSynchronize(st));
+    switch (chk & 3) {
+      case NA_NODIAG: return 402;
+      case NA_BADCOL: return na_fail(ADCGPU_E_ARG, "jcoef out of range");
+      case NA_ZERODIAG: return 401;
+      default: return na_fail(ADCGPU_E_UNSUPPORTED, "negative diagonal (nonsymmetric scaling)");
+    }
+  }
   if (f[F_ERROR] & ERR_BARRIER) return na_fail(ADCGPU_E_HIP, "JCG wait timed out");
   if (f[F_ERROR] & ERR_DIAG) return na_fail(ADCGPU_E_DIAG, "diagonal <= 0");
-  hipLaunchKernelGGL(k_na_scatter, dim3((n + 255) / 256), dim3(256), 0, st, n, maxnz, in_coef,
-                     (const int*)in_jcoef, (const double*)dcoef);
-  NACHK(hipGetLastError());
-  NACHK(hipMemcpy2DAsync(coef, (size_t)ndim * 8, in_coef, (size_t)n * 8, (size_t)n * 8, maxnz,
-                         hipMemcpyDeviceToHost, st));
+  NACHK(columns(coef, (size_t)ndim * 8, in_coef, (size_t)n * 8, (size_t)n * 8,
+                hipMemcpyDeviceToHost));
   NACHK(hipMemcpyAsync(rhs, drhs, (size_t)n * 8, hipMemcpyDeviceToHost, st));
   NACHK(hipMemcpyAsync(u, du, (size_t)n * 8, hipMemcpyDeviceToHost, st));
   NACHK(hipStreamSynchronize(st));
