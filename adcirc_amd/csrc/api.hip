@@ -916,6 +916,9 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     if (e == hipSuccess)
       e = hipFuncSetAttribute((const void*)k_wd_chain, hipFuncAttributeMaxDynamicSharedMemorySize,
                               WD_CHAIN_LDS);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)k_wd_chain_batch,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, WD_CHAIN_LDS);
     if (e != hipSuccess) rc = fail(ADCGPU_E_UNSUPPORTED, std::string("LDS request: ") +
                                                          hipGetErrorString(e));
   }
@@ -1198,6 +1201,35 @@ struct GwceStep {
   int slot0 = 0;
 };
 
+static RhsPrm rhs_prm(const adcgpu_ctx* c, bool fric) {
+  const bool lumped = c->prm.ilump != 0;
+  return RhsPrm{c->ifnlfa, c->ifnlct, c->ifnlcat, lumped ? 4.0 : 2.0, lumped ? 0.0 : 1.0,
+                fric ? 1 : 0, c->prm.nws};
+}
+static WdPrm wd_prm(const adcgpu_ctx* c) {
+  return WdPrm{c->prm.h0, c->habsmin, c->hoff, c->prm.velmin, c->iflinbf, c->ifnlbf, c->tkmax,
+               c->hyb};
+}
+static JcgPre jcg_pre(const adcgpu_ctx* c) {
+  return JcgPre{c->jw, c->jbar, jcg_barrier_words(c),
+                reinterpret_cast<unsigned long long*>(c->jpart), jcg_part_doubles(c->nch),
+                c->flags, c->jcg_giveup ? JCG_ABORT : 0u, c->etas_prev, c->prm.warm_start,
+                (c->prm.warm_start != 0 || c->ml_ready) ? 1 : 0, c->ml_corr, c->ml_u};
+}
+static int wd_chain_blocks(const adcgpu_ctx* c) {
+  return std::min(nblk(c->ne, WD_BLOCK), WD_CHAIN_BLOCKS);
+}
+static int wd_list_blocks(const adcgpu_ctx* c) { return nblk(nblk(c->ne, 256), WD_TILES); }
+
+// NCEle of every patch element, which the momentum pass left unless the flags
+// changed since.
+static void ncele_ready(adcgpu_ctx* c) {
+  if (c->ncele_fresh) return;
+  hipLaunchKernelGGL(k_ncele, dim3(nblk(c->patch.nq, 256)), dim3(256), 0, c->stream, c->mesh(),
+                     c->state(), c->patch);
+  c->ncele_fresh = true;
+}
+
 // The GWCE assembly up to the solve: matrix, right-hand side, time-level
 // rotation, the learned start's inputs, and the node pass that scales the
 // rows for JCG (or, with ILump = 1, solves).
@@ -1205,15 +1237,8 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceS
   const int np = c->np;
   const bool lumped = c->prm.ilump != 0;
   const double* rw = c->coef_scaled ? (const double*)c->jw : nullptr;
-  // the passes multiply each element's terms by its NCEle, which the momentum
-  // pass left unless the flags changed since
-  if (!c->ncele_fresh) {
-    hipLaunchKernelGGL(k_ncele, dim3(nblk(c->patch.nq, 256)), dim3(256), 0, c->stream, c->mesh(),
-                       c->state(), c->patch);
-    c->ncele_fresh = true;
-  }
-  const RhsPrm q{c->ifnlfa, c->ifnlct, c->ifnlcat, lumped ? 4.0 : 2.0, lumped ? 0.0 : 1.0,
-                 fric ? 1 : 0, c->prm.nws};
+  ncele_ready(c);
+  const RhsPrm q = rhs_prm(c, fric);
   const dim3 pg(c->patch.n), pb(PATCH_THREADS);
   const size_t lds = patch_lds_bytes(PATCH_GWCE_FIELDS, PATCH_GWCE_TERMS, c->patch.wmax);
   auto gwce = lumped ? (c->mixed ? k_gwce<true, float> : k_gwce<true, double>)
@@ -1238,10 +1263,7 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceS
       hipLaunchKernelGGL(k_ml_collect, dim3(nblk(c->ml_collect, 128)), dim3(256), 0, c->stream,
                          in, c->smp, slot0, c->ml_collect, c->cur_it);
   }
-  JcgPre pre{c->jw, c->jbar, jcg_barrier_words(c),
-             reinterpret_cast<unsigned long long*>(c->jpart), jcg_part_doubles(c->nch),
-             c->flags, c->jcg_giveup ? JCG_ABORT : 0u, c->etas_prev, c->prm.warm_start,
-             (c->prm.warm_start != 0 || c->ml_ready) ? 1 : 0, c->ml_corr, c->ml_u};
+  const JcgPre pre = jcg_pre(c);
   // with ILump = 1 the explicit solve of the lumped GWCE ends the node pass; no JCG
   static_assert(RED_XTHREADS == 256, "the node pass forms EP with its 256 threads");
   hipLaunchKernelGGL(lumped ? k_rhs_node<true> : k_rhs_node<false>, dim3(nblk(np, 256)), dim3(256),
@@ -1319,15 +1341,13 @@ static int wetdry_device(adcgpu_ctx* c, bool alpha_pass) {
                        c->ifnlfa, c->h2);
     return check_launch("h2");
   }
-  const WdPrm q{c->prm.h0, c->habsmin, c->hoff, c->prm.velmin, c->iflinbf, c->ifnlbf, c->tkmax,
-                c->hyb};
+  const WdPrm q = wd_prm(c);
   const DevPatch& pp = c->patch;
   hipLaunchKernelGGL(k_wd_elem, dim3(pp.n), dim3(PATCH_THREADS), 0, c->stream, c->mesh(),
                      c->state(), pp, q, c->wd, c->flags);
-  hipLaunchKernelGGL(k_wd_d2, dim3(pp.n + nblk(nblk(ne, 256), WD_TILES)), dim3(PATCH_THREADS), 0, c->stream, c->mesh(),
+  hipLaunchKernelGGL(k_wd_d2, dim3(pp.n + wd_list_blocks(c)), dim3(PATCH_THREADS), 0, c->stream, c->mesh(),
                      c->state(), pp, q, c->wd, c->flags, c->ifnlfa);
-  const int nwb = std::min((ne + WD_BLOCK - 1) / WD_BLOCK, WD_CHAIN_BLOCKS);
-  hipLaunchKernelGGL(k_wd_chain, dim3(nwb), dim3(WD_BLOCK), WD_CHAIN_LDS, c->stream, c->mesh(),
+  hipLaunchKernelGGL(k_wd_chain, dim3(wd_chain_blocks(c)), dim3(WD_BLOCK), WD_CHAIN_LDS, c->stream, c->mesh(),
                      c->state(), c->wd, c->flags);
   if (alpha_pass)
     hipLaunchKernelGGL(k_wd_alpha, dim3(nblk(ne, 256)), dim3(256), 0, c->stream, c->mesh(),
@@ -1416,10 +1436,7 @@ static int run_prepare(adcgpu_ctx* c, int nsteps, const double* eta_bc_table,
     HIPCHK(hipMemcpyAsync(c->eta_bc_table, eta_bc_table, (size_t)nsteps * c->neta * 8,
                           hipMemcpyHostToDevice, c->stream));
   }
-  // F_ITSUM and F_NREBUILD are adjacent: one fill clears both
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_ITSUM, 0, 2);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_NITMAX, 0, 1);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_MLUSED, 0, 1);
+  hipLaunchKernelGGL(k_run_clear, dim3(1), dim3(64), 0, c->stream, c->flags);
   return check_launch("run set-up");
 }
 
@@ -1498,6 +1515,8 @@ int adcgpu_run(adcgpu_ctx* c, int it0, int nsteps, const double* eta_bc_table,
 
 // ---- batches of contexts (ensembles, uneven meshes)
 struct adcgpu_batch {
+  MemberArgs* margs = nullptr;   // [3][n]: the first step's, then by step parity
+  MemberArgs* hmargs = nullptr;  // pinned host copy
   std::vector<adcgpu_ctx*> m;
   int device = 0;
   hipStream_t stream = nullptr;
@@ -1519,6 +1538,8 @@ void batch_free(adcgpu_batch* b) {
   if (b->dfirst) (void)hipFree(b->dfirst);
   if (b->dargs) (void)hipFree(b->dargs);
   if (b->hargs) (void)hipHostFree(b->hargs);
+  if (b->margs) (void)hipFree(b->margs);
+  if (b->hmargs) (void)hipHostFree(b->hmargs);
   delete b;
 }
 }  // namespace
@@ -1591,6 +1612,9 @@ int adcgpu_batch_create(adcgpu_ctx* const* members, int n, adcgpu_batch** out) {
   }
   int rc = 0;
   if (!first.empty()) rc = upload(&b->dfirst, first);
+  if (!rc) rc = dmalloc(&b->margs, 3 * b->m.size());
+  if (!rc && hipHostMalloc((void**)&b->hmargs, 3 * b->m.size() * sizeof(MemberArgs), 0) != hipSuccess)
+    rc = fail(ADCGPU_E_HIP, "pinned host buffer");
   if (!rc && !b->sm.empty()) rc = dmalloc(&b->dargs, 2 * b->sm.size());
   if (!rc && !b->sm.empty() &&
       hipHostMalloc((void**)&b->hargs, 2 * b->sm.size() * sizeof(JcgArgs), 0) != hipSuccess)
@@ -1608,6 +1632,44 @@ void adcgpu_batch_destroy(adcgpu_batch* b) {
   (void)hipSetDevice(b->device);
   (void)hipStreamSynchronize(b->stream);
   batch_free(b);
+}
+
+// A member whose passes can go out with the others': the wet/dry step with the
+// consistent GWCE, without what takes passes of its own (flux boundaries, tidal
+// potential, the learned start and its samples).
+static bool batch_plain(const adcgpu_ctx* c) {
+  return c->prm.ilump == 0 && c->prm.nolifa == 2 && !c->nfluxf && !c->has_rad && !c->ctip &&
+         c->prm.warm_start != 2 && c->ml_collect == 0;
+}
+
+// run_step_assemble's host work for such a member, and its arguments.
+static int batch_member(adcgpu_ctx* c, int it, const double* holland, MemberArgs* a) {
+  if (int rc = begin_step(c, it, nullptr)) return rc;
+  ncele_ready(c);
+  a->restore_w = c->coef_scaled ? (const double*)c->jw : nullptr;
+  c->coef_scaled = false;
+  a->f = fric_prm(c);
+  std::swap(c->eta1, c->eta2);
+  std::swap(c->h1, c->h2);
+  a->m = c->mesh();
+  a->s = c->state();
+  a->pp = c->patch;
+  a->rq = rhs_prm(c, true);
+  a->wq = wd_prm(c);
+  a->wd = c->wd;
+  a->mq = MomPrm{c->ifnlct, c->prm.nws, 0, c->errorelev, c->flags};
+  a->pre = jcg_pre(c);
+  if (holland)
+    for (int k = 0; k < 13; ++k) a->hol.v[k] = holland[k];
+  a->eta_bc = c->neta > 0 ? c->eta_bc_table : c->eta_bc;
+  a->ep_part = c->ep_part;
+  a->scal = c->scal;
+  a->ifnlfa = c->ifnlfa;
+  a->dt = c->prm.dtdp;
+  a->nch = c->nch;
+  a->nlist = wd_list_blocks(c);
+  a->nchain = wd_chain_blocks(c);
+  return check_launch("batch member");
 }
 
 int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* eta_bc_tables,
@@ -1633,8 +1695,58 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
   for (int k = 0; k < n && !rc; ++k) rc = run_prepare(b->m[k], nsteps, table(k), hol(k));
   std::vector<GwceStep> g(n);
   const size_t ns = b->sm.size();
+  // The members whose passes go out in one launch each, alike in precision and
+  // forcing; the others' go out one by one.  A pass of one member fills a small
+  // part of the chip and costs a launch: eight members of 50,000 nodes took 750 us
+  // a step beside the solves.
+  std::vector<int> tog;
+  std::vector<char> in(n, 0);
+  for (int k = 0; k < n; ++k) {
+    const adcgpu_ctx* c = b->m[k];
+    if (!batch_plain(c)) continue;
+    if (!tog.empty() && (b->m[tog[0]]->mixed != c->mixed || !hol(tog[0]) != !hol(k))) continue;
+    tog.push_back(k);
+  }
+  if (tog.size() < 2) tog.clear();
+  for (int k : tog) in[k] = 1;
+  const unsigned nt = (unsigned)tog.size();
+  int np_max = 0, nch_max = 0, patches = 0, listed = 0, chain = 0, wmax = 0;
+  for (int k : tog) {
+    const adcgpu_ctx* c = b->m[k];
+    np_max = std::max(np_max, c->np);
+    nch_max = std::max(nch_max, c->nch);
+    patches = std::max(patches, c->patch.n);
+    listed = std::max(listed, c->patch.n + wd_list_blocks(c));
+    chain = std::max(chain, wd_chain_blocks(c));
+    wmax = std::max(wmax, c->patch.wmax);
+  }
+  const dim3 pg(patches, nt), pb(PATCH_THREADS), ng(nblk(np_max, 256), nt), nb(256);
+  const bool mixed = nt && b->m[tog[0]]->mixed, met = nt && hol(tog[0]);
   for (int s = 0; s < nsteps && !rc; ++s) {
-    for (int k = 0; k < n && !rc; ++k) rc = run_step_assemble(b->m[k], it0 + s, s, hol(k), &g[k]);
+    for (int k = 0; k < n && !rc; ++k)
+      if (!in[k]) rc = run_step_assemble(b->m[k], it0 + s, s, hol(k), &g[k]);
+    // the arguments are the first step's, then alternate with the time levels
+    const size_t slot = (s == 0 ? 0 : 1 + (s & 1)) * (size_t)n;
+    for (unsigned k = 0; k < nt && !rc; ++k) {
+      MemberArgs x;
+      std::memset(&x, 0, sizeof(x));
+      rc = batch_member(b->m[tog[k]], it0 + s, hol(tog[k]), &x);
+      if (s < 3) b->hmargs[slot + k] = x;
+      g[tog[k]] = GwceStep{};
+      g[tog[k]].solve = true;
+    }
+    const MemberArgs* const ma = b->margs + slot;
+    if (!rc && nt) {
+      if (s < 3)
+        HIPCHK(hipMemcpyAsync(b->margs + slot, b->hmargs + slot, nt * sizeof(MemberArgs),
+                              hipMemcpyHostToDevice, b->stream));
+      if (met) hipLaunchKernelGGL(k_holland_batch, ng, nb, 0, b->stream, ma, it0 + s);
+      hipLaunchKernelGGL(mixed ? k_gwce_batch<float> : k_gwce_batch<double>, pg, pb,
+                         patch_lds_bytes(PATCH_GWCE_FIELDS, PATCH_GWCE_TERMS, wmax), b->stream, ma);
+      hipLaunchKernelGGL(k_lhs_ep_batch, dim3(nch_max, nt), dim3(RED_THREADS), 0, b->stream, ma);
+      hipLaunchKernelGGL(k_rhs_node_batch, ng, nb, 0, b->stream, ma, s);
+      rc = check_launch("batch assembly");
+    }
     // the solves: this step's arguments (they alternate with the time-level
     // rotation, so each parity's are uploaded once), then one launch per group
     const int par = s & 1;
@@ -1692,7 +1804,18 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
                                                          hipGetErrorString(e));
       }
     }
-    for (int k = 0; k < n && !rc; ++k) rc = run_step_finish(b->m[k], g[k]);
+    for (int k = 0; k < n && !rc; ++k)
+      rc = in[k] ? gwce_finish(b->m[k], g[k], true) : run_step_finish(b->m[k], g[k]);
+    if (!rc && nt) {
+      hipLaunchKernelGGL(k_wd_elem_batch, pg, pb, 0, b->stream, ma);
+      hipLaunchKernelGGL(k_wd_d2_batch, dim3(listed, nt), pb, 0, b->stream, ma);
+      hipLaunchKernelGGL(k_wd_chain_batch, dim3(chain, nt), dim3(WD_BLOCK), WD_CHAIN_LDS, b->stream,
+                         ma);
+      hipLaunchKernelGGL(mixed ? k_mom_batch<float> : k_mom_batch<double>, pg, pb,
+                         patch_lds_bytes(PATCH_MOM_FIELDS, PATCH_MOM_TERMS, wmax), b->stream, ma,
+                         it0 + s);
+      rc = check_launch("batch step");
+    }
     if (!rc && (s & 63) == 63)
       for (int k = 0; k < n && !rc; ++k) {
         bool error = false;

@@ -371,6 +371,39 @@ struct JcgPre {
   const double* ml_corr;  // warm == 2: the network's correction per node
   double* ml_u;           // warm == 2: the learned start, scaled
 };
+// One member of a batch: what the passes of a step take.  `s` is the state after
+// the GWCE's time-level rotation (k_gwce runs before it: ETA1 and ETA2, H1 and H2
+// change places there).  What changes with the step is passed beside it.
+struct MemberArgs {
+  DevMesh m;
+  DevState s;
+  DevPatch pp;
+  RhsPrm rq;
+  FricPrm f;
+  WdPrm wq;
+  WdWork wd;
+  MomPrm mq;
+  JcgPre pre;
+  HollandPrm hol;
+  const double* restore_w;
+  const double* eta_bc;  // the run's table, or the one row of a member without boundary
+  double* ep_part;
+  double* scal;
+  double ifnlfa, dt;
+  int nch, nlist, nchain;
+};
+// The passes for all members in one launch each: member blockIdx.y, whose blocks
+// past its own number leave at once.
+template <typename CT>
+__global__ void k_gwce_batch(const MemberArgs* a);
+__global__ void k_lhs_ep_batch(const MemberArgs* a);
+__global__ void k_rhs_node_batch(const MemberArgs* a, int step);
+__global__ void k_holland_batch(const MemberArgs* a, int it);
+__global__ void k_wd_elem_batch(const MemberArgs* a);
+__global__ void k_wd_d2_batch(const MemberArgs* a);
+__global__ void k_wd_chain_batch(const MemberArgs* a);
+template <typename CT>
+__global__ void k_mom_batch(const MemberArgs* a, int it);
 template <bool LUMPED>
 __global__ void k_rhs_node(DevMesh m, DevState s, const double* eta_bc, int nch,
                            const double* ep_part, double* scal, JcgPre pre);
@@ -411,6 +444,7 @@ __global__ void k_na_scatter(int n, int maxnz, double* in_coef, const int* in_jc
 __global__ void k_na_clear(int* flags, int* check, unsigned* bar, int bar_words);
 __global__ void k_fill_u32(unsigned* p, unsigned v, int n);
 __global__ void k_fill_i32(int* p, int v, int n);
+__global__ void k_run_clear(int* flags);  // the counters of a run
 __global__ void k_total_area(DevMesh m, DevState s);
 
 }  // namespace adcgpu

@@ -96,6 +96,14 @@ __global__ __launch_bounds__(256) void k_holland(int np, const double* __restric
   if (i >= np) return;
   holland_node(i, x, y, p, wsx, wsy, pr);
 }
+__global__ __launch_bounds__(256) void k_holland_batch(const MemberArgs* __restrict__ a, int it) {
+  const MemberArgs& x = a[blockIdx.y];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= x.m.np) return;
+  HollandPrm p = x.hol;
+  p.t = it * x.dt;
+  holland_node(i, x.m.x, x.m.y, p, x.s.wsx2, x.s.wsy2, x.s.pr2);
+}
 
 // --------------------------------------------------------------- GWCE
 // EP chunk partials: sum COEF(i,1)^2 (src/gwce.F:646-650) in the fixed blocked
@@ -103,10 +111,10 @@ __global__ __launch_bounds__(256) void k_holland(int np, const double* __restric
 // then the chunk tree).  The matrix is rebuilt when NCChange > 0 and NCChange is
 // then cleared (src/gwce.F:427-428): this pass, between the kernel that tests it
 // and those that set it, clears it and leaves F_REBUILT for the node pass.
-__global__ __launch_bounds__(RED_THREADS) void k_lhs_ep(DevMesh m, DevState s, int* flags,
-                                                        double* __restrict__ ep_part) {
+__device__ __forceinline__ void lhs_ep_block(const DevMesh& m, const DevState& s, int* flags,
+                                             double* __restrict__ ep_part, int bid, int nch) {
   __shared__ double lds[8];
-  const int chunk = xcd_tile(blockIdx.x, gridDim.x);
+  const int chunk = xcd_tile(bid, nch);
   const int base = chunk * RED_CHUNK + threadIdx.x;
   double d[RED_PER_THREAD];
 #pragma unroll
@@ -119,12 +127,22 @@ __global__ __launch_bounds__(RED_THREADS) void k_lhs_ep(DevMesh m, DevState s, i
   for (int r = 0; r < RED_PER_THREAD; ++r) acc = acc + d[r] * d[r];
   const double tot = chunk_tree(acc, lds);
   if (threadIdx.x == 0) ep_part[chunk] = tot;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (bid == 0 && threadIdx.x == 0) {
     const int ncc = flags[F_NCCHANGE];
     flags[F_REBUILT] = ncc > 0 ? 1 : 0;
     if (ncc > 0) flags[F_NREBUILD] += 1;
     flags[F_NCCHANGE] = 0;
   }
+}
+
+__global__ __launch_bounds__(RED_THREADS) void k_lhs_ep(DevMesh m, DevState s, int* flags,
+                                                        double* __restrict__ ep_part) {
+  lhs_ep_block(m, s, flags, ep_part, blockIdx.x, gridDim.x);
+}
+__global__ __launch_bounds__(RED_THREADS) void k_lhs_ep_batch(const MemberArgs* __restrict__ a) {
+  const MemberArgs& x = a[blockIdx.y];
+  if ((int)blockIdx.x >= x.nch) return;
+  lhs_ep_block(x.m, x.s, x.pre.flags, x.ep_part, blockIdx.x, x.nch);
 }
 
 // The off-diagonals of a solve whose unscaling was deferred, scaled and
@@ -207,13 +225,14 @@ __global__ __launch_bounds__(256) void k_flux_shift(DevMesh m, DevState s,
 // chunk partials, by every block that has a row that takes it (a boundary row,
 // or a zero diagonal).
 template <bool LUMPED>
-__global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s,
-                           const double* __restrict__ eta_bc, int nch,
-                           const double* __restrict__ ep_part, double* __restrict__ scal,
-                           JcgPre pre) {
+__device__ __forceinline__ void rhs_node_block(const DevMesh& m, DevState s,
+                                               const double* __restrict__ eta_bc, int nch,
+                                               const double* __restrict__ ep_part,
+                                               double* __restrict__ scal, const JcgPre& pre, int bid,
+                                               int nb) {
   __shared__ double lds[4];
   __shared__ double ep_s;
-  const int i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int i = xcd_tile(bid, nb) * blockDim.x + threadIdx.x;
   if (i < pre.barrier_words) pre.barrier[i] = 0u;
   if (i < pre.part_words) pre.part[i] = JCG_EMPTY;
   if (i == 0) pre.barrier[JCG_ADMIT_WORD] = pre.admit0;
@@ -224,14 +243,14 @@ __global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s,
   const bool take_ep = dg == 0.0 || bi >= 0;
   double ep = 0.0;
   // block 0 also keeps EP for the steps without a rebuild
-  if (__syncthreads_or(take_ep || (rebuilt && blockIdx.x == 0))) {
+  if (__syncthreads_or(take_ep || (rebuilt && bid == 0))) {
     if (rebuilt) {
       double acc = 0.0;
       for (int c = threadIdx.x; c < nch; c += RED_XTHREADS) acc = acc + ep_part[c];
       const double tot = block_tree(acc, lds);
       if (threadIdx.x == 0) {
         ep_s = __builtin_sqrt(tot / (double)m.np);
-        if (blockIdx.x == 0) scal[S_EP] = ep_s;
+        if (bid == 0) scal[S_EP] = ep_s;
       }
       __syncthreads();
       ep = ep_s;
@@ -313,6 +332,21 @@ __global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s,
   pre.w[i] = w;
   s.gwce_lv[i] = rhs * w;
 }
+
+template <bool LUMPED>
+__global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s,
+                                                  const double* __restrict__ eta_bc, int nch,
+                                                  const double* __restrict__ ep_part,
+                                                  double* __restrict__ scal, JcgPre pre) {
+  rhs_node_block<LUMPED>(m, s, eta_bc, nch, ep_part, scal, pre, blockIdx.x, gridDim.x);
+}
+__global__ __launch_bounds__(256) void k_rhs_node_batch(const MemberArgs* __restrict__ a, int step) {
+  const MemberArgs& x = a[blockIdx.y];
+  const int nb = (x.m.np + 255) / 256;
+  if ((int)blockIdx.x >= nb) return;
+  rhs_node_block<false>(x.m, x.s, x.eta_bc + (size_t)step * x.m.neta, x.nch, x.ep_part, x.scal, x.pre,
+                        blockIdx.x, nb);
+}
 template __global__ void k_rhs_node<false>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre);
 template __global__ void k_rhs_node<true>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre);
 
@@ -366,7 +400,7 @@ __device__ __forceinline__ void wd_add(int* u, int& nu, int f) {
 }
 
 __device__ __forceinline__ void wd_close(const DevMesh& m, const DevState& s, const WdWork& w,
-                                         int* flags, double* wc_lds) {
+                                         int* flags, double* wc_lds, int bid, int nb) {
   double* sv = wc_lds;                                                       // [2][WD_BLOCK]
   unsigned long long* sE = reinterpret_cast<unsigned long long*>(sv + 2 * WD_BLOCK);  // [2][WD_XW][WD_BLOCK]
   int* sF = reinterpret_cast<int*>(sE + 2 * WD_XW * WD_BLOCK);               // [2][WD_BLOCK]
@@ -376,7 +410,7 @@ __device__ __forceinline__ void wd_close(const DevMesh& m, const DevState& s, co
   const int n = flags[F_NCAND];
   const int nblk = (n + WD_BLOCK - 1) / WD_BLOCK;
   const int l = threadIdx.x;
-  for (int b = blockIdx.x; b < nblk; b += gridDim.x) {
+  for (int b = bid; b < nblk; b += nb) {
     const int base = b * WD_BLOCK, k = base + l;
     for (int i = l; i < WD_HASH; i += WD_BLOCK) hkey[i] = -1;
     if (l == 0) xn = 0;
@@ -605,14 +639,15 @@ __device__ __forceinline__ void wd_link(const WdWork& w, int n, double* __restri
 // pass before): block closure by as many blocks as have candidates; the block
 // that ends last joins the blocks' values and writes TK, so that no block waits
 // for another.  Dynamic LDS: WD_CHAIN_LDS bytes.
-__global__ __launch_bounds__(WD_BLOCK) void k_wd_chain(DevMesh m, DevState s, WdWork w, int* flags) {
+__device__ __forceinline__ void wd_chain_block(const DevMesh& m, const DevState& s, const WdWork& w,
+                                               int* flags, int bid, int nb) {
   extern __shared__ double ch_lds[];
   __shared__ int last;
   const int n = flags[F_NCAND];
   const int nblk = (n + WD_BLOCK - 1) / WD_BLOCK;
-  const int active = min(nblk, (int)gridDim.x);
-  if ((int)blockIdx.x >= active) return;
-  wd_close(m, s, w, flags, ch_lds);
+  const int active = min(nblk, nb);
+  if (bid >= active) return;
+  wd_close(m, s, w, flags, ch_lds, bid, nb);
   if (nblk > 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's values are written
     __syncthreads();
@@ -634,6 +669,15 @@ __global__ __launch_bounds__(WD_BLOCK) void k_wd_chain(DevMesh m, DevState s, Wd
     w.bcnt[e >> 8] = 0;
     w.lc[e] = make_int2(-1, -1);
   }
+}
+
+__global__ __launch_bounds__(WD_BLOCK) void k_wd_chain(DevMesh m, DevState s, WdWork w, int* flags) {
+  wd_chain_block(m, s, w, flags, blockIdx.x, gridDim.x);
+}
+__global__ __launch_bounds__(WD_BLOCK) void k_wd_chain_batch(const MemberArgs* __restrict__ a) {
+  const MemberArgs& x = a[blockIdx.y];
+  if ((int)blockIdx.x >= x.nchain) return;
+  wd_chain_block(x.m, x.s, x.wd, x.pre.flags, blockIdx.x, x.nchain);
 }
 
 // computeAlpha (src/wetdry.F:1561-1652): ALPHAL of element e.
@@ -693,6 +737,11 @@ __global__ __launch_bounds__(256) void k_fill_u32(unsigned* p, unsigned v, int n
 __global__ __launch_bounds__(256) void k_fill_i32(int* p, int v, int n) {
   int i = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
+}
+
+__global__ void k_run_clear(int* flags) {
+  if (threadIdx.x == 0)
+    flags[F_ITSUM] = flags[F_NREBUILD] = flags[F_NITMAX] = flags[F_MLUSED] = 0;
 }
 
 // TotalArea / MJU at cold start (src/mesh.F:3360-3400), node gather.

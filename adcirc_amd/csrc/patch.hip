@@ -311,13 +311,13 @@ __device__ __forceinline__ void lhs_terms(const double* sh, int ws, int n1, int 
 // (src/itpackv.F:2394-2400, 2460-2479): the previous solve left them as they were
 // before its scaling.
 template <bool LUMPED, typename CT>
-__global__ __launch_bounds__(PATCH_THREADS, 3) void k_gwce(DevMesh m, DevState s, DevPatch pp, RhsPrm q,
-                                                           FricPrm f, const int* flags,
-                                                           const double* __restrict__ restore_w) {
+__device__ __forceinline__ void gwce_block(const DevMesh& m, const DevState& s, const DevPatch& pp,
+                                           const RhsPrm& q, const FricPrm& f, const int* flags,
+                                           const double* __restrict__ restore_w, int bid) {
   extern __shared__ double sh[];
   __shared__ __attribute__((aligned(4))) unsigned short code[3 * PATCH_ELEMS];
   __shared__ int win_own[PATCH_NODES];
-  const int patch = xcd_tile(blockIdx.x, gridDim.x);
+  const int patch = xcd_tile(bid, pp.n);
   const int t = threadIdx.x, ws = pp.wmax, np = m.np;
   // what does not hang on another load first: the block's lists
   const int i = t < PATCH_WIN ? pp.win[patch * PATCH_WIN + t] : -1;
@@ -472,6 +472,26 @@ __global__ __launch_bounds__(PATCH_THREADS, 3) void k_gwce(DevMesh m, DevState s
     }
   }
 }
+
+template <bool LUMPED, typename CT>
+__global__ __launch_bounds__(PATCH_THREADS, 3) void k_gwce(DevMesh m, DevState s, DevPatch pp, RhsPrm q,
+                                                           FricPrm f, const int* flags,
+                                                           const double* __restrict__ restore_w) {
+  gwce_block<LUMPED, CT>(m, s, pp, q, f, flags, restore_w, blockIdx.x);
+}
+template <typename CT>
+__global__ __launch_bounds__(PATCH_THREADS, 3) void k_gwce_batch(const MemberArgs* __restrict__ a) {
+  const MemberArgs& x = a[blockIdx.y];
+  if ((int)blockIdx.x >= x.pp.n) return;
+  DevState s = x.s;  // before the time levels change places
+  s.eta1 = x.s.eta2;
+  s.eta2 = x.s.eta1;
+  s.h1 = x.s.h2;
+  s.h2 = x.s.h1;
+  gwce_block<false, CT>(x.m, s, x.pp, x.rq, x.f, x.pre.flags, x.restore_w, blockIdx.x);
+}
+template __global__ void k_gwce_batch<double>(const MemberArgs*);
+template __global__ void k_gwce_batch<float>(const MemberArgs*);
 template __global__ void k_gwce<false, double>(DevMesh, DevState, DevPatch, RhsPrm, FricPrm, const int*, const double*);
 template __global__ void k_gwce<true, double>(DevMesh, DevState, DevPatch, RhsPrm, FricPrm, const int*, const double*);
 template __global__ void k_gwce<false, float>(DevMesh, DevState, DevPatch, RhsPrm, FricPrm, const int*, const double*);
@@ -560,11 +580,11 @@ __device__ __forceinline__ int wd_dry(int nc, double dp, const WdPrm& q, double&
 // read them here.  The candidates' friction updates depend on element order:
 // each leaves its TK_TMP value and local vertices at its element and sets its
 // bit in the candidate mask.
-__global__ __launch_bounds__(PATCH_THREADS) void k_wd_elem(DevMesh m, DevState s, DevPatch pp, WdPrm q,
-                                                           WdWork w, int* flags) {
+__device__ __forceinline__ void wd_elem_block(const DevMesh& m, const DevState& s, const DevPatch& pp,
+                                              const WdPrm& q, const WdWork& w, int* flags, int bid) {
   __shared__ double se[PATCH_WIN], sp[PATCH_WIN];
   __shared__ unsigned char sc[PATCH_WIN], sn[PATCH_WIN];
-  const int patch = xcd_tile(blockIdx.x, gridDim.x);
+  const int patch = xcd_tile(bid, pp.n);
   const int t = threadIdx.x;
   const int i = t < PATCH_WIN ? pp.win[patch * PATCH_WIN + t] : -1;
   const int ke = patch * PATCH_ELEMS + t;
@@ -574,7 +594,7 @@ __global__ __launch_bounds__(PATCH_THREADS) void k_wd_elem(DevMesh m, DevState s
   const int old = s.noff[e];
   // this step's ALPHAL pass sets F_ALPHA again where needed; it rewrites ALPHAL
   // while the last pass (or the host) left some value other than 1
-  if (blockIdx.x == 0 && t == 0) {
+  if (bid == 0 && t == 0) {
     flags[F_ALPHA0] = flags[F_ALPHA];
     flags[F_ALPHA] = 0;
   }
@@ -640,6 +660,16 @@ __global__ __launch_bounds__(PATCH_THREADS) void k_wd_elem(DevMesh m, DevState s
   }
   __syncthreads();
   if (c.y >= c.x) s.nnodecode[i] = sn[t];
+}
+
+__global__ __launch_bounds__(PATCH_THREADS) void k_wd_elem(DevMesh m, DevState s, DevPatch pp, WdPrm q,
+                                                           WdWork w, int* flags) {
+  wd_elem_block(m, s, pp, q, w, flags, blockIdx.x);
+}
+__global__ __launch_bounds__(PATCH_THREADS) void k_wd_elem_batch(const MemberArgs* __restrict__ a) {
+  const MemberArgs& x = a[blockIdx.y];
+  if ((int)blockIdx.x >= x.pp.n) return;
+  wd_elem_block(x.m, x.s, x.pp, x.wq, x.wd, x.pre.flags, blockIdx.x);
 }
 
 // Does candidate code 3*e2+k2 (element e2, local vertex k2; lc = w.lc[e2].x)
@@ -783,17 +813,17 @@ __device__ __forceinline__ void wd_list(const DevMesh& m, const WdWork& w, int r
 // H2 = DP + IFNLFA*ETA2 (src/wetdry.F:1361-1430, src/timestep.F:1097-1099), and
 // D1's ETA2; and the candidates' links and list.  MJU counts the wet elements of a node: AREAS > 0, so NCEle = 1
 // exactly when an element's term is non-zero.
-__global__ __launch_bounds__(PATCH_THREADS) void k_wd_d2(DevMesh m, DevState s, DevPatch pp, WdPrm q,
-                                                         WdWork w, int* flags, double ifnlfa) {
+__device__ __forceinline__ void wd_d2_block(const DevMesh& m, const DevState& s, const DevPatch& pp,
+                                            const WdPrm& q, const WdWork& w, int* flags, double ifnlfa,
+                                            int bid, int nlist) {
   __shared__ double sa[PATCH_ELEMS];
   __shared__ unsigned char sn[PATCH_WIN];
   __shared__ __attribute__((aligned(4))) unsigned short code[3 * PATCH_ELEMS];
-  const int nlist = (int)gridDim.x - pp.n;
-  if ((int)blockIdx.x < nlist) {
-    wd_list(m, w, blockIdx.x, nlist, flags);
+  if (bid < nlist) {
+    wd_list(m, w, bid, nlist, flags);
     return;
   }
-  const int patch = xcd_tile((int)blockIdx.x - nlist, pp.n);
+  const int patch = xcd_tile(bid - nlist, pp.n);
   const int t = threadIdx.x;
   const int i = t < PATCH_WIN ? pp.win[patch * PATCH_WIN + t] : -1;
   const int ke = patch * PATCH_ELEMS + t;
@@ -843,6 +873,16 @@ __global__ __launch_bounds__(PATCH_THREADS) void k_wd_d2(DevMesh m, DevState s, 
   if (nn != nc || nc != old) atomicOr(&flags[F_NCCHANGE], 1);
   if (e2 != was) s.eta2[i] = e2;
   s.h2[i] = dp + ifnlfa * e2;
+}
+
+__global__ __launch_bounds__(PATCH_THREADS) void k_wd_d2(DevMesh m, DevState s, DevPatch pp, WdPrm q,
+                                                         WdWork w, int* flags, double ifnlfa) {
+  wd_d2_block(m, s, pp, q, w, flags, ifnlfa, blockIdx.x, (int)gridDim.x - pp.n);
+}
+__global__ __launch_bounds__(PATCH_THREADS) void k_wd_d2_batch(const MemberArgs* __restrict__ a) {
+  const MemberArgs& x = a[blockIdx.y];
+  if ((int)blockIdx.x >= x.pp.n + x.nlist) return;
+  wd_d2_block(x.m, x.s, x.pp, x.wq, x.wd, x.pre.flags, x.ifnlfa, blockIdx.x, x.nlist);
 }
 
 // --------------------------------------------------------------- momentum
@@ -1115,11 +1155,12 @@ __device__ __forceinline__ void mom_node(const DevMesh& m, const DevState& s, co
 // the element's wet/dry ALPHAL is formed here first (nothing reads it between
 // the wet/dry pass and this one).
 template <bool ALPHA, typename CT>
-__global__ __launch_bounds__(PATCH_THREADS, 5) void k_mom(DevMesh m, DevState s, DevPatch pp, MomPrm q) {
+__device__ __forceinline__ void mom_block(const DevMesh& m, const DevState& s, const DevPatch& pp,
+                                          const MomPrm& q, int bid) {
   extern __shared__ double sh[];
   __shared__ __attribute__((aligned(4))) unsigned short code[3 * PATCH_ELEMS];
   __shared__ unsigned char wet[PATCH_WIN];
-  const int patch = xcd_tile(blockIdx.x, gridDim.x);
+  const int patch = xcd_tile(bid, pp.n);
   const int t = threadIdx.x, ws = pp.wmax;
   const int i = t < PATCH_WIN ? pp.win[patch * PATCH_WIN + t] : -1;
   const int ke = patch * PATCH_ELEMS + t;
@@ -1213,6 +1254,21 @@ __global__ __launch_bounds__(PATCH_THREADS, 5) void k_mom(DevMesh m, DevState s,
   }
   mom_node(m, s, q, nd, i, mx, my);
 }
+
+template <bool ALPHA, typename CT>
+__global__ __launch_bounds__(PATCH_THREADS, 5) void k_mom(DevMesh m, DevState s, DevPatch pp, MomPrm q) {
+  mom_block<ALPHA, CT>(m, s, pp, q, blockIdx.x);
+}
+template <typename CT>
+__global__ __launch_bounds__(PATCH_THREADS, 5) void k_mom_batch(const MemberArgs* __restrict__ a, int it) {
+  const MemberArgs& x = a[blockIdx.y];
+  if ((int)blockIdx.x >= x.pp.n) return;
+  MomPrm q = x.mq;
+  q.it = it;
+  mom_block<true, CT>(x.m, x.s, x.pp, q, blockIdx.x);
+}
+template __global__ void k_mom_batch<double>(const MemberArgs*, int);
+template __global__ void k_mom_batch<float>(const MemberArgs*, int);
 template __global__ void k_mom<false, double>(DevMesh, DevState, DevPatch, MomPrm);
 template __global__ void k_mom<true, double>(DevMesh, DevState, DevPatch, MomPrm);
 template __global__ void k_mom<false, float>(DevMesh, DevState, DevPatch, MomPrm);
