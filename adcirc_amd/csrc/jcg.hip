@@ -218,7 +218,7 @@ __device__ __forceinline__ void jcg_scalars(ItLocal& L, const JcgArgs& a, double
     L.cmold = cmold_in;
     L.delnnm = delnnm;
     jcg_pstop(L, need_u ? unorm_s : 1.0, delnnm);
-    if (!L.halt) jcg_parcon(L, dtnrm);
+    if (!L.halt) jcg_parcon(L, dtnrm, L.in);
   }
   __syncthreads();
 }
@@ -229,7 +229,7 @@ __device__ __forceinline__ void jcg_scalars(ItLocal& L, const JcgArgs& a, double
 __device__ __forceinline__ void jcg_eig_step(ItLocal& L, const JcgArgs& a, double* tri1,
                                              double* tri2, int in) {
   if (threadIdx.x < 64) {
-    jcg_eig_wave(L, tri1, tri2, in);
+    jcg_eig_wave<false>(L, tri1, tri2, in);
     if (threadIdx.x == 0) {
       a.saved[6 + 2 * (in & 1)] = L.cme;
       a.saved[7 + 2 * (in & 1)] = L.cmold;

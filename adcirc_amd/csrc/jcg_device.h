@@ -69,20 +69,67 @@ __device__ __forceinline__ double jcg_determ(int n, const double* tri1, const do
   return a1;
 }
 
+// The tridiagonal's values for the evaluations of one zbrent call.  REG: up to
+// JCG_TRI_REG rows in registers, last row first (from LDS, whose latency exceeds
+// the recurrence's, an evaluation takes twice as long); for kernels with
+// registers to spare.
+constexpr int JCG_TRI_REG = 20;
+template <bool REG>
+struct JcgTri {
+  int n;
+  const double *tri1, *tri2;
+  double p[REG ? JCG_TRI_REG : 1], q[REG ? JCG_TRI_REG : 1];  // tri1, tri2 of row n-1-k
+  __device__ __forceinline__ JcgTri(int n_, const double* t1, const double* t2)
+      : n(n_), tri1(t1), tri2(t2) {
+    if (REG) {
+#pragma unroll
+      for (int k = 0; k < (REG ? JCG_TRI_REG : 1); ++k) {
+        const int r = n - 1 - k > 0 ? n - 1 - k : 0;
+        p[k] = tri1[r];
+        q[k] = tri2[r];
+      }
+    }
+  }
+  template <int K>
+  __device__ __forceinline__ double rows(double a1, double a2, double x) const {
+    if constexpr (K < JCG_TRI_REG) {
+      if (K < n) return rows<K + 1>((p[K] - x) * a1 + q[K - 1] * a2, a1, x);
+    }
+    return a1;
+  }
+  // determ: the same operations in the same order from either place
+  __device__ __forceinline__ double operator()(double x) const {
+    if constexpr (REG) {
+      if (n <= JCG_TRI_REG) {
+        const double a2 = p[0] - x;
+        return rows<2>((p[1] - x) * a2 + q[0], a2, x);
+      }
+    }
+    return jcg_determ(n, tri1, tri2, x);
+  }
+};
+
+// A condition that holds in all lanes or in none, as a scalar branch.
+__device__ __forceinline__ bool in_wave(bool c) { return __ballot(c) != 0ull; }
+
 // zbrent (src/itpackv.F:2521-2781) with eps = 0; returns ier, result in *pb.
 // Called by a whole wave, whose lanes all follow the same path; lanes 0 and 1
-// evaluate the two ends of the interval at once.
+// evaluate the two ends of the interval at once.  The three quotients of the
+// interpolation are formed side by side, whether the step takes them or not:
+// the call is one chain of latencies.
+template <bool REG>
 __device__ __forceinline__ int jcg_zbrent(int n, const double* tri1, const double* tri2, double t, int maxfn,
                           double a, double* pb) {
   double b = 1.0, c = 0, d = 0, e = 0, p, qq, r, ss, fa, fb, fc = 0, tol, rm, rone, temp;
   int ic = 2;
   const double eps = 0.0;
+  const JcgTri<REG> determ(n, tri1, tri2);
   {
-    const double f = jcg_determ(n, tri1, tri2, (threadIdx.x & 63) == 1 ? b : a);
+    const double f = determ((threadIdx.x & 63) == 1 ? b : a);
     fa = __shfl(f, 0, 64);
     fb = __shfl(f, 1, 64);
   }
-  if ((fa > 0.0 && fb > 0.0) || (fa < 0.0 && fb < 0.0)) {
+  if (in_wave((fa > 0.0 && fb > 0.0) || (fa < 0.0 && fb < 0.0))) {
     *pb = b;
     return 502;
   }
@@ -91,22 +138,23 @@ __device__ __forceinline__ int jcg_zbrent(int n, const double* tri1, const doubl
     if (reset) {
       c = a; fc = fa; d = b - c; e = d;
     }
-    if (!(fabs(fc) >= fabs(fb))) {
+    if (in_wave(!(fabs(fc) >= fabs(fb)))) {
       a = b; b = c; c = a; fa = fb; fb = fc; fc = fa;
     }
     tol = t * fmax(fabs(b), 0.1);
     rm = (c - b) * 0.5;
-    if (fabs(fb) <= eps || fabs(c - b) <= tol) { *pb = b; return 0; }
+    if (in_wave(fabs(fb) <= eps || fabs(c - b) <= tol)) { *pb = b; return 0; }
     if (ic >= maxfn) { *pb = b; return 501; }
-    bool bisect = (fabs(e) < tol) || (fabs(fa) <= fabs(fb));
+    bool bisect = in_wave((fabs(e) < tol) || (fabs(fa) <= fabs(fb)));
     if (!bisect) {
       ss = fb / fa;
-      if (a == c) {
+      const double q3 = fa / fc, r3 = fb / fc;
+      if (in_wave(a == c)) {
         p = (c - b) * ss;
         qq = 1.0 - ss;
       } else {
-        qq = fa / fc;
-        r = fb / fc;
+        qq = q3;
+        r = r3;
         rone = r - 1.0;
         p = ss * ((c - b) * qq * (qq - r) - (b - a) * rone);
         qq = (qq - 1.0) * rone * (ss - 1.0);
@@ -115,10 +163,11 @@ __device__ __forceinline__ int jcg_zbrent(int n, const double* tri1, const doubl
       if (p < 0.0) p = -p;
       ss = e;
       e = d;
-      if (p + p >= 3.0 * rm * qq || p + p >= fabs(ss * qq)) {
+      const double step = p / qq;
+      if (in_wave(p + p >= 3.0 * rm * qq || p + p >= fabs(ss * qq))) {
         bisect = true;
       } else {
-        d = p / qq;
+        d = step;
       }
     }
     if (bisect) { e = rm; d = e; }
@@ -127,17 +176,16 @@ __device__ __forceinline__ int jcg_zbrent(int n, const double* tri1, const doubl
     temp = d;
     if (fabs(temp) <= 0.5 * tol) temp = copysign(0.5 * tol, rm);
     b = b + temp;
-    fb = jcg_determ(n, tri1, tri2, b);
+    fb = determ(b);
     ic = ic + 1;
-    if (fb == 0.0 || fc == 0.0) { reset = false; continue; }
-    if ((fb > 0.0 && fc < 0.0) || (fb < 0.0 && fc > 0.0)) { reset = false; continue; }
-    reset = true;
+    reset = !in_wave(fb == 0.0 || fc == 0.0 || (fb > 0.0 && fc < 0.0) || (fb < 0.0 && fc > 0.0));
   }
 }
 
 // chgcon(ibmth=1) (src/itpackv.F:893-1027); tri1/tri2 are the two columns.
 // Called by one whole wave with its own copy of the state in L (the lanes
 // hold the same values); tri1, tri2 are in LDS and read by that wave only.
+template <bool REG>
 __device__ __forceinline__ void jcg_chgcon(ItLocal& L, double* tri1, double* tri2) {
   const int ip = L.in;
   double start = L.cme, end1;
@@ -157,7 +205,7 @@ __device__ __forceinline__ void jcg_chgcon(ItLocal& L, double* tri1, double* tri
     tri1[ip - 1] = 1.0 - 1.0 / L.gamma;
     tri2[ip - 1] = (1.0 - L.rho) / (L.rho * L.rhoold * L.gamma * L.gamold);
     double b;
-    int ier = jcg_zbrent(ip, tri1, tri2, L.tz, L.maxfn, start, &b);
+    int ier = jcg_zbrent<REG>(ip, tri1, tri2, L.tz, L.maxfn, start, &b);
     if (ier != 0) {
       L.adapt = 0;
       return;
@@ -169,10 +217,11 @@ __device__ __forceinline__ void jcg_chgcon(ItLocal& L, double* tri1, double* tri
 
 // The eigenvalue estimate of iteration `in` (one whole wave): chgcon on the
 // wave's own copy of the state, its results back to L by lane 0.
+template <bool REG>
 __device__ __forceinline__ void jcg_eig_wave(ItLocal& L, double* tri1, double* tri2, int in) {
   ItLocal m = L;
   m.in = in;
-  if (m.adapt) jcg_chgcon(m, tri1, tri2);
+  if (m.adapt) jcg_chgcon<REG>(m, tri1, tri2);
   if ((threadIdx.x & 63) == 0) {
     L.in = in;
     L.adapt = m.adapt;
@@ -209,8 +258,7 @@ __device__ __forceinline__ void jcg_pstop(ItLocal& L, double unrm, double dnrm) 
 }
 
 // parcon(ibmth=1) (src/itpackv.F:1774-1851)
-__device__ __forceinline__ void jcg_parcon(ItLocal& L, double dtnrm) {
-  const int ip = L.in;
+__device__ __forceinline__ void jcg_parcon(ItLocal& L, double dtnrm, int ip) {
   const double rhoold = L.rho;
   L.gamold = L.gamma;
   L.gamma = 1.0 / (1.0 - dtnrm / L.delnnm);

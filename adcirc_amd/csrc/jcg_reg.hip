@@ -17,16 +17,28 @@
 //   of their own; every block polls all of them, a value being its own arrival
 //   flag (a slot holds JCG_EMPTY until it is written).  Barrier and reduction
 //   are one trip instead of three (two counter levels, generation word,
-//   partials).  A slot is written in iterations in, in+3, ..: its owner marks
-//   it empty in iteration in+2, when every block has read it (all have
-//   published in+1), and before it publishes in+2, so nobody can wait on the
-//   slot of in+3 before it is empty.
+//   partials).  A slot is written in iterations in, in+4, ..; its owner marks
+//   it empty in iteration in+3.  By then every row block has read it (all have
+//   published in+2, hence passed the wait of in+1), and so has the eigenvalue
+//   block, whose estimate of in+1 (or in+2) was needed to pass the wait of in+2; and nobody
+//   waits on the slot of in+4 before all have published in+3.
 // - Neighbours.  N d is published before the partials, so a block that has
 //   seen all partials can read its neighbours' N d and form their new d by
 //   itself (the owner's operations on the owner's values): the update needs no
 //   wait of its own.  Two buffers suffice: in+2 is written after all have
 //   published in+1, hence read in.
-// - The eigenvalue estimate (chgcon) runs in a block of its own, as before.
+// - The eigenvalue estimate (chgcon) runs in a block of its own: a serial chain, a
+//   root search of some nine evaluations, 3.6 to 7 us with the tridiagonal in LDS.
+//   With one chunk per block that is longer than a row block's own 4.7 us, and
+//   only the stopping test takes the result: such blocks test iteration `in` while
+//   they wait for the partials of in+1 (LATE).  By then u has moved on by one
+//   update, and the iterate before is still held.  With two chunks per block
+//   (14 us an iteration) the half iteration done past the halt costs more than
+//   the wait (20 steps at 999,151 rows: 15.58 ms late, 15.10 at once).  The
+//   tridiagonal is kept in registers during a search.
+//   The estimates have four slots: that of in is read in in or in+1, and its slot
+//   is marked empty in in+3, when all have published in+2, hence passed the wait
+//   of in+1.
 //
 // The sums' trees, the rows' operations and the scalar recurrences are those
 // of k_jcg; results are the same bits.
@@ -50,7 +62,7 @@ namespace adcgpu {
 // that lasts admit_ticks while some block has not started gives the launch up: the
 // abort bit is set (by an exchange on the count, so never once all have
 // started), every block leaves, and nothing but scratch has been written: no block
-// gets past the first iteration's partials before all have started.  k_jcg_mem,
+// gets past the second iteration's waits before all have started.  k_jcg_mem,
 // enqueued behind, then solves the system with two blocks.
 struct BoundedWait {
   const JcgArgs& a;
@@ -101,13 +113,12 @@ __device__ __forceinline__ void publish_vec(double* v, int i, double x) {
 // All of this wave's stores have reached memory (they are written through).
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// The cross-chunk sums of slot `part` into sum[0..2] (thread 0 adds the waves):
-// thread t < 256 waits for chunks t and t + 256 and adds them in that order,
-// then the butterfly.  Thread 256 waits for the eigenvalue block's pair when
-// `eig`.  t: the thread's index.  A thread whose wait failed sets *failed.  lds: 12 doubles.
-__device__ __forceinline__ void poll_partials(int t, const double* part, int nch, bool eig,
-                                              double* lds, double* pair, int* failed,
-                                              BoundedWait& w) {
+// The cross-chunk sums of slot `part` into lds (sum4 of each four): thread
+// t < 256 waits for chunks t and t + 256 and adds them in that order, then the
+// butterfly.  t: the thread's index.  A thread whose wait failed sets *failed.
+// lds: 12 doubles.
+__device__ __forceinline__ void poll_partials(int t, const double* part, int nch, double* lds,
+                                              int* failed, BoundedWait& w) {
   if (t < RED_XTHREADS) {
     double r0 = 0.0, r1 = 0.0, r2 = 0.0;
     if (t < nch) {
@@ -147,37 +158,11 @@ __device__ __forceinline__ void poll_partials(int t, const double* part, int nch
       lds[4 + (t >> 6)] = r1;
       lds[8 + (t >> 6)] = r2;
     }
-  } else if (eig && t == RED_XTHREADS) {
-    const double* p = part + 4 * nch;
-    double c0, c1;
-    for (;;) {
-      c0 = ld_agent(p);
-      c1 = ld_agent(p + 1);
-      if (!(is_empty(c0) || is_empty(c1))) break;
-      if (!w.more()) {
-        *failed = 1;
-        break;
-      }
-    }
-    pair[0] = c0;
-    pair[1] = c1;
   }
 }
 __device__ __forceinline__ double sum4(const double* v) { return (v[0] + v[1]) + (v[2] + v[3]); }
 
-// After a poll: pstop and parcon by thread 0, from the reduced partials and
-// the eigenvalue block's pair.
-__device__ __forceinline__ void reg_scalars(ItLocal& L, const double* lds, const double* pair,
-                                            int in, bool need_u) {
-  if (threadIdx.x == 0) {
-    L.in = in;
-    L.cme = pair[0];
-    L.cmold = pair[1];
-    L.delnnm = sum4(lds);
-    jcg_pstop(L, need_u ? sum4(lds + 8) : 1.0, L.delnnm);
-    if (!L.halt) jcg_parcon(L, sum4(lds + 4));
-  }
-}
+// Whether iteration `in` forms u.u, by the state after the test of in-1.
 __device__ __forceinline__ bool reg_need_u(const ItLocal& L, int in) {
   return !(L.q1 || (in > 5 && (in % 5) != 0));
 }
@@ -185,7 +170,9 @@ __device__ __forceinline__ bool reg_need_u(const ItLocal& L, int in) {
 // The LDS that the eigenvalue block and the row blocks share the use of.
 struct RegShared {
   ItLocal L;
-  double lds[12], pair[2];
+  double lds[12];
+  double dn, uu;          // d.d and u.u of the last iteration, not tested yet
+  double gamold, rhoold;  // as they were before its parcon
   int failed, ovn;
 };
 
@@ -197,23 +184,50 @@ __device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh, int
   const int t = threadIdx.x;
   const int nch = (a.n + RED_CHUNK - 1) / RED_CHUNK;
   BoundedWait wait(a, nblocks);
-  auto slot = [&](int k) { return a.part + (size_t)k * 4 * (nch + 1) + 4 * nch; };
+  auto slot = [&](int k) { return a.part + (size_t)k * 4 * (nch + 1); };
   for (int in = 0; in <= a.itmax; ++in) {
     const bool need_u = reg_need_u(sh.L, in);
     if (t < 64) {
-      if (t < 2) put_bits(slot((in + 1) % 3) + t, JCG_EMPTY);
-      jcg_eig_wave(sh.L, tri1, tri2, in);
+      if (t < 2) put_bits(slot((in + 1) & 3) + 4 * nch + t, JCG_EMPTY);
+      jcg_eig_wave<true>(sh.L, tri1, tri2, in);
       stores_done();
-      if (t < 2) publish(slot(in % 3) + t, t == 0 ? sh.L.cme : sh.L.cmold);
+      if (t < 2) publish(slot(in & 3) + 4 * nch + t, t == 0 ? sh.L.cme : sh.L.cmold);
     }
     __syncthreads();
-    poll_partials(t, slot(in % 3) - 4 * nch, nch, true, sh.lds, sh.pair, &sh.failed, wait);
+    poll_partials(t, slot(in & 3), nch, sh.lds, &sh.failed, wait);
     __syncthreads();
     if (sh.failed) return;
-    reg_scalars(sh.L, sh.lds, sh.pair, in, need_u);
+    if (t == 0) {
+      sh.L.delnnm = sum4(sh.lds);
+      jcg_pstop(sh.L, need_u ? sum4(sh.lds + 8) : 1.0, sh.L.delnnm);
+      if (!sh.L.halt) jcg_parcon(sh.L, sum4(sh.lds + 4), in);
+    }
     __syncthreads();
     if (sh.L.halt) break;
   }
+}
+
+// An estimate into the block's state (one thread of a row block).
+__device__ __forceinline__ bool reg_pair(RegShared& sh, const double* pair, BoundedWait& w) {
+  double c0, c1;
+  for (;;) {
+    c0 = ld_agent(pair);
+    c1 = ld_agent(pair + 1);
+    if (!(is_empty(c0) || is_empty(c1))) break;
+    if (!w.more()) {
+      sh.failed = 1;
+      return false;
+    }
+  }
+  sh.L.cme = c0;
+  sh.L.cmold = c1;
+  return true;
+}
+// The stopping test of the iteration before (LATE): touches what parcon does not.
+__device__ __forceinline__ void reg_test(RegShared& sh, const double* pair, int in, BoundedWait& w) {
+  if (!reg_pair(sh, pair, w)) return;
+  sh.L.in = in;
+  jcg_pstop(sh.L, reg_need_u(sh.L, in) ? sh.uu : 1.0, sh.dn);
 }
 
 // `bid` and `nblocks`: this block's index among the blocks that solve this
@@ -224,6 +238,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
   constexpr int W = CPB == 1 ? JCG_REG_W1 : JCG_REG_W2;     // entries per row in registers
   constexpr int TILE = CPB * RED_CHUNK;
   constexpr int K = CPB == 1 ? 6 : 10;  // neighbouring rows per thread read ahead
+  constexpr bool LATE = CPB == 1;       // the stopping test one iteration late
   __shared__ RegShared sh;
   __shared__ double wsum[CPB][24];
   extern __shared__ double dsh[];
@@ -413,7 +428,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
   const double* dv = a.ndv;
   int flip = 0;  // N d of even iterations goes to a.ndv: a.d holds the start
   if (DUAL) {
-    poll_partials(t, slot(3), nch, false, sh.lds, sh.pair, &sh.failed, wait);
+    poll_partials(t, slot(3), nch, sh.lds, &sh.failed, wait);
     __syncthreads();
     if (sh.failed) return;
     // the start with the smaller initial pseudo-residual
@@ -462,10 +477,13 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
   // ---- iterations
   for (int in = 0; in <= a.itmax; ++in) {
     opaque();
-    const bool need_u = reg_need_u(sh.L, in);
+    // u.u is formed where the test will take it (LATE: q1 is the last call's at
+    // first, cleared by the first test, then at most one test old, and only ever
+    // set)
+    const bool need_u = (LATE && in == 1) || reg_need_u(sh.L, in);
     double* const pv = ((in ^ flip) & 1) ? a.ndv : a.d;
-    if (in >= 1 && tl < 3 * CPB && c0 + tl / 3 < nch)
-      put_bits(slot((in + 1) % 3) + 4 * (c0 + tl / 3) + tl % 3, JCG_EMPTY);
+    if (in >= 2 && tl < 3 * CPB && c0 + tl / 3 < nch)
+      put_bits(slot((in + 1) & 3) + 4 * (c0 + tl / 3) + tl % 3, JCG_EMPTY);
     // N d, published for the neighbours; the rows' partials
 #pragma unroll
     for (int q = 0; q < R; ++q) nd[q] = 0.0;
@@ -496,11 +514,16 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
     __syncthreads();
     if (tl < 3 * CPB) {
       const int g = tl / 3, k = tl % 3, c = c0 + g;
-      if (c < nch) publish(slot(in % 3) + 4 * c + k, chunk_value(wsum[g] + 8 * k));
+      if (c < nch) publish(slot(in & 3) + 4 * c + k, chunk_value(wsum[g] + 8 * k));
     }
-    poll_partials(tl, slot(in % 3), nch, true, sh.lds, sh.pair, &sh.failed, wait);
+    if (t == RED_XTHREADS) {
+      if (!LATE) reg_pair(sh, slot(in & 3) + 4 * nch, wait);
+      else if (in > 0) reg_test(sh, slot((in - 1) & 3) + 4 * nch, in - 1, wait);
+    }
+    poll_partials(tl, slot(in & 3), nch, sh.lds, &sh.failed, wait);
     __syncthreads();
     if (sh.failed) return;
+    if (LATE && sh.L.halt) break;
     // the neighbours' N d on its way while thread 0 forms the scalars
     double x[K];
 #pragma unroll
@@ -508,9 +531,21 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
       const int k = tl + m * RED_THREADS;
       if (k < nh) x[m] = ld_agent(&at(pv, (unsigned)(lo + (k < nlo ? k : k + TILE))));
     }
-    reg_scalars(sh.L, sh.lds, sh.pair, in, need_u);
+    if (t == 0) {
+      sh.L.delnnm = sum4(sh.lds);
+      if (LATE) {
+        sh.gamold = sh.L.gamold;
+        sh.rhoold = sh.L.rhoold;
+        sh.dn = sh.L.delnnm;
+        sh.uu = sum4(sh.lds + 8);
+      } else {
+        sh.L.in = in;
+        jcg_pstop(sh.L, need_u ? sum4(sh.lds + 8) : 1.0, sh.L.delnnm);
+      }
+      if (LATE || !sh.L.halt) jcg_parcon(sh.L, sum4(sh.lds + 4), in);
+    }
     __syncthreads();
-    if (sh.L.halt) break;
+    if (!LATE && sh.L.halt) break;
     const double k1 = sh.L.c1, k2 = sh.L.c2, k3 = sh.L.c3, k4 = sh.L.c4;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
@@ -550,9 +585,19 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
     }
     __syncthreads();
   }
-  // the result is the iterate of the last iteration index: u at the halt,
-  // or the one before the final update when ITMAX ran out
+  // ITMAX iterations done: the test of the last one
+  if (LATE && !sh.L.halt) {
+    if (t == RED_XTHREADS) reg_test(sh, slot(a.itmax & 3) + 4 * nch, a.itmax, wait);
+    __syncthreads();
+    if (sh.failed) return;
+  }
+  // the result is the iterate of the last iteration index: the one before the
+  // last update, unless the test halted before that update
   const bool halted = sh.L.halt != 0;
+  if (LATE && t == 0 && halted) {
+    sh.L.gamold = sh.gamold;
+    sh.L.rhoold = sh.rhoold;
+  }
 
   opaque();
   int o = ovb;
@@ -568,7 +613,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
     const int i = ROW(q);
     if (i < np) {
       const double wi = at(a.w, (unsigned)i);
-      const double u = (halted ? uc[q] : up[q]) * wi;
+      const double u = (!LATE && halted ? uc[q] : up[q]) * wi;
       const double ri = 1.0 / wi;
       at(a.coef, (unsigned)i) = ri * ri;
       at(a.rhs, (unsigned)i) = at(a.rhs, (unsigned)i) * ri;
