@@ -132,6 +132,7 @@ struct adcgpu_ctx {
   double* qn_table = nullptr;
   int qn_table_steps = 0, qn_table_cap = 0;
   int64_t run_iters = 0, run_rebuilds = 0, run_itmax = 0, run_errstep = 0, run_mlused = 0;
+  int ep_steps = 2;          // steps whose matrix the host may have asked to rebuild
   bool coef_scaled = false;  // off-diagonals of COEF left scaled by a deferred solve
   // the patches of the GWCE and momentum passes, and each patch element's
   // NCEle as the next GWCE pass sees it (written by the momentum pass;
@@ -1023,6 +1024,7 @@ int adcgpu_set_field(adcgpu_ctx* c, int f, const void* host, int64_t count) {
   if (!c || !host) return fail(ADCGPU_E_ARG, "null argument");
   if (count != field_len(c, f)) return fail(ADCGPU_E_ARG, "field length");
   HIPCHK(hipSetDevice(c->device));
+  c->ep_steps = 2;
   if (double** p = field_ptr(c, f)) {
     // COEF(NP,MNEI) column-major is the device layout too; a COEF from the
     // host replaces any scaled off-diagonals a deferred solve left
@@ -1070,6 +1072,7 @@ int adcgpu_cold_start(adcgpu_ctx* c, const double* eta2, const int32_t* nodecode
                       const int32_t* noff) {
   if (!c || !eta2 || !nodecode || !noff) return fail(ADCGPU_E_ARG, "null argument");
   HIPCHK(hipSetDevice(c->device));
+  c->ep_steps = 2;
   const size_t np = c->np, ne = c->ne;
   // everything else starts cold too, so that a context can be cold-started
   // again: velocities, fluxes, increments, friction, forcing, the running
@@ -1233,7 +1236,8 @@ static void ncele_ready(adcgpu_ctx* c) {
 // The GWCE assembly up to the solve: matrix, right-hand side, time-level
 // rotation, the learned start's inputs, and the node pass that scales the
 // rows for JCG (or, with ILump = 1, solves).
-static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceStep* g) {
+static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceStep* g,
+                         const HollandPrm* met = nullptr) {
   const int np = c->np;
   const bool lumped = c->prm.ilump != 0;
   const double* rw = c->coef_scaled ? (const double*)c->jw : nullptr;
@@ -1246,8 +1250,13 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceS
   hipLaunchKernelGGL(gwce, pg, pb, lds, c->stream, c->mesh(), c->state(), c->patch, q, fric_prm(c),
                      (const int*)c->flags, rw);
   c->coef_scaled = false;
-  hipLaunchKernelGGL(k_lhs_ep, dim3(c->nch), dim3(RED_THREADS), 0, c->stream, c->mesh(),
-                     c->state(), c->flags, c->ep_part);
+  // without wet/dry only the host sets NCChange: once that rebuild and the step
+  // after it (which clears F_REBUILT) are past, EP stays
+  const bool ep = c->prm.nolifa == 2 || c->ep_steps > 0;
+  if (c->ep_steps > 0) --c->ep_steps;
+  if (ep)
+    hipLaunchKernelGGL(k_lhs_ep, dim3(c->nch), dim3(RED_THREADS), 0, c->stream, c->mesh(),
+                       c->state(), c->flags, c->ep_part);
   // ETA1 <- ETA2, H1 <- H2 (src/gwce.F:1622-1631) by rotation
   std::swap(c->eta1, c->eta2);
   std::swap(c->h1, c->h2);
@@ -1255,6 +1264,14 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceS
   // the state before the solve (eta^k now in ETA1)
   const bool learned = c->prm.warm_start == 2 && !lumped;
   const bool collect = c->ml_collect > 0 && c->ml_ready && !lumped;
+  // the forcing rides on the node pass, unless the learned start reads it first
+  HollandPrm hol;
+  std::memset(&hol, 0, sizeof(hol));
+  if (met) hol = *met;
+  const bool first = met && (learned || collect);
+  if (first)
+    hipLaunchKernelGGL(k_holland, dim3(nblk(np, 256)), dim3(256), 0, c->stream, np, c->x, c->y, hol,
+                       c->wsx2, c->wsy2, c->pr2);
   const int slot0 = collect ? (int)(c->smp_total % c->smp.cap) : 0;
   if (learned || collect) {
     const MlIn in = ml_in(c, c->eta1);
@@ -1268,7 +1285,7 @@ static int gwce_assemble(adcgpu_ctx* c, const double* d_eta_bc, bool fric, GwceS
   static_assert(RED_XTHREADS == 256, "the node pass forms EP with its 256 threads");
   hipLaunchKernelGGL(lumped ? k_rhs_node<true> : k_rhs_node<false>, dim3(nblk(np, 256)), dim3(256),
                      0, c->stream, c->mesh(), c->state(), d_eta_bc, c->nch,
-                     (const double*)c->ep_part, c->scal, pre);
+                     (const double*)c->ep_part, c->scal, pre, hol, met && !first ? 1 : 0);
   g->solve = !lumped;
   g->learned = learned;
   g->collect = collect;
@@ -1332,11 +1349,12 @@ int adcgpu_solve_gwce(adcgpu_ctx* c, int it, const double* eta_bc) {
 
 // Wet/dry; without `alpha_pass` the ALPHAL pass is left to the momentum
 // element pass (the resident run).
-static int wetdry_device(adcgpu_ctx* c, bool alpha_pass) {
+static int wetdry_device(adcgpu_ctx* c, bool alpha_pass, bool h2_pass = true) {
   const int np = c->np, ne = c->ne;
   // the flags change here; the momentum element pass records NCEle again
   c->ncele_fresh = false;
   if (c->prm.nolifa != 2) {
+    if (!h2_pass) return 0;  // the momentum pass forms H2
     hipLaunchKernelGGL(k_h2, dim3(nblk(np, 256)), dim3(256), 0, c->stream, np, c->dp, c->eta2,
                        c->ifnlfa, c->h2);
     return check_launch("h2");
@@ -1362,8 +1380,8 @@ int adcgpu_wetdry(adcgpu_ctx* c, int it) {
 }
 
 // Momentum; with `alpha` the pass forms ALPHAL first.
-static int momentum_device(adcgpu_ctx* c, bool alpha) {
-  MomPrm q{c->ifnlct, c->prm.nws, c->cur_it, c->errorelev, c->flags};
+static int momentum_device(adcgpu_ctx* c, bool alpha, bool h2 = false) {
+  const MomPrm q{c->ifnlct, c->prm.nws, c->cur_it, c->errorelev, c->flags, h2 ? 1 : 0, c->ifnlfa};
   auto mom = alpha ? (c->mixed ? k_mom<true, float> : k_mom<true, double>)
                    : (c->mixed ? k_mom<false, float> : k_mom<false, double>);
   hipLaunchKernelGGL(mom, dim3(c->patch.n), dim3(PATCH_THREADS),
@@ -1385,8 +1403,8 @@ int adcgpu_timestep(adcgpu_ctx* c, int it, const double* eta_bc, const double* w
   int rc = adcgpu_begin_step(c, it);
   if (!rc && c->prm.nws != 0) rc = adcgpu_set_forcing(c, wsx2, wsy2, pr2);
   if (!rc) rc = solve_gwce(c, eta_bc, true);
-  if (!rc) rc = wetdry_device(c, !wd);
-  if (!rc) rc = momentum_device(c, wd);
+  if (!rc) rc = wetdry_device(c, !wd, false);
+  if (!rc) rc = momentum_device(c, wd, !wd);
   return rc;
 }
 
@@ -1440,22 +1458,19 @@ static int run_prepare(adcgpu_ctx* c, int nsteps, const double* eta_bc_table,
   return check_launch("run set-up");
 }
 
-// A resident step up to the GWCE solve: begin, this step's Holland forcing, the
-// assembly (with friction).
+// A resident step up to the GWCE solve: begin, the assembly (with friction and
+// this step's Holland forcing).
 static int run_step_assemble(adcgpu_ctx* c, int it, int s, const double* holland, GwceStep* g) {
   const bool rows = c->nfluxf && c->qn_table_steps > s;
   int rc = begin_step(c, it, rows ? c->qn_table + (size_t)s * c->nvel : nullptr);
-  if (!rc && holland) {
-    HollandPrm hp;
+  HollandPrm hp;
+  if (holland) {
     for (int k = 0; k < 13; ++k) hp.v[k] = holland[k];
     hp.t = it * c->prm.dtdp;
-    hipLaunchKernelGGL(k_holland, dim3(nblk(c->np, 256)), dim3(256), 0, c->stream, c->np, c->x,
-                       c->y, hp, c->wsx2, c->wsy2, c->pr2);
-    rc = check_launch("forcing");
   }
   if (!rc)
     rc = gwce_assemble(c, c->neta > 0 ? c->eta_bc_table + (size_t)s * c->neta : c->eta_bc,
-                       true, g);
+                       true, g, holland ? &hp : nullptr);
   return rc;
 }
 
@@ -1464,8 +1479,8 @@ static int run_step_assemble(adcgpu_ctx* c, int it, int s, const double* holland
 static int run_step_finish(adcgpu_ctx* c, const GwceStep& g) {
   int rc = gwce_finish(c, g, true);
   const bool wd = c->prm.nolifa == 2;
-  if (!rc) rc = wetdry_device(c, !wd);
-  if (!rc) rc = momentum_device(c, wd);
+  if (!rc) rc = wetdry_device(c, !wd, false);
+  if (!rc) rc = momentum_device(c, wd, !wd);
   return rc;
 }
 
@@ -1657,7 +1672,7 @@ static int batch_member(adcgpu_ctx* c, int it, const double* holland, MemberArgs
   a->rq = rhs_prm(c, true);
   a->wq = wd_prm(c);
   a->wd = c->wd;
-  a->mq = MomPrm{c->ifnlct, c->prm.nws, 0, c->errorelev, c->flags};
+  a->mq = MomPrm{c->ifnlct, c->prm.nws, 0, c->errorelev, c->flags, 0, c->ifnlfa};
   a->pre = jcg_pre(c);
   if (holland)
     for (int k = 0; k < 13; ++k) a->hol.v[k] = holland[k];
@@ -1740,11 +1755,10 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
       if (s < 3)
         HIPCHK(hipMemcpyAsync(b->margs + slot, b->hmargs + slot, nt * sizeof(MemberArgs),
                               hipMemcpyHostToDevice, b->stream));
-      if (met) hipLaunchKernelGGL(k_holland_batch, ng, nb, 0, b->stream, ma, it0 + s);
       hipLaunchKernelGGL(mixed ? k_gwce_batch<float> : k_gwce_batch<double>, pg, pb,
                          patch_lds_bytes(PATCH_GWCE_FIELDS, PATCH_GWCE_TERMS, wmax), b->stream, ma);
       hipLaunchKernelGGL(k_lhs_ep_batch, dim3(nch_max, nt), dim3(RED_THREADS), 0, b->stream, ma);
-      hipLaunchKernelGGL(k_rhs_node_batch, ng, nb, 0, b->stream, ma, s);
+      hipLaunchKernelGGL(k_rhs_node_batch, ng, nb, 0, b->stream, ma, s, it0 + s, met ? 1 : 0);
       rc = check_launch("batch assembly");
     }
     // the solves: this step's arguments (they alternate with the time-level
@@ -2237,6 +2251,7 @@ int adcgpu_state_load(adcgpu_ctx* c, const void* buf, int64_t bytes) {
     return fail(ADCGPU_E_ARG, "snapshot of another mesh");
   o += 16;
   HIPCHK(hipSetDevice(c->device));
+  c->ep_steps = 2;
   for (const StatePart& p : state_parts(c)) {
     HIPCHK(hipMemcpyAsync(p.dev, o, p.bytes, hipMemcpyHostToDevice, c->stream));
     o += p.bytes;

@@ -215,6 +215,8 @@ struct MomPrm {
   int it;            // this step, recorded where ETAMAX rises
   double errorelev;  // ErrorElev: |ETA2| above it at a wet node stops the run
   int* flags;        // run-time error flags (ERR_ELEV, ERR_NONFINITE, F_ERRSTEP)
+  int form_h2;       // without wet/dry: H2 = DP + IFNLFA*ETA2 formed by the pass
+  double ifnlfa;
 };
 
 // Hybrid bottom friction (NOLIBF = 2): IFHYBF and fort.15's HBREAK, FTHETA,
@@ -299,7 +301,7 @@ struct JcgArgs {
   double* saved;      // [12] ITPACK SAVE state q1, gamold, rhoold, cmold, cme,
                       // stptst; [6..9] = cme, cmold of the running iteration, by parity
   int prescaled;      // rows already scaled (w, u, rhs) by k_rhs_node
-  int defer_unscal;   // leave the off-diagonals unscaled (k_lhs_rows scales and
+  int defer_unscal;   // leave the off-diagonals unscaled (k_gwce scales and
                       // unscales them if they are needed again)
   unsigned* barrier;  // [JCG_BAR_WORDS] grid barrier counters, then per-tile halo flags
   int hrows;          // >= 0: the pseudo-residual of the tile's rows and of hrows
@@ -397,8 +399,7 @@ struct MemberArgs {
 template <typename CT>
 __global__ void k_gwce_batch(const MemberArgs* a);
 __global__ void k_lhs_ep_batch(const MemberArgs* a);
-__global__ void k_rhs_node_batch(const MemberArgs* a, int step);
-__global__ void k_holland_batch(const MemberArgs* a, int it);
+__global__ void k_rhs_node_batch(const MemberArgs* a, int step, int it, int met);
 __global__ void k_wd_elem_batch(const MemberArgs* a);
 __global__ void k_wd_d2_batch(const MemberArgs* a);
 __global__ void k_wd_chain_batch(const MemberArgs* a);
@@ -406,7 +407,8 @@ template <typename CT>
 __global__ void k_mom_batch(const MemberArgs* a, int it);
 template <bool LUMPED>
 __global__ void k_rhs_node(DevMesh m, DevState s, const double* eta_bc, int nch,
-                           const double* ep_part, double* scal, JcgPre pre);
+                           const double* ep_part, double* scal, JcgPre pre, HollandPrm hol,
+                           int met);
 // DUAL: start from the better (smaller initial pseudo-residual) of a.u and a.u2;
 // STAGED: the products read the pseudo-residual from LDS (a.hrows >= 0).
 // Instantiated for all four combinations.

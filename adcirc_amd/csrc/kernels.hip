@@ -96,14 +96,6 @@ __global__ __launch_bounds__(256) void k_holland(int np, const double* __restric
   if (i >= np) return;
   holland_node(i, x, y, p, wsx, wsy, pr);
 }
-__global__ __launch_bounds__(256) void k_holland_batch(const MemberArgs* __restrict__ a, int it) {
-  const MemberArgs& x = a[blockIdx.y];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= x.m.np) return;
-  HollandPrm p = x.hol;
-  p.t = it * x.dt;
-  holland_node(i, x.m.x, x.m.y, p, x.s.wsx2, x.s.wsy2, x.s.pr2);
-}
 
 // --------------------------------------------------------------- GWCE
 // EP chunk partials: sum COEF(i,1)^2 (src/gwce.F:646-650) in the fixed blocked
@@ -228,8 +220,8 @@ template <bool LUMPED>
 __device__ __forceinline__ void rhs_node_block(const DevMesh& m, DevState s,
                                                const double* __restrict__ eta_bc, int nch,
                                                const double* __restrict__ ep_part,
-                                               double* __restrict__ scal, const JcgPre& pre, int bid,
-                                               int nb) {
+                                               double* __restrict__ scal, const JcgPre& pre,
+                                               const HollandPrm& hol, int met, int bid, int nb) {
   __shared__ double lds[4];
   __shared__ double ep_s;
   const int i = xcd_tile(bid, nb) * blockDim.x + threadIdx.x;
@@ -238,6 +230,9 @@ __device__ __forceinline__ void rhs_node_block(const DevMesh& m, DevState s,
   if (i == 0) pre.barrier[JCG_ADMIT_WORD] = pre.admit0;
   const bool rebuilt = pre.flags[F_REBUILT] != 0;
   const bool in = i < m.np;
+  // the step's forcing beside: arithmetic, where the rest of the pass waits for
+  // memory (a pass of its own took 23 us at 1M nodes, 5 at 20,000)
+  if (met && in) holland_node(i, m.x, m.y, hol, s.wsx2, s.wsy2, s.pr2);
   const int bi = in ? m.bnd_index[i] : -1;
   double dg = in ? s.coef[i] : 1.0;
   const bool take_ep = dg == 0.0 || bi >= 0;
@@ -337,18 +332,22 @@ template <bool LUMPED>
 __global__ __launch_bounds__(256) void k_rhs_node(DevMesh m, DevState s,
                                                   const double* __restrict__ eta_bc, int nch,
                                                   const double* __restrict__ ep_part,
-                                                  double* __restrict__ scal, JcgPre pre) {
-  rhs_node_block<LUMPED>(m, s, eta_bc, nch, ep_part, scal, pre, blockIdx.x, gridDim.x);
+                                                  double* __restrict__ scal, JcgPre pre,
+                                                  HollandPrm hol, int met) {
+  rhs_node_block<LUMPED>(m, s, eta_bc, nch, ep_part, scal, pre, hol, met, blockIdx.x, gridDim.x);
 }
-__global__ __launch_bounds__(256) void k_rhs_node_batch(const MemberArgs* __restrict__ a, int step) {
+__global__ __launch_bounds__(256) void k_rhs_node_batch(const MemberArgs* __restrict__ a, int step,
+                                                        int it, int met) {
   const MemberArgs& x = a[blockIdx.y];
   const int nb = (x.m.np + 255) / 256;
   if ((int)blockIdx.x >= nb) return;
+  HollandPrm hol = x.hol;
+  hol.t = it * x.dt;
   rhs_node_block<false>(x.m, x.s, x.eta_bc + (size_t)step * x.m.neta, x.nch, x.ep_part, x.scal, x.pre,
-                        blockIdx.x, nb);
+                        hol, met, blockIdx.x, nb);
 }
-template __global__ void k_rhs_node<false>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre);
-template __global__ void k_rhs_node<true>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre);
+template __global__ void k_rhs_node<false>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre, HollandPrm, int);
+template __global__ void k_rhs_node<true>(DevMesh, DevState, const double*, int, const double*, double*, JcgPre, HollandPrm, int);
 
 // ---------------------------------------------------------------- wet/dry
 // Values that another block of the launch reads: written through, and read past

@@ -1183,7 +1183,10 @@ __device__ __forceinline__ void mom_block(const DevMesh& m, const DevState& s, c
     nd.h1 = s.h1[i];
     nd.e2 = s.eta2[i];
     nd.nci = s.nodecode[i];
-    if (own) nd.load(m, s, q, i);
+    if (own) {
+      nd.load(m, s, q, i);
+      if (q.form_h2) s.h2[i] = nd.h2 = m.dp[i] + q.ifnlfa * nd.e2;
+    }
     W(MF_X, t) = m.x[i];
     W(MF_Y, t) = m.y[i];
     W(MF_EVM, t) = m.evm[i];
