@@ -43,8 +43,8 @@
 // The sums' trees, the rows' operations and the scalar recurrences are those
 // of k_jcg; results are the same bits.
 // Measured (MI355X, FP64, about 15 iterations; us per launch, k_jcg before):
-// 5,151 rows 118 (248), 20,646 rows 132 (257), 250,244 rows 146 (276),
-// 999,151 rows 253 (447).
+// 5,151 rows 109 to 114 (248), 20,646 rows 117 (257), 250,244 rows 131 (276),
+// 999,151 rows 251 (447); with every test at once 128, 133, 146, 251.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

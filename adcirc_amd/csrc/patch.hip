@@ -15,10 +15,10 @@
 // threads share a CU at different stages: half as many of 512 threads took 6%
 // longer.
 //
-// us at 999,151 nodes (wet/dry, storm), before and after: k_gwce 167, the passes
+// us at 999,151 nodes (wet/dry, storm), before and after: k_gwce 154, the passes
 // it replaces (element terms 102, matrix 76, friction 8, a launch each for the
-// matrix's other cases 11) 197; k_mom 115, before 106 + 54.  At 20,646 nodes 9.7
-// (23.5) and 7.5 (12.3), where a launch costs 5.  About 3 TB/s at 1M: the window's
+// matrix's other cases 11) 197; k_mom 104 to 110, before 106 + 54.  At 20,646 nodes
+// 9.1 (23.5) and 7.3 (12.3), where a launch costs 5.  About 3 TB/s at 1M: the window's
 // runs of some 16 nodes are shorter than what memory streams at (a copy: 5).
 //
 // Every sum keeps the reference's order: a node's contributions are listed in

@@ -1,10 +1,9 @@
 """Per-kernel summary of rocprofv3 kernel-trace databases of a resident run
 (profiling aid; reads the rocpd SQLite files rocprofv3 writes).
 
-Each time step of ``adcgpu_run`` starts with the friction pass
-(``k_friction``, or ``k_friction_holland`` with device forcing), makes exactly
-one ``k_jcg`` launch and ends with ``k_mom_node``, so a dispatch belongs to
-the step of the last friction pass before it.  A database whose window opens
+Each time step of ``adcgpu_run`` starts with the GWCE pass (``k_gwce``), makes
+exactly one solve and ends with ``k_mom``, so a dispatch belongs to the step of
+the last GWCE pass before it.  A database whose window opens
 with the run is numbered forward from its first step, one whose window closes
 with the run backward from the last.  Several databases recorded over
 overlapping windows of the same run (``rocprofv3 -P``) are stitched: a step
@@ -39,19 +38,19 @@ def _base(name: str) -> str:
 def _groups(path: str):
     rows = sqlite3.connect(path).execute(
         "select name, start, end from kernels order by start").fetchall()
-    # a step opens at the friction pass; dispatches before the first one
+    # a step opens at the GWCE pass; dispatches before the first one
     # belong to a step cut off by the window's start
     groups, cur = [], None
     for name, t0, t1 in rows:
         name = _name(name)
-        if _base(name) in ("k_friction", "k_friction_holland"):
+        if _base(name) == "k_gwce":
             cur = []
             groups.append(cur)
         if cur is not None:
             cur.append((name, t1 - t0))
-    # a last step cut off by the window's end (no k_jcg, or not all of the
-    # step's kernels) is dropped: the step's last kernel is k_mom_node
-    while groups and _base(groups[-1][-1][0]) != "k_mom_node":
+    # a last step cut off by the window's end (no solve, or not all of the
+    # step's kernels) is dropped: the step's last kernel is k_mom
+    while groups and _base(groups[-1][-1][0]) != "k_mom":
         groups.pop()
     return groups
 

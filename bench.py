@@ -148,13 +148,13 @@ def cpu_baseline(case, tables, eta2, nodecode, noff, steps: int, budget_s: float
 
 
 def jcg_traffic_fit():
-    """HBM bytes per JCG launch as a + b * iterations, fitted from the
-    per-dispatch FETCH_SIZE + WRITE_SIZE counters of a profiled run."""
-    path = os.path.join(REPO, "profiles", "k_jcg_coastal1m_traffic.json")
+    """HBM bytes per k_jcg_reg launch from the per-dispatch FETCH_SIZE +
+    WRITE_SIZE counters of a profiled run, and its iterations per launch."""
+    path = os.path.join(REPO, "profiles", "k_jcg_reg_coastal1m_traffic.json")
     if not os.path.exists(path):
         return None
     rec = json.load(open(path))
-    if "bytes_per_launch" not in rec or "bytes_per_iteration" not in rec:
+    if "bytes_per_launch" not in rec or "iterations" not in rec:
         return None
     return rec
 
@@ -420,21 +420,23 @@ def main() -> int:
             "noff_mismatch": int((fin["noff"] != base["noff"]).sum()),
         }
 
-    # roofline of the dominant kernel (k_jcg) from the plain leg
+    # roofline of the dominant kernel (k_jcg_reg) from the plain leg
     roof = None
     if "_jcg" in p:
         jcg_ms, launches, iters = p.pop("_jcg")
         Z = int(np.asarray(tables["nneigh"]).sum()) - npn
-        # algorithmic bytes: k*(12 Z + 48 NP) per iteration + (12 Z + 64 NP) per launch
-        jcg_bytes = iters * (12.0 * Z + 48.0 * npn) + launches * (12.0 * Z + 64.0 * npn)
+        # algorithmic bytes: the matrix and the vectors once per launch
+        # (12 Z + 64 NP: the iterations keep both on the chip), N d handed to the
+        # neighbouring blocks per iteration (16 NP)
+        jcg_bytes = iters * 16.0 * npn + launches * (12.0 * Z + 64.0 * npn)
         achieved = jcg_bytes / (jcg_ms * 1e-3) / 1e9 if jcg_ms > 0 else 0.0
         fit = jcg_traffic_fit()
         traffic = None
-        if fit and launches:
-            traffic = (fit["bytes_per_launch"] + fit["bytes_per_iteration"] * iters / launches) / 1e9
+        if fit and launches and abs(iters / launches - fit["iterations"]) < 0.5:
+            traffic = fit["bytes_per_launch"] / 1e9
         roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                "traffic_unit": "GB/launch", "kernel": "k_jcg",
+                "traffic_unit": "GB/launch", "kernel": "k_jcg_reg",
                 "algorithmic_gb_per_launch": jcg_bytes / max(launches, 1) / 1e9,
                 "kernel_ms_avg": jcg_ms / max(launches, 1),
                 "kernel_share_of_step": (jcg_ms / 1e3) / (p["ms_per_step"] * K / 1e3)}
