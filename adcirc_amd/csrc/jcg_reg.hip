@@ -43,8 +43,8 @@
 // The sums' trees, the rows' operations and the scalar recurrences are those
 // of k_jcg; results are the same bits.
 // Measured (MI355X, FP64, about 15 iterations; us per launch, k_jcg before):
-// 5,151 rows 109 to 114 (248), 20,646 rows 117 (257), 250,244 rows 131 (276),
-// 999,151 rows 251 (447); with every test at once 128, 133, 146, 251.
+// 5,151 rows 101 (248), 20,646 rows 111 (257), 250,244 rows 126 (276),
+// 999,151 rows 242 (447); with every test at once 128, 133, 146, 251.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -176,34 +176,49 @@ struct RegShared {
   int failed, ovn;
 };
 
-// The eigenvalue block: the adaptive estimate of each iteration beside the
-// row blocks' products, then the same scalars as theirs.
+// The eigenvalue block: the adaptive estimate of each iteration beside the row
+// blocks' products.  Its cycle sets the pace of most solves, so its first wave
+// does only what the next estimate hangs on: the state is in its registers, the
+// same in every lane, and the stopping test, which only tells the block when to
+// leave, is made by another wave beside the next estimate (14,300 cycles an
+// iteration with the test before it).
 template <bool DUAL>
 __device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh, int nblocks) {
   __shared__ double tri1[JCG_MAX_ITMAX], tri2[JCG_MAX_ITMAX];
+  __shared__ double cmes[2];
   const int t = threadIdx.x;
   const int nch = (a.n + RED_CHUNK - 1) / RED_CHUNK;
   BoundedWait wait(a, nblocks);
   auto slot = [&](int k) { return a.part + (size_t)k * 4 * (nch + 1); };
+  ItLocal m = sh.L;  // the first wave's: the estimate and the recurrence; the second's: the test
+  double dn = 0.0, uu = 0.0;
   for (int in = 0; in <= a.itmax; ++in) {
-    const bool need_u = reg_need_u(sh.L, in);
     if (t < 64) {
       if (t < 2) put_bits(slot((in + 1) & 3) + 4 * nch + t, JCG_EMPTY);
-      jcg_eig_wave<true>(sh.L, tri1, tri2, in);
+      m.in = in;
+      if (in_wave(m.adapt != 0)) jcg_chgcon<true>(m, tri1, tri2);
       stores_done();
-      if (t < 2) publish(slot(in & 3) + 4 * nch + t, t == 0 ? sh.L.cme : sh.L.cmold);
+      if (t < 2) publish(slot(in & 3) + 4 * nch + t, t == 0 ? m.cme : m.cmold);
+      if (t == 0) cmes[in & 1] = m.cme;
+    } else if (t == 64 && in > 0) {
+      m.in = in - 1;
+      m.cme = cmes[(in - 1) & 1];
+      jcg_pstop(m, reg_need_u(m, in - 1) ? uu : 1.0, dn);
+      sh.L.halt = m.halt;
     }
     __syncthreads();
+    // (row blocks that have stopped may publish no more partials)
+    if (sh.L.halt) break;
     poll_partials(t, slot(in & 3), nch, sh.lds, &sh.failed, wait);
     __syncthreads();
     if (sh.failed) return;
-    if (t == 0) {
-      sh.L.delnnm = sum4(sh.lds);
-      jcg_pstop(sh.L, need_u ? sum4(sh.lds + 8) : 1.0, sh.L.delnnm);
-      if (!sh.L.halt) jcg_parcon(sh.L, sum4(sh.lds + 4), in);
+    if (t < 64) {
+      m.delnnm = sum4(sh.lds);
+      jcg_parcon(m, sum4(sh.lds + 4), in);
+    } else if (t == 64) {
+      dn = sum4(sh.lds);
+      uu = sum4(sh.lds + 8);
     }
-    __syncthreads();
-    if (sh.L.halt) break;
   }
 }
 
