@@ -54,8 +54,10 @@
 
 namespace adcgpu {
 
-// A bounded wait: every 64th unsuccessful poll looks at the error flag and at
-// the clock; a wait that runs out sets the flag, so every block drains.
+// One bounded wait (an object per wait, so that the bound is each wait's own and
+// nothing of it is kept in registers between waits): every 64th unsuccessful poll
+// looks at the error flag and at the clock; a wait that runs out sets the flag, so
+// every block drains.
 //
 // An ordinary launch (JcgArgs::admit) may find part of the chip taken by blocks
 // that wait for it in turn.  Each block counts itself in when it starts; a wait
@@ -118,8 +120,9 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 // butterfly.  t: the thread's index.  A thread whose wait failed sets *failed.
 // lds: 12 doubles.
 __device__ __forceinline__ void poll_partials(int t, const double* part, int nch, double* lds,
-                                              int* failed, BoundedWait& w) {
+                                              int* failed, const JcgArgs& args, int nblocks) {
   if (t < RED_XTHREADS) {
+    BoundedWait w(args, nblocks);
     double r0 = 0.0, r1 = 0.0, r2 = 0.0;
     if (t < nch) {
       const double* p = part + 4 * t;
@@ -188,7 +191,6 @@ __device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh, int
   __shared__ double cmes[2];
   const int t = threadIdx.x;
   const int nch = (a.n + RED_CHUNK - 1) / RED_CHUNK;
-  BoundedWait wait(a, nblocks);
   auto slot = [&](int k) { return a.part + (size_t)k * 4 * (nch + 1); };
   ItLocal m = sh.L;  // the first wave's: the estimate and the recurrence; the second's: the test
   double dn = 0.0, uu = 0.0;
@@ -209,7 +211,7 @@ __device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh, int
     __syncthreads();
     // (row blocks that have stopped may publish no more partials)
     if (sh.L.halt) break;
-    poll_partials(t, slot(in & 3), nch, sh.lds, &sh.failed, wait);
+    poll_partials(t, slot(in & 3), nch, sh.lds, &sh.failed, a, nblocks);
     __syncthreads();
     if (sh.failed) return;
     if (t < 64) {
@@ -223,7 +225,9 @@ __device__ __forceinline__ void jcg_reg_eig(const JcgArgs& a, RegShared& sh, int
 }
 
 // An estimate into the block's state (one thread of a row block).
-__device__ __forceinline__ bool reg_pair(RegShared& sh, const double* pair, BoundedWait& w) {
+__device__ __forceinline__ bool reg_pair(RegShared& sh, const double* pair, const JcgArgs& a,
+                                         int nblocks) {
+  BoundedWait w(a, nblocks);
   double c0, c1;
   for (;;) {
     c0 = ld_agent(pair);
@@ -239,8 +243,9 @@ __device__ __forceinline__ bool reg_pair(RegShared& sh, const double* pair, Boun
   return true;
 }
 // The stopping test of the iteration before (LATE): touches what parcon does not.
-__device__ __forceinline__ void reg_test(RegShared& sh, const double* pair, int in, BoundedWait& w) {
-  if (!reg_pair(sh, pair, w)) return;
+__device__ __forceinline__ void reg_test(RegShared& sh, const double* pair, int in,
+                                         const JcgArgs& a, int nblocks) {
+  if (!reg_pair(sh, pair, a, nblocks)) return;
   sh.L.in = in;
   jcg_pstop(sh.L, reg_need_u(sh.L, in) ? sh.uu : 1.0, sh.dn);
 }
@@ -281,7 +286,6 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
     return;
   }
   const int lane = t & 63, wave = t >> 6;
-  BoundedWait wait(a, nblocks);
   const int tile = xcd_tile(bid, nrb);
   const int c0 = tile * CPB;  // first chunk
   const int t0 = tile * TILE, t1 = t0 + TILE < np ? t0 + TILE : np;
@@ -443,7 +447,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
   const double* dv = a.ndv;
   int flip = 0;  // N d of even iterations goes to a.ndv: a.d holds the start
   if (DUAL) {
-    poll_partials(t, slot(3), nch, sh.lds, &sh.failed, wait);
+    poll_partials(t, slot(3), nch, sh.lds, &sh.failed, a, nblocks);
     __syncthreads();
     if (sh.failed) return;
     // the start with the smaller initial pseudo-residual
@@ -469,6 +473,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
     const int ca = lo / RED_CHUNK, cb = (hi - 1) / RED_CHUNK;
     for (int c = ca + t; c <= cb; c += RED_THREADS) {
       const double* p = slot(3) + 4 * c;
+      BoundedWait wait(a, nblocks);
       while (is_empty(ld_agent(p)))
         if (!wait.more()) {
           sh.failed = 1;
@@ -532,10 +537,10 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
       if (c < nch) publish(slot(in & 3) + 4 * c + k, chunk_value(wsum[g] + 8 * k));
     }
     if (t == RED_XTHREADS) {
-      if (!LATE) reg_pair(sh, slot(in & 3) + 4 * nch, wait);
-      else if (in > 0) reg_test(sh, slot((in - 1) & 3) + 4 * nch, in - 1, wait);
+      if (!LATE) reg_pair(sh, slot(in & 3) + 4 * nch, a, nblocks);
+      else if (in > 0) reg_test(sh, slot((in - 1) & 3) + 4 * nch, in - 1, a, nblocks);
     }
-    poll_partials(tl, slot(in & 3), nch, sh.lds, &sh.failed, wait);
+    poll_partials(tl, slot(in & 3), nch, sh.lds, &sh.failed, a, nblocks);
     __syncthreads();
     if (sh.failed) return;
     if (LATE && sh.L.halt) break;
@@ -602,7 +607,7 @@ __device__ __forceinline__ void jcg_solve_reg(const JcgArgs& a, int bid, int nbl
   }
   // ITMAX iterations done: the test of the last one
   if (LATE && !sh.L.halt) {
-    if (t == RED_XTHREADS) reg_test(sh, slot(a.itmax & 3) + 4 * nch, a.itmax, wait);
+    if (t == RED_XTHREADS) reg_test(sh, slot(a.itmax & 3) + 4 * nch, a.itmax, a, nblocks);
     __syncthreads();
     if (sh.failed) return;
   }
