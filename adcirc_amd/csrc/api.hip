@@ -352,6 +352,13 @@ void solves_done(adcgpu_ctx* c) {
   c->solving = false;
 }
 
+// Every wait for a context's stream: its solves are done then.
+hipError_t stream_wait(adcgpu_ctx* c) {
+  const hipError_t e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) solves_done(c);
+  return e;
+}
+
 // Chunks per block of the register kernel for the context's own launches; 0:
 // another kernel.  One chunk per block while the blocks are all resident: half
 // the rows per thread and twice the CUs; two beyond that.
@@ -441,7 +448,7 @@ int patch_setup(adcgpu_ctx* c) {
                      dim3(256), 0, c->stream, c->mesh(), pp, pair, c->flags + F_NUMITR);
   int f[2] = {0, 0};
   HIPCHK(hipMemcpyAsync(f, c->flags + F_NUMITR, sizeof(f), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   if (f[0] == 0) pp.pair = pair;
   if (f[1] != 0) {
     if (int rc = dmalloc(&geo, 7 * (size_t)pp.nq)) return rc;
@@ -451,7 +458,7 @@ int patch_setup(adcgpu_ctx* c) {
     pp.geo = geo;
   }
   hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_NUMITR, 0, 2);
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   return check_launch("patch set-up");
 }
 
@@ -526,7 +533,7 @@ int ml_setup(adcgpu_ctx* c) {
   HIPCHK(hipMemcpy(c->ml_master, p.data(), p.size() * 4, hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_ml_pack, dim3(nblk(ML_W2 * 2, 256)), dim3(256), 0, c->stream,
                      (const float*)c->ml_master, c->mlw);
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   return check_launch("learned start set-up");
 }
 
@@ -1041,8 +1048,7 @@ int adcgpu_set_field(adcgpu_ctx* c, int f, const void* host, int64_t count) {
   if (f == ADCGPU_NODECODE || f == ADCGPU_NOFF) c->ncele_fresh = false;
   if (f == ADCGPU_ALPHAL)
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->flags + F_ALPHA, 1, 1);
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   return check_launch("set_field");
 }
 
@@ -1061,8 +1067,7 @@ int adcgpu_get_field(adcgpu_ctx* c, int f, void* host, int64_t count) {
   } else {
     return fail(ADCGPU_E_ARG, "unknown field");
   }
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   return 0;
 }
 
@@ -1094,7 +1099,7 @@ int adcgpu_cold_start(adcgpu_ctx* c, const double* eta2, const int32_t* nodecode
     HIPCHK(hipMemcpyAsync(c->etamax, low.data(), np * 8, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->umax, low.data(), np * 8, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->alphal, ones.data(), ne * 8, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(stream_wait(c));
   }
   c->coef_scaled = false;
   c->ncele_fresh = false;
@@ -1108,7 +1113,7 @@ int adcgpu_cold_start(adcgpu_ctx* c, const double* eta2, const int32_t* nodecode
   int f[F_COUNT] = {0};
   f[F_NCCHANGE] = 1;
   HIPCHK(hipMemcpyAsync(c->flags, f, sizeof(f), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   if (c->nfluxf)
     if (int rc = set_elevdisc(c)) return rc;
   return check_launch("cold start");
@@ -1412,8 +1417,7 @@ int adcgpu_last_numitr(adcgpu_ctx* c, int* numitr, int* ier) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
   int f[F_COUNT];
   HIPCHK(hipMemcpyAsync(f, c->flags, sizeof(f), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   if (numitr) *numitr = f[F_NUMITR];
   if (ier) *ier = f[F_IER];
   return flag_errors(f);
@@ -1421,8 +1425,7 @@ int adcgpu_last_numitr(adcgpu_ctx* c, int* numitr, int* ier) {
 
 int adcgpu_synchronize(adcgpu_ctx* c) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   return 0;
 }
 
@@ -1488,8 +1491,7 @@ static int run_step_finish(adcgpu_ctx* c, const GwceStep& g) {
 static int run_read_flags(adcgpu_ctx* c, bool* error) {
   int f[F_COUNT];
   HIPCHK(hipMemcpyAsync(f, c->flags, sizeof(f), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   c->run_iters = f[F_ITSUM];
   c->run_rebuilds = f[F_NREBUILD];
   c->run_itmax = f[F_NITMAX];
@@ -1557,6 +1559,31 @@ void batch_free(adcgpu_batch* b) {
   if (b->hmargs) (void)hipHostFree(b->hmargs);
   delete b;
 }
+
+// Every member's work goes to the batch's stream for a run, so that the shared
+// JCG launches are ordered after and before each member's passes; however the
+// run ends, the members get their own streams back, with nothing left in the
+// batch's.
+struct BatchStream {
+  adcgpu_batch* b;
+  std::vector<hipStream_t> own;
+  explicit BatchStream(adcgpu_batch* batch) : b(batch) { own.reserve(b->m.size()); }
+  // members in order
+  hipError_t take(adcgpu_ctx* c) {
+    const hipError_t e = stream_wait(c);
+    if (e != hipSuccess) return e;
+    own.push_back(c->stream);
+    c->stream = b->stream;
+    return hipSuccess;
+  }
+  ~BatchStream() {
+    (void)hipStreamSynchronize(b->stream);
+    for (size_t k = 0; k < own.size(); ++k) {
+      solves_done(b->m[k]);
+      b->m[k]->stream = own[k];
+    }
+  }
+};
 }  // namespace
 
 extern "C" {
@@ -1694,18 +1721,8 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
   const int n = (int)b->m.size();
   auto table = [&](int k) { return eta_bc_tables ? eta_bc_tables[k] : nullptr; };
   auto hol = [&](int k) { return holland ? holland[k] : nullptr; };
-  // every member's work goes to the batch's stream for the run, so that the
-  // shared JCG launches are ordered after and before each member's passes
-  std::vector<hipStream_t> own(n);
-  for (int k = 0; k < n; ++k) {
-    own[k] = b->m[k]->stream;
-    HIPCHK(hipStreamSynchronize(own[k]));
-    b->m[k]->stream = b->stream;
-  }
-  auto restore = [&]() {
-    (void)hipStreamSynchronize(b->stream);
-    for (int k = 0; k < n; ++k) b->m[k]->stream = own[k];
-  };
+  BatchStream loan(b);
+  for (adcgpu_ctx* c : b->m) HIPCHK(loan.take(c));
   int rc = 0;
   for (int k = 0; k < n && !rc; ++k) rc = run_prepare(b->m[k], nsteps, table(k), hol(k));
   std::vector<GwceStep> g(n);
@@ -1780,6 +1797,7 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
       }
       if (!b->hvalid[par] || std::memcmp(h, cur.data(), ns * sizeof(JcgArgs)) != 0) {
         HIPCHK(hipStreamSynchronize(b->stream));
+        b->hvalid[par] = false;  // until the device holds them too
         std::memcpy(h, cur.data(), ns * sizeof(JcgArgs));
         HIPCHK(hipMemcpyAsync(b->dargs + par * ns, h, ns * sizeof(JcgArgs),
                               hipMemcpyHostToDevice, b->stream));
@@ -1842,7 +1860,6 @@ int adcgpu_batch_run(adcgpu_batch* b, int it0, int nsteps, const double* const* 
     bool error = false;
     rc = run_read_flags(b->m[k], &error);
   }
-  restore();
   return rc;
 }
 
@@ -1860,7 +1877,7 @@ int adcgpu_last_solve(adcgpu_ctx* c, double* out4) {
   if (!c || !out4) return fail(ADCGPU_E_ARG, "null argument");
   double s[12];
   HIPCHK(hipMemcpyAsync(s, c->jsaved, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   JcgArgs a;
   jcg_tolerances(a, c->prm.itmax, c->prm.convcr);
   out4[0] = s[5];
@@ -1898,7 +1915,7 @@ static int set_elevdisc(adcgpu_ctx* c) {
   const int nvel = c->nvel;
   std::vector<double> eta((size_t)c->np), ed((size_t)nvel, 0.0);
   std::vector<int> lbc((size_t)nvel);
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   HIPCHK(hipMemcpy(eta.data(), c->eta2, (size_t)c->np * 8, hipMemcpyDeviceToHost));
   HIPCHK(hipMemcpy(lbc.data(), c->lbcodei, (size_t)nvel * sizeof(int), hipMemcpyDeviceToHost));
   for (int k = 0; k < nvel; ++k)
@@ -1921,7 +1938,7 @@ int adcgpu_set_hybrid_friction(adcgpu_ctx* c, double hbreak, double ftheta, doub
 int adcgpu_set_flux_boundary(adcgpu_ctx* c, const double* bndlen2o3) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
   HIPCHK(hipSetDevice(c->device));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   const int np = c->np, nvel = c->nvel;
   for (void** p : {(void**)&c->fb_ptr, (void**)&c->fb_ent, (void**)&c->nbv0, (void**)&c->bndlen})
     if (*p) {
@@ -1980,7 +1997,7 @@ int adcgpu_set_flux_table(adcgpu_ctx* c, int nsteps, const double* qn2_table) {
   if (!c || nsteps < 0 || (nsteps > 0 && !qn2_table)) return fail(ADCGPU_E_ARG, "invalid argument");
   if (!c->nfluxf) return fail(ADCGPU_E_ARG, "no flux boundaries set up (adcgpu_set_flux_boundary)");
   HIPCHK(hipSetDevice(c->device));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   if (c->qn_table_cap < nsteps) {
     if (c->qn_table) (void)hipFree(c->qn_table);
     c->qn_table = nullptr;
@@ -2003,7 +2020,7 @@ int adcgpu_set_tide_potential(adcgpu_ctx* c, int ntif, const double* tpk, const 
   if (ntif > 0 && (!tpk || !amigt || !etrf || !fft || !facet || !slam || !sfea))
     return fail(ADCGPU_E_ARG, "null argument");
   HIPCHK(hipSetDevice(c->device));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   if (ntif == 0) {
     c->ctip = false;
     return 0;
@@ -2065,7 +2082,7 @@ int adcgpu_ml_params(adcgpu_ctx* c, const float* in, float* out) {
   if (out)
     HIPCHK(hipMemcpyAsync(out, c->ml_master, (size_t)ML_NPARAM * 4, hipMemcpyDeviceToHost,
                           c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   return check_launch("ml params");
 }
 
@@ -2113,7 +2130,7 @@ int adcgpu_ml_train(adcgpu_ctx* c, int epochs, double lr, uint64_t seed, double*
     }
     float l = 0.0f;
     HIPCHK(hipMemcpyAsync(&l, lossacc, 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(stream_wait(c));
     last = (double)l / nb;
   }
   if (loss_out) *loss_out = last;
@@ -2143,7 +2160,7 @@ int adcgpu_ml_grad(adcgpu_ctx* c, int n, const float* x, const float* y, const f
   float l = 0.0f;
   HIPCHK(hipMemcpyAsync(grad, gdev, (size_t)ML_NPARAM * 4, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipMemcpyAsync(&l, lossacc, 4, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   if (loss) *loss = l;
   return 0;
 }
@@ -2160,7 +2177,7 @@ int adcgpu_ml_features(adcgpu_ctx* c, float* x_out, double* s_out) {
   std::vector<float> s(c->np);
   HIPCHK(hipMemcpyAsync(xb.data(), c->smp.x, xb.size() * 2, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipMemcpyAsync(s.data(), c->smp.s, (size_t)c->np * 4, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   for (size_t k = 0; k < xb.size(); ++k) x_out[k] = bf16_to_f32(xb[k]);
   if (s_out)
     for (int i = 0; i < c->np; ++i) s_out[i] = s[i];
@@ -2174,7 +2191,7 @@ int adcgpu_ml_correction(adcgpu_ctx* c, double* corr_out) {
   ml_infer(c, in);
   HIPCHK(hipMemcpyAsync(corr_out, c->ml_corr, (size_t)c->np * 8, hipMemcpyDeviceToHost,
                         c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   return check_launch("ml correction");
 }
 
@@ -2236,8 +2253,7 @@ int adcgpu_state_save(adcgpu_ctx* c, void* buf, int64_t bytes) {
     HIPCHK(hipMemcpyAsync(o, p.dev, p.bytes, hipMemcpyDeviceToHost, c->stream));
     o += p.bytes;
   }
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   return 0;
 }
 
@@ -2256,8 +2272,7 @@ int adcgpu_state_load(adcgpu_ctx* c, const void* buf, int64_t bytes) {
     HIPCHK(hipMemcpyAsync(p.dev, o, p.bytes, hipMemcpyHostToDevice, c->stream));
     o += p.bytes;
   }
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   c->cur_it = hdr[3];
   c->coef_scaled = false;
   c->ncele_fresh = false;
@@ -2284,7 +2299,7 @@ int adcgpu_jcg_shape(adcgpu_ctx* c, int* shape3) {
 
 int adcgpu_profile(adcgpu_ctx* c, int enable) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   c->ev_used = 0;
   c->profile = enable != 0;
   if (enable) return grow_events(c, std::max<size_t>(c->jcg_events.size(),
@@ -2294,7 +2309,7 @@ int adcgpu_profile(adcgpu_ctx* c, int enable) {
 
 int adcgpu_profile_read(adcgpu_ctx* c, double* jcg_ms, int64_t* launches) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   double tot = 0.0;
   for (size_t k = 0; k < c->ev_used; ++k) {
     float ms = 0.f;
@@ -2447,8 +2462,7 @@ int adcgpu_jcg(int n, int ndim, int maxnz, int32_t* jcoef, double* coef, double*
     int f[F_COUNT + 2];
   } out;
   HIPCHK(hipMemcpyAsync(&out, c->jsaved, sizeof(out), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  solves_done(c);
+  HIPCHK(stream_wait(c));
   const double* const saved = out.saved;
   const int* const f = out.f;
   // the device copies are left as the failed call left them; the caller's
@@ -2464,7 +2478,7 @@ int adcgpu_jcg(int n, int ndim, int maxnz, int32_t* jcoef, double* coef, double*
                  hipMemcpyDeviceToHost));
   HIPCHK(hipMemcpyAsync(rhs, c->gwce_lv, n * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipMemcpyAsync(u, c->etas, n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(stream_wait(c));
   const int in = f[F_NUMITR];
   const int ier = f[F_IER];
   iparm[7] = 4 * n + 4 * in;

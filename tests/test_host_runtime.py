@@ -1,0 +1,139 @@
+"""The library's host code over a HIP runtime without a device
+(hip_host_stub.cpp: kernels are not run, calls can be made to fail): what a
+failed call leaves behind, which launch a small solve takes, and contexts
+driven from several threads.  Each check runs in a process of its own, where
+the stub is loaded ahead of the library."""
+from __future__ import annotations
+
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def stub_path(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "libhip_host_stub.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-pthread",
+                    "-D__HIP_PLATFORM_AMD__=1", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_host_stub.cpp"), "-o", out], check=True)
+    return out
+
+
+def _child(stub_path, check, *args):
+    code = ("import sys; sys.path[:0] = [%r, %r]; import test_host_runtime as t; t.%s(%s)"
+            % (os.path.dirname(HERE), HERE, check, ", ".join(map(repr, (stub_path,) + args))))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
+
+
+class _Stub:
+    def __init__(self, path):
+        self.lib = C.CDLL(path, C.RTLD_GLOBAL)  # found before the HIP runtime's symbols
+        for f in ("ordinary", "cooperative", "dead_uses", "live_streams"):
+            getattr(self.lib, "stub_" + f).restype = C.c_long
+        for f in ("fail_copy", "fail_cooperative"):
+            getattr(self.lib, "stub_" + f).argtypes = [C.c_long]
+
+    def __getattr__(self, name):
+        return getattr(self.lib, "stub_" + name)
+
+
+def _models(n, nodes=2000, **over):
+    import dataclasses
+    from adcirc_amd import meshgen
+    from adcirc_amd.model import Model
+    from gpu_helpers import case_setup, golden_tables
+    case = meshgen.coastal(nodes)
+    run = dataclasses.replace(case.run, **over)
+    d = case_setup(case)
+    t = golden_tables(d)
+    got = []
+    for _ in range(n):
+        g = Model(t, run, emo=np.asarray(d["emo"]).reshape(t["neta"], -1),
+                  efa=np.asarray(d["efa"]).reshape(t["neta"], -1))
+        g.cold_start(d["eta2_0"], d["nodecode0"], d["noff0"])
+        got.append(g)
+    return got, run
+
+
+def _step(m, it):
+    w = np.zeros(m.np_)
+    m.timestep(it, (w, w, w))
+
+
+# ---- a run of a batch that fails part way
+def child_failed_batch(path, what):
+    from adcirc_amd.model import Batch
+    stub = _Stub(path)
+    models, run = _models(3)
+    streams = stub.live_streams()
+    failed = 0
+    for nth in range(1, 200):
+        b = Batch(models)
+        getattr(stub, "fail_" + what)(nth)
+        try:
+            b.run(1, 3, holland=[run.holland] * 3)
+            done = True
+        except RuntimeError as e:
+            assert "stub error" in str(e), e
+            done = False
+        getattr(stub, "fail_" + what)(0)
+        b.close()
+        assert stub.live_streams() == streams
+        # no member holds the batch's stream, and none counts as solving: a small
+        # solve takes the ordinary launch
+        for m in models:
+            coop = stub.cooperative()
+            _step(m, 5)
+            m.synchronize()
+            assert stub.dead_uses() == 0, (nth, stub.dead_uses())
+            assert stub.cooperative() == coop, nth
+        if done:
+            break
+        failed += 1
+    assert done and failed > 0, failed
+    for m in models:
+        m.close()
+    assert stub.live_streams() == 0 and stub.dead_uses() == 0
+
+
+@pytest.mark.parametrize("what", ["copy", "cooperative"])
+def test_failed_batch_gives_the_streams_back(stub_path, what):
+    """Each copy, or each cooperative launch, of a three-step run fails in turn."""
+    _child(stub_path, "child_failed_batch", what)
+
+
+# ---- the launch of a small solve
+def child_launch_choice(path):
+    stub = _Stub(path)
+    (a, b), _ = _models(2)
+
+    def cooperative(m, it):
+        before = stub.cooperative()
+        _step(m, it)
+        return stub.cooperative() - before
+
+    assert cooperative(a, 1) == 0      # alone
+    assert cooperative(a, 2) == 0
+    assert cooperative(b, 1) == 1      # a's solves have not been waited for
+    assert cooperative(a, 3) == 1
+    for wait in (a.synchronize, a.numitr, a.last_solve, lambda: a.get("eta2"), a.save_state,
+                 lambda: a.set("tk", a.get("tk"))):
+        b.synchronize()
+        _step(a, 4)
+        wait()
+        assert cooperative(b, 2) == 0, wait   # a has been waited for
+    a.close()
+    b.close()
+
+
+def test_launch_follows_what_is_solving(stub_path):
+    """A small solve takes the ordinary launch exactly while no other context has
+    solves that nobody has waited for; every call that waits counts."""
+    _child(stub_path, "child_launch_choice")
