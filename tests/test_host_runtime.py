@@ -137,3 +137,46 @@ def test_launch_follows_what_is_solving(stub_path):
     """A small solve takes the ordinary launch exactly while no other context has
     solves that nobody has waited for; every call that waits counts."""
     _child(stub_path, "child_launch_choice")
+
+
+# ---- contexts driven from several threads
+def child_threads(path, close):
+    import threading
+    stub = _Stub(path)
+    models, _ = _models(4)
+    errors = []
+
+    def work(m):
+        try:
+            for it in range(1, 121):
+                _step(m, it)
+                if it % 3 == 0:
+                    m.numitr()
+            m.get("eta2")
+            if close:
+                m.close()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(m,)) for m in models]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert stub.dead_uses() == 0
+    assert stub.live_streams() == (0 if close else 4)
+    # every context has been waited for: none counts as solving
+    (last,), _ = _models(1)
+    coop = stub.cooperative()
+    _step(last, 1)
+    assert stub.cooperative() == coop
+    # what is open is left to the interpreter's end
+
+
+@pytest.mark.parametrize("close", [True, False])
+def test_contexts_of_several_threads(stub_path, close):
+    """Four threads step a context each at once; the count of solving contexts ends
+    at none, and the process ends cleanly with the contexts closed by their threads
+    or left open."""
+    _child(stub_path, "child_threads", close)
