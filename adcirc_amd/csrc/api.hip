@@ -62,6 +62,10 @@ inline int nblk(int n, int b) { return (n + b - 1) / b; }
 
 }  // namespace
 
+// Solves that take the cooperative launch after a first ordinary launch that was
+// given up (at 122,561 nodes: 11 ms lost, and 22 us a solve while it lasts).
+constexpr int JCG_COOP_AFTER = 512;
+
 struct adcgpu_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -106,6 +110,9 @@ struct adcgpu_ctx {
   double* jin_coef = nullptr;   // the drop-in's ELLPACK arrays as the caller holds them
   int* jin_jcoef = nullptr;
   bool jcg_giveup = false;      // adcgpu_set_jcg_giveup
+  volatile int* given = nullptr;  // pinned: set when an ordinary launch was given up
+  int coop_left = 0;            // solves to come that take the cooperative launch after one
+  int coop_next = JCG_COOP_AFTER;  // how many the next given-up launch brings
   bool solving = false;         // solves enqueued since the stream was last waited for
   int jcg_limit = 0;            // caller's limit on JCG blocks per launch (0: the device's)
   bool jcg_mem = false;         // more row tiles than blocks: k_jcg_mem
@@ -322,6 +329,7 @@ JcgArgs make_jcg_args(adcgpu_ctx* c, double* coef, const int* col, const int* nn
   }
   a.barrier_ticks = (long long)((double)c->clock_khz * 1000.0 * g_wait_seconds);
   a.flags = c->flags;
+  a.given = const_cast<int*>(c->given);
   a.eta2 = eta2;
   a.eta1 = eta1;
   a.nodecode = nodecode;
@@ -414,8 +422,20 @@ int launch_jcg(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh, d
   // nothing to do) solves with two blocks.  Up to a quarter of the resident
   // blocks, so that several processes' solves fit side by side; beyond, the gaps
   // are a small part of the step, and two blocks would take too long.
+  // A given-up solve is slow (us a step of the coastal mesh, with the ordinary
+  // launch, the cooperative one, and given up, less the 2 ms: 5,774 nodes 152, 169,
+  // 507; 20,646 147, 169, 1224; 50,541 167, 189, 3870; 122,561 187, 209, 9237), so
+  // on a chip that is shared for long the context goes back to the cooperative
+  // launch, which waits for its turn: after each given-up launch for twice as many
+  // solves as after the last.
   const bool alone = solve_begins(c);
-  if (cpb > 0 && !u2 && alone && 4 * grid <= c->jcg_cap) {
+  if (c->given && *c->given) {
+    *c->given = 0;
+    c->coop_left = c->coop_next;
+    c->coop_next = std::min(2 * c->coop_next, 1 << 20);
+  }
+  const bool small = cpb > 0 && !u2 && 4 * grid <= c->jcg_cap;
+  if (small && alone && c->coop_left == 0) {
     JcgArgs f = make_jcg_args(c, coef, col, nneigh, rhs, u, n, itmax, zeta, eta2, eta1, nodecode,
                               prescaled, defer_unscal, u2, 0);
     f.hrows = f.halo = -1;
@@ -425,6 +445,7 @@ int launch_jcg(adcgpu_ctx* c, double* coef, const int* col, const int* nneigh, d
     hipLaunchKernelGGL(k_jcg_mem, dim3(2), dim3(JCG_BLOCK), 0, c->stream, f);
     if (int rc = check_launch("JCG")) return rc;
   } else {
+    if (small && c->coop_left > 0) --c->coop_left;
     HIPCHK(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(threads), args, (unsigned)lds,
                                       c->stream));
   }
@@ -904,6 +925,9 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     hipError_t e = hipStreamCreate(&c->stream);
     if (e != hipSuccess) rc = fail(ADCGPU_E_HIP, hipGetErrorString(e));
   }
+  if (!rc && hipHostMalloc((void**)&c->given, sizeof(int), 0) != hipSuccess)
+    rc = fail(ADCGPU_E_HIP, "pinned host buffer");
+  if (!rc) *c->given = 0;
   if (!rc) rc = setup_jcg_grid(c);
   if (!rc) {
     // the patch passes' windows; the wetting propagation stages candidates
@@ -967,6 +991,7 @@ void adcgpu_destroy(adcgpu_ctx* c) {
     (void)hipEventDestroy(ev.second);
   }
   for (void* p : c->allocs) (void)hipFree(p);
+  if (c->given) (void)hipHostFree((void*)c->given);
   if (c->eta_bc_table) (void)hipFree(c->eta_bc_table);
   for (void* p : {(void*)c->fb_ptr, (void*)c->fb_ent, (void*)c->nbv0, (void*)c->bndlen,
                   (void*)c->qn_table})
@@ -1891,6 +1916,10 @@ int adcgpu_last_solve(adcgpu_ctx* c, double* out4) {
 int adcgpu_set_jcg_giveup(adcgpu_ctx* c, int on) {
   if (!c) return fail(ADCGPU_E_ARG, "null context");
   c->jcg_giveup = on != 0;
+  // and what earlier given-up launches brought is forgotten
+  if (c->given) *c->given = 0;
+  c->coop_left = 0;
+  c->coop_next = JCG_COOP_AFTER;
   return 0;
 }
 

@@ -815,6 +815,8 @@ __global__ __launch_bounds__(JCG_BLOCK) void k_jcg_mem(JcgArgs a) {
   if (a.admit &&
       !(__hip_atomic_load(a.admit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & JCG_ABORT))
     return;
+  if (a.given && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(a.given, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   jcg_solve_mem(a, (int)blockIdx.x, (int)gridDim.x);
 }
 

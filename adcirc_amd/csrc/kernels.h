@@ -320,6 +320,7 @@ struct JcgArgs {
   unsigned* admit;          // an ordinary launch of k_jcg_reg: the admission word
                             // (JCG_ABORT); null: a cooperative launch
   long long admit_ticks;    // the longest wait for blocks that have not started
+  int* given;               // k_jcg_mem behind it: set (host memory) when it does the work
   int* flags;
   double* eta2;       // optional: ETA2 = NODECODE*(ETAS+0)+ETA1
   const double* eta1;

@@ -396,7 +396,9 @@ int adcgpu_set_wait_limit(double seconds);
 
 /* For tests: with on != 0 the context's small solves, which are launched like
  * any kernel, are given up as if the chip were taken, so that the two-block
- * solver enqueued behind them does the work (same results). */
+ * solver enqueued behind them does the work (same results).  A given-up launch
+ * sends the context's next 512 solves (then 1024, ...) through the cooperative
+ * launch; every call of this function forgets that. */
 int adcgpu_set_jcg_giveup(adcgpu_ctx* ctx, int on);
 
 /* ---- synthetic forcing ---- */

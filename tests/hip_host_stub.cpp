@@ -14,6 +14,7 @@ namespace {
 std::mutex lock;
 std::set<hipStream_t> streams;  // those not destroyed
 std::atomic<long> ordinary{0}, cooperative{0}, dead_uses{0}, live_streams{0};
+std::atomic<void*> last_pinned{nullptr};
 std::atomic<long> copy_countdown{0}, coop_countdown{0};
 
 void use(hipStream_t s) {
@@ -36,6 +37,7 @@ long stub_ordinary() { return ordinary; }
 long stub_cooperative() { return cooperative; }
 long stub_dead_uses() { return dead_uses; }
 long stub_live_streams() { return live_streams; }
+void* stub_last_pinned() { return last_pinned; }
 void stub_fail_copy(long nth) { copy_countdown = nth; }         // the nth copy from now
 void stub_fail_cooperative(long nth) { coop_countdown = nth; }  // the nth such launch
 
@@ -64,7 +66,11 @@ hipError_t hipMalloc(void** p, size_t n) {
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  const hipError_t e = hipMalloc(p, n);
+  last_pinned = *p;
+  return e;
+}
 hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipGetSymbolAddress(void** p, const void*) {
   static void* scratch = std::calloc(1, 64u << 20);

@@ -46,6 +46,26 @@ def test_two_contexts_bitexact():
         g.close()
 
 
+def test_given_up_launch_is_followed_by_cooperative_ones():
+    """The context sees that a launch was given up: the next solves wait for their
+    turn (the cooperative launch) instead of being given up too.  A given-up solve of
+    this size takes over 1 ms, a cooperative one some 0.15."""
+    case = _basin(160, 130)
+    g, o = build_pair(case_setup(case), case.run)
+    check(g.lib.adcgpu_set_jcg_giveup(g.h, 1), "giveup")
+    ms = []
+    for it in range(1, 7):
+        g.profile(True)
+        step_pair(g, o, it)
+        ms.append(g.profile_read()[0])
+        bad = compare(g, o, it)
+        assert not bad, f"step {it}: " + "; ".join(bad)
+    g.profile(False)
+    log(f"basin {160 * 130} nodes, launches given up: solves took {ms} ms")
+    assert ms[0] > 2.0 * max(ms[2:])
+    g.close()
+
+
 @pytest.mark.skip(reason="a process that ran this ended in SIGSEGV at its exit, after all tests had "
                          "passed; the cause is not known, the host code is clean without a device "
                          "(test_host_runtime.py)")

@@ -37,6 +37,7 @@ class _Stub:
         self.lib = C.CDLL(path, C.RTLD_GLOBAL)  # found before the HIP runtime's symbols
         for f in ("ordinary", "cooperative", "dead_uses", "live_streams"):
             getattr(self.lib, "stub_" + f).restype = C.c_long
+        self.lib.stub_last_pinned.restype = C.c_void_p
         for f in ("fail_copy", "fail_cooperative"):
             getattr(self.lib, "stub_" + f).argtypes = [C.c_long]
 
@@ -137,6 +138,41 @@ def test_launch_follows_what_is_solving(stub_path):
     """A small solve takes the ordinary launch exactly while no other context has
     solves that nobody has waited for; every call that waits counts."""
     _child(stub_path, "child_launch_choice")
+
+
+def child_given_up(path):
+    stub = _Stub(path)
+    (m,), _ = _models(1)
+    given = C.c_int.from_address(stub.last_pinned())
+    it = 0
+
+    def cooperative(n):
+        nonlocal it
+        before = stub.cooperative()
+        for _ in range(n):
+            it += 1
+            _step(m, it)
+        return stub.cooperative() - before
+
+    assert cooperative(3) == 0
+    n = 512
+    for _ in range(3):
+        given.value = 1                      # what k_jcg_mem leaves
+        assert cooperative(n) == n
+        assert given.value == 0
+        assert cooperative(2) == 0
+        n *= 2
+    m.lib.adcgpu_set_jcg_giveup(m.h, 0)
+    given.value = 1
+    assert cooperative(512) == 512
+    assert cooperative(1) == 0
+    m.close()
+
+
+def test_given_up_launch_brings_back_the_cooperative_one(stub_path):
+    """After a small solve's launch was given up (the chip is shared) the context's
+    solves take the cooperative launch, each time for twice as long."""
+    _child(stub_path, "child_given_up")
 
 
 # ---- contexts driven from several threads
