@@ -77,7 +77,7 @@ struct adcgpu_ctx {
   // mesh
   int *nm = nullptr, *inc_ptr = nullptr, *inc = nullptr, *slot = nullptr, *nneigh = nullptr;
   int *col = nullptr, *slot_cols = nullptr;
-  int *csrpos = nullptr, *bnd_index = nullptr, *nbd = nullptr;
+  int *bnd_index = nullptr, *nbd = nullptr;
   int *obcg_ptr = nullptr, *obcg = nullptr, *obcg_q = nullptr, *vbc_ptr = nullptr, *vbc = nullptr, *lbcodei = nullptr;
   double *fdx = nullptr, *fdy = nullptr, *areas = nullptr, *x = nullptr, *y = nullptr, *dp = nullptr;
   double *tau0 = nullptr, *evm = nullptr, *corif = nullptr, *csii = nullptr, *siii = nullptr;
@@ -85,7 +85,7 @@ struct adcgpu_ctx {
   double *eta1, *eta2, *etas, *uu1, *vv1, *uu2, *vv2, *qx1, *qy1, *qx2, *qy2, *h1, *h2, *tk;
   double *etamax, *totalarea, *wsx1, *wsy1, *wsx2, *wsy2, *pr1, *pr2, *gwce_lv, *alphal;
   double *coef, *obc, *fric, *etas_prev = nullptr, *umax = nullptr;
-  int *nodecode, *nnodecode, *noff, *noffold, *mju, *etamax_it, *umax_it;
+  int *nodecode, *nnodecode, *noff, *mju, *etamax_it, *umax_it;
   int cur_it = 0;  // step opened by adcgpu_begin_step
   // work
   double *ep_part = nullptr, *scal = nullptr;
@@ -180,7 +180,7 @@ struct adcgpu_ctx {
     m.nm = nm; m.fdx = fdx; m.fdy = fdy; m.areas = areas; m.x = x; m.y = y; m.dp = dp;
     m.tau0 = tau0; m.evm = evm; m.corif = corif; m.inc_ptr = inc_ptr; m.inc = inc;
     m.slot = slot; m.slot_cols = slot_cols;
-    m.nneigh = nneigh; m.col = col; m.csrpos = csrpos; m.bnd_index = bnd_index; m.nbd = nbd;
+    m.nneigh = nneigh; m.col = col; m.bnd_index = bnd_index; m.nbd = nbd;
     m.obcg_ptr = obcg_ptr; m.obcg = obcg; m.obcg_q = obcg_q; m.vbc_ptr = vbc_ptr;
     m.vbc = vbc; m.lbcodei = lbcodei; m.csii = csii; m.siii = siii;
     m.fb_ptr = nfluxf ? fb_ptr : nullptr; m.fb_ent = nfluxf ? fb_ent : nullptr;
@@ -194,7 +194,7 @@ struct adcgpu_ctx {
     s.tk = tk; s.etamax = etamax; s.totalarea = totalarea; s.wsx1 = wsx1; s.wsy1 = wsy1;
     s.wsx2 = wsx2; s.wsy2 = wsy2; s.pr1 = pr1; s.pr2 = pr2; s.gwce_lv = gwce_lv;
     s.alphal = alphal; s.coef = coef; s.obc = obc; s.fric = fric; s.nodecode = nodecode;
-    s.nnodecode = nnodecode; s.noff = noff; s.noffold = noffold; s.mju = mju;
+    s.nnodecode = nnodecode; s.noff = noff; s.mju = mju;
     s.etamax_it = etamax_it; s.umax = umax; s.umax_it = umax_it; s.ncele = ncele;
     s.tip1 = ctip ? tip1 : nullptr;
     s.tip2 = ctip ? tip2 : nullptr;
@@ -862,7 +862,7 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
   U(&c->nm, nm0); U(&c->inc_ptr, cnt); U(&c->inc, inc); U(&c->slot, slot); U(&c->slot_cols, slot_cols); U(&c->nneigh, nneigh); U(&c->col, col);
   U(&c->jhrange, hrange);
   if (!lcol.empty()) U(&c->jlcol, lcol);
-  U(&c->csrpos, csrpos); U(&c->bnd_index, bnd_index); U(&c->nbd, nbd0);
+  U(&c->bnd_index, bnd_index); U(&c->nbd, nbd0);
   c->nvel = M->nvel;
   for (int I = 0; I < M->nvel; ++I) {
     c->has_rad = c->has_rad || lbc[I] == 30 || lbc[I] == 52;
@@ -886,7 +886,7 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
                          (size_t)c->jreg[1].hmem * nblk(np, 2 * RED_CHUNK)));
   A(&c->alphal, ne); A(&c->coef, (size_t)mnei * np); A(&c->cs, (size_t)mnei * np);
   A(&c->obc, (size_t)std::max(neta, 1) * mnei);
-  A(&c->nodecode, np); A(&c->nnodecode, np); A(&c->noff, ne); A(&c->noffold, ne);
+  A(&c->nodecode, np); A(&c->nnodecode, np); A(&c->noff, ne);
   A(&c->mju, np); A(&c->etamax_it, np); A(&c->etas_prev, np);
   A(&c->umax, np); A(&c->umax_it, np);
   c->mixed = P->precision == ADCGPU_MIXED;
@@ -2228,7 +2228,7 @@ int adcgpu_ml_correction(adcgpu_ctx* c, double* corr_out) {
 extern "C++" {
 namespace {
 struct StatePart {
-  void* dev;
+  void* dev;  // null: nothing kept on the device
   size_t bytes;
 };
 std::vector<StatePart> state_parts(adcgpu_ctx* c) {
@@ -2242,7 +2242,7 @@ std::vector<StatePart> state_parts(adcgpu_ctx* c) {
   int* inodal[] = {c->nodecode, c->nnodecode, c->mju, c->etamax_it, c->umax_it};
   for (int* p : inodal) v.push_back({p, np * 4});
   v.push_back({c->noff, ne * 4});
-  v.push_back({c->noffold, ne * 4});
+  v.push_back({nullptr, ne * 4});  // the layout keeps a place for NOFFOLD: zeros, not read
   v.push_back({c->alphal, ne * 8});
   v.push_back({c->coef, mn * 8});
   v.push_back({c->obc, (size_t)std::max(c->neta, 1) * c->mnei * 8});
@@ -2279,7 +2279,10 @@ int adcgpu_state_save(adcgpu_ctx* c, void* buf, int64_t bytes) {
   std::memcpy(o, hdr, 16);
   o += 16;
   for (const StatePart& p : state_parts(c)) {
-    HIPCHK(hipMemcpyAsync(o, p.dev, p.bytes, hipMemcpyDeviceToHost, c->stream));
+    if (p.dev)
+      HIPCHK(hipMemcpyAsync(o, p.dev, p.bytes, hipMemcpyDeviceToHost, c->stream));
+    else
+      std::memset(o, 0, p.bytes);
     o += p.bytes;
   }
   HIPCHK(stream_wait(c));
@@ -2298,7 +2301,7 @@ int adcgpu_state_load(adcgpu_ctx* c, const void* buf, int64_t bytes) {
   HIPCHK(hipSetDevice(c->device));
   c->ep_steps = 2;
   for (const StatePart& p : state_parts(c)) {
-    HIPCHK(hipMemcpyAsync(p.dev, o, p.bytes, hipMemcpyHostToDevice, c->stream));
+    if (p.dev) HIPCHK(hipMemcpyAsync(p.dev, o, p.bytes, hipMemcpyHostToDevice, c->stream));
     o += p.bytes;
   }
   HIPCHK(stream_wait(c));

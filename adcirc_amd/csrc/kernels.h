@@ -101,7 +101,6 @@ struct DevMesh {
   const int* slot_cols; // [ne*3] per slot p: CSR_POSITION slots ja | jb << 16 (0-based)
   const int* nneigh;    // [np]
   const int* col;       // [mnei*np] column-major, 0-based (slot 0 = self)
-  const int* csrpos;    // [ne*3*2] 0-based column slots
   const int* bnd_index; // [np] elevation-boundary index, -1, or -2-k for the
                         //      k-th node that takes specified-flux edge terms
   const int* nbd;       // [neta] 0-based
@@ -127,7 +126,7 @@ struct DevState {
   double *eta1, *eta2, *etas, *uu1, *vv1, *uu2, *vv2, *qx1, *qy1, *qx2, *qy2;
   double *h1, *h2, *tk, *etamax, *totalarea, *wsx1, *wsy1, *wsx2, *wsy2, *pr1, *pr2;
   double *gwce_lv, *alphal, *coef, *obc, *fric;
-  int *nodecode, *nnodecode, *noff, *noffold, *mju;
+  int *nodecode, *nnodecode, *noff, *mju;
   int *etamax_it;  // step of the last ETAMAX rise (0: never)
   double *umax;    // peak depth-averaged speed at wet nodes
   int *umax_it;    // step of the last UMAX rise (0: never)

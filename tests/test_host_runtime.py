@@ -175,6 +175,27 @@ def test_given_up_launch_brings_back_the_cooperative_one(stub_path):
     _child(stub_path, "child_given_up")
 
 
+def child_snapshot_layout(path):
+    _Stub(path)
+    (m,), _ = _models(1)
+    np_, ne, mnei = m.np_, m.ne, m.mnei
+    a = m.save_state()
+    noffold = 16 + 25 * 8 * np_ + 5 * 4 * np_ + 4 * ne
+    assert a.size == (noffold + 4 * ne + 8 * ne + 8 * mnei * np_ + 8 * max(m.neta, 1) * mnei
+                      + 8 * 8 + 12 * 8 + 16 * 4)
+    b = np.random.default_rng(1).integers(0, 256, a.size).astype(np.uint8)
+    b[:16] = a[:16]
+    m.load_state(b)
+    b[noffold:noffold + 4 * ne] = 0  # NOFFOLD: once kept, not read
+    assert np.array_equal(m.save_state(), b)
+    m.close()
+
+
+def test_snapshot_layout(stub_path):
+    """The snapshot's layout is that of earlier files."""
+    _child(stub_path, "child_snapshot_layout")
+
+
 # ---- contexts driven from several threads
 def child_threads(path, close):
     import threading
