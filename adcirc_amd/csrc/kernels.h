@@ -284,6 +284,37 @@ __device__ __forceinline__ double friction(const FricPrm& f, int i, double u, do
   return fmin(a, f.tkmax);
 }
 
+// computeAlpha (src/wetdry.F:1561-1652): ALPHAL of a wet element from ETA2 and DP
+// of its vertices.  `geometry` leaves FDXE and FDYE and returns AREAS; it is called
+// where some vertex is shallow only.
+template <class Geometry>
+__device__ __forceinline__ double compute_alpha(double e1, double e2, double e3, double d1,
+                                                double d2, double d3, double slim,
+                                                const Geometry& geometry) {
+  double al = 1.0;
+  const double hn1 = e1 + d1, hn2 = e2 + d2, hn3 = e3 + d3;
+  if ((hn1 <= 5.0e-1) || (hn2 <= 5.0e-1) || (hn3 <= 5.0e-1)) {
+    double fx[3], fy[3];
+    const double area = geometry(fx, fy);
+    const double DPDXA = d1 * fx[0] + d2 * fx[1] + d3 * fx[2];
+    const double DPDYA = d1 * fy[0] + d2 * fy[1] + d3 * fy[2];
+    const double DETADXA = e1 * fx[0] + e2 * fx[1] + e3 * fx[2];
+    const double DETADYA = e1 * fy[0] + e2 * fy[1] + e3 * fy[2];
+    const double DPM = __builtin_sqrt(DPDXA * DPDXA + DPDYA * DPDYA) / area;
+    if (DPM > 1e-5) {
+      const double DDTMP = DETADXA * (-DPDXA) + DETADYA * (-DPDYA);
+      if (fabs(DDTMP) > 1e-12)
+        al = slim * (__builtin_sqrt(DPDXA * DPDXA + DPDYA * DPDYA) / ((1.0 / area) * (DDTMP)));
+    } else {
+      const double DETAM = __builtin_sqrt(DETADXA * DETADXA + DETADYA * DETADYA) / area;
+      if (fabs(DETAM) > 1e-12) al = slim / DETAM;
+    }
+    if (al <= 0.0) al = 1.0;
+    if (al >= 1.0) al = 1.0;
+  }
+  return al;
+}
+
 struct JcgArgs {
   int n, itmax, maxfn;
   double zeta, tz;

@@ -679,36 +679,21 @@ __global__ __launch_bounds__(WD_BLOCK) void k_wd_chain_batch(const MemberArgs* _
   wd_chain_block(x.m, x.s, x.wd, x.pre.flags, blockIdx.x, x.nchain);
 }
 
-// computeAlpha (src/wetdry.F:1561-1652): ALPHAL of element e.
+// computeAlpha: ALPHAL of element e.
 __device__ __forceinline__ double wd_alpha(const DevMesh& m, const DevState& s, int e, int* flags,
                                            double slim) {
   const int n1 = m.nm[3 * e], n2 = m.nm[3 * e + 1], n3 = m.nm[3 * e + 2];
   double al = 1.0;
   const int ncele = s.nodecode[n1] * s.nodecode[n2] * s.nodecode[n3] * s.noff[e];
-  if (ncele == 1) {
-    const double hn1 = s.eta2[n1] + m.dp[n1], hn2 = s.eta2[n2] + m.dp[n2],
-                 hn3 = s.eta2[n3] + m.dp[n3];
-    if ((hn1 <= 5.0e-1) || (hn2 <= 5.0e-1) || (hn3 <= 5.0e-1)) {
-      const double FDX1 = m.fdx[3 * e], FDX2 = m.fdx[3 * e + 1], FDX3 = m.fdx[3 * e + 2];
-      const double FDY1 = m.fdy[3 * e], FDY2 = m.fdy[3 * e + 1], FDY3 = m.fdy[3 * e + 2];
-      const double DPDXA = m.dp[n1] * FDX1 + m.dp[n2] * FDX2 + m.dp[n3] * FDX3;
-      const double DPDYA = m.dp[n1] * FDY1 + m.dp[n2] * FDY2 + m.dp[n3] * FDY3;
-      const double DETADXA = s.eta2[n1] * FDX1 + s.eta2[n2] * FDX2 + s.eta2[n3] * FDX3;
-      const double DETADYA = s.eta2[n1] * FDY1 + s.eta2[n2] * FDY2 + s.eta2[n3] * FDY3;
-      const double area = m.areas[e];
-      const double DPM = __builtin_sqrt(DPDXA * DPDXA + DPDYA * DPDYA) / area;
-      if (DPM > 1e-5) {
-        const double DDTMP = DETADXA * (-DPDXA) + DETADYA * (-DPDYA);
-        if (fabs(DDTMP) > 1e-12)
-          al = slim * (__builtin_sqrt(DPDXA * DPDXA + DPDYA * DPDYA) / ((1.0 / area) * (DDTMP)));
-      } else {
-        const double DETAM = __builtin_sqrt(DETADXA * DETADXA + DETADYA * DETADYA) / area;
-        if (fabs(DETAM) > 1e-12) al = slim / DETAM;
-      }
-      if (al <= 0.0) al = 1.0;
-      if (al >= 1.0) al = 1.0;
-    }
-  }
+  if (ncele == 1)
+    al = compute_alpha(s.eta2[n1], s.eta2[n2], s.eta2[n3], m.dp[n1], m.dp[n2], m.dp[n3], slim,
+                       [&](double fx[3], double fy[3]) {
+                         for (int k = 0; k < 3; ++k) {
+                           fx[k] = m.fdx[3 * e + k];
+                           fy[k] = m.fdy[3 * e + k];
+                         }
+                         return m.areas[e];
+                       });
   s.alphal[e] = al;
   // the passes that read ALPHAL take 1 unless this is set
   if (al != 1.0) atomicOr(&flags[F_ALPHA], 1);

@@ -889,33 +889,15 @@ __global__ __launch_bounds__(PATCH_THREADS) void k_wd_d2_batch(const MemberArgs*
 enum { MF_X, MF_Y, MF_U, MF_V, MF_H1, MF_EVM, MF_E1, MF_E2, MF_DP, MF_P1, MF_P2, MF_T1, MF_T2, MF_COUNT };
 static_assert(MF_COUNT == PATCH_MOM_FIELDS, "LDS of k_mom");
 
-// computeAlpha (src/wetdry.F:1561-1652) of a wet element.
+// computeAlpha of a wet element of the patch.
 __device__ __forceinline__ double alpha_terms(const double* sh, int ws, int n1, int n2, int n3,
                                               const ElemGeo<double>& g, double slim) {
-  const double FDX1 = g.x1, FDX2 = g.x2, FDX3 = g.x3, FDY1 = g.y1, FDY2 = g.y2, FDY3 = g.y3;
-  const double AreaIE2 = g.a;
-  double al = 1.0;
-  const double hn1 = W(MF_E2, n1) + W(MF_DP, n1), hn2 = W(MF_E2, n2) + W(MF_DP, n2),
-               hn3 = W(MF_E2, n3) + W(MF_DP, n3);
-  if ((hn1 <= 5.0e-1) || (hn2 <= 5.0e-1) || (hn3 <= 5.0e-1)) {
-    const double DPDXA = W(MF_DP, n1) * FDX1 + W(MF_DP, n2) * FDX2 + W(MF_DP, n3) * FDX3;
-    const double DPDYA = W(MF_DP, n1) * FDY1 + W(MF_DP, n2) * FDY2 + W(MF_DP, n3) * FDY3;
-    const double DETADXA = W(MF_E2, n1) * FDX1 + W(MF_E2, n2) * FDX2 + W(MF_E2, n3) * FDX3;
-    const double DETADYA = W(MF_E2, n1) * FDY1 + W(MF_E2, n2) * FDY2 + W(MF_E2, n3) * FDY3;
-    const double area = AreaIE2;
-    const double DPM = __builtin_sqrt(DPDXA * DPDXA + DPDYA * DPDYA) / area;
-    if (DPM > 1e-5) {
-      const double DDTMP = DETADXA * (-DPDXA) + DETADYA * (-DPDYA);
-      if (fabs(DDTMP) > 1e-12)
-        al = slim * (__builtin_sqrt(DPDXA * DPDXA + DPDYA * DPDYA) / ((1.0 / area) * (DDTMP)));
-    } else {
-      const double DETAM = __builtin_sqrt(DETADXA * DETADXA + DETADYA * DETADYA) / area;
-      if (fabs(DETAM) > 1e-12) al = slim / DETAM;
-    }
-    if (al <= 0.0) al = 1.0;
-    if (al >= 1.0) al = 1.0;
-  }
-  return al;
+  return compute_alpha(W(MF_E2, n1), W(MF_E2, n2), W(MF_E2, n3), W(MF_DP, n1), W(MF_DP, n2),
+                       W(MF_DP, n3), slim, [&](double fx[3], double fy[3]) {
+                         fx[0] = g.x1; fx[1] = g.x2; fx[2] = g.x3;
+                         fy[0] = g.y1; fy[1] = g.y2; fy[2] = g.y3;
+                         return g.a;
+                       });
 }
 
 // Element loop of Mom_Eqs_New_NC (src/momentum.F:298-699): advection,
