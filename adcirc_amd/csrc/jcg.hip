@@ -1,4 +1,11 @@
-// ITPACK jcg (src/itpackv.F:63-456) for one persistent cooperative launch.
+// ITPACK jcg (src/itpackv.F:63-456) for one persistent cooperative launch: the
+// solver of the drop-ins, and of contexts whose rows k_jcg_reg cannot hold.  Those
+// are bandwidths whose window of 2,048 or 4,096 rows and all rows they reference
+// passes 152 KB of LDS (a mesh numbered at random from some 19,000 nodes: the
+// products gather from memory), and rows with so many entries past the register
+// slots that they do not fit beside the window (three overlapping layers of
+// triangles and a bandwidth of 5,002: the pseudo-residual alone is staged in LDS,
+// 327 us a solve of 25,000 rows where the gathering kernel takes 527 on 22,500).
 //
 // Launch: blocks of JCG_CPB x 512 threads, each 512-thread group owning one
 // 2048-row chunk, plus one eigenvalue block.
