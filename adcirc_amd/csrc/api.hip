@@ -673,9 +673,8 @@ int adcgpu_create(const adcgpu_mesh* M, const adcgpu_params* P, int device, adcg
     for (int k = 0; k < 3; ++k) cnt[nm0[3 * (size_t)e + k] + 1]++;
   for (int i = 0; i < np; ++i) cnt[i + 1] += cnt[i];
   std::vector<int> inc(3 * (size_t)ne), fillp(cnt.begin(), cnt.end() - 1);
-  // ascending element order per node; slot is the inverse map, so element
-  // kernels write each (element, vertex) contribution where its node's
-  // ordered sum reads it
+  // ascending element order per node; slot is the inverse map (a wetting
+  // candidate finds itself in its nodes' lists)
   std::vector<int> slot(3 * (size_t)ne);
   for (int e = 0; e < ne; ++e)
     for (int k = 0; k < 3; ++k) {

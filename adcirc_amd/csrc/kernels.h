@@ -37,7 +37,7 @@ constexpr int JCG_STAGE_MAX_BYTES = 120 * 1024;
 static_assert(JCG_STAGE_MAX_BYTES / 8 <= 65536, "staged positions are 16-bit");
 // patches: a block's threads, and at most so many elements (one per thread),
 // window nodes, and own nodes.  About 10 x 10 nodes have 235 elements: one per
-// thread, and a sixth more element evaluations than the mesh has elements.
+// thread, and a fifth more element evaluations than the mesh has elements.
 constexpr int PATCH_THREADS = 256, PATCH_ELEMS = 256, PATCH_WIN = 192, PATCH_NODES = 96;
 static_assert(PATCH_NODES <= PATCH_THREADS / 2 && PATCH_WIN <= PATCH_THREADS, "patch shape");
 constexpr int PATCH_GWCE_FIELDS = 18, PATCH_MOM_FIELDS = 13;
@@ -45,7 +45,7 @@ constexpr int patch_lds_bytes(int fields, int terms, int wmax) {
   return 8 * (fields * wmax > terms ? fields * wmax : terms);
 }
 constexpr int PATCH_GWCE_TERMS = 9 * PATCH_ELEMS + 1, PATCH_MOM_TERMS = 6 * PATCH_ELEMS;
-constexpr int LHS_MAXW = 32;         // widest COEF row (MNEI): LDS of the row kernel
+constexpr int LHS_MAXW = 32;         // widest COEF row (MNEI) that a context takes
 // ordered wetting updates: candidates are closed in blocks of WD_BLOCK, each
 // block naming at most WD_XMAX earlier candidates it depends on
 constexpr int WD_BLOCK = 1024;

@@ -2,13 +2,11 @@
 //
 // Parity design: every per-node sum the reference forms by scattering element
 // contributions in ascending element order (GWCE matrix, GWCE load vector,
-// momentum load vectors, TotalArea) is formed here by a node-centric gather
-// over the node's incident elements in ascending element id, which is the same
-// order, so the result is bit-identical.  Inner products use one fixed blocked
-// tree (2048-row chunks, 8 rows per thread, xor butterfly over the 64 lanes,
-// (w0+w1)+(w2+w3) over the 4 waves; chunk sums reduced with the same pattern),
-// identical on every launch shape.  Built with -ffp-contract=off so no
-// multiply-add is fused.
+// momentum load vectors, TotalArea) is formed node by node over the node's
+// incident elements in ascending element id (here and in patch.hip), which is the
+// same order, so the result is bit-identical.  Inner products use one fixed
+// blocked tree (reduce.h), identical on every launch shape.  Built with
+// -ffp-contract=off so no multiply-add is fused.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -1,8 +1,9 @@
 // adcgpu_jcg_noalloc: the drop-in JCG for callers that cannot allocate
 // memory (code under graph capture, tight serving loops, harnesses that
 // forbid hipMalloc).  Every device buffer of the solve lives in one static
-// device array, `scratch`; the host side allocates nothing either: the
-// ELLPACK compaction that adcgpu_jcg does on the host runs here in a kernel.
+// device array, `scratch`; the host side allocates nothing either.  The kernels
+// that compact the caller's ELLPACK rows and put the solved ones back
+// (k_na_compact, k_na_scatter) are adcgpu_jcg's too.
 //
 // Each GPU holds its own copy of `scratch` at its own address, obtained once
 // per device with hipGetSymbolAddress; host code uses that address, never
@@ -50,10 +51,10 @@ static_assert(NA_BYTES == ADCGPU_JCG_NOALLOC_SCRATCH_BYTES,
 
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 
-// First failing row and check of the system, as the host drop-in finds them
-// row by row: per row, no diagonal (402) before a column index above n
-// (argument error) before a zero diagonal (401) before a negative one
-// (unsupported).  `check` holds the smallest row*4 + kind seen.
+// First failing row and check of the system, as a pass row by row finds them:
+// per row, no diagonal (402) before a column index above n (argument error)
+// before a zero diagonal (401) before a negative one (unsupported).  `check`
+// holds the smallest row*4 + kind seen.
 
 // One row per thread: the ELLPACK row of the caller's (n, maxnz) arrays,
 // copied with leading dimension n, compacted to the solver's layout with the

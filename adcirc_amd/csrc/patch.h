@@ -23,7 +23,7 @@ namespace adcgpu {
 // than PATCH_ELEMS elements: `ok` is false then).  Every list of a patch starts
 // at a multiple of its longest length, so that a block's first loads need no
 // directory.  Compact leaves keep the elements formed by two patches few: a
-// sixth more than the mesh has.
+// fifth more than the mesh has.
 struct PatchPlan {
   std::vector<int> win, el;
   std::vector<ushort4> lv;
