@@ -43,8 +43,8 @@
 // The sums' trees, the rows' operations and the scalar recurrences are those
 // of k_jcg; results are the same bits.
 // Measured (MI355X, FP64, about 15 iterations; us per launch, k_jcg before):
-// 5,151 rows 101 (248), 20,646 rows 111 (257), 250,244 rows 126 (276),
-// 999,151 rows 242 (447); with every test at once 128, 133, 146, 251.
+// 5,151 rows 102 (248), 20,646 rows 110 (257), 250,244 rows 121 (276),
+// 999,151 rows 244 (447); with every test at once 128, 133, 146, 251.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -18,8 +18,9 @@
 // us at 999,151 nodes (wet/dry, storm), before and after: k_gwce 154, the passes
 // it replaces (element terms 102, matrix 76, friction 8, a launch each for the
 // matrix's other cases 11) 197; k_mom 104 to 110, before 106 + 54.  At 20,646 nodes
-// 9.1 (23.5) and 7.3 (12.3), where a launch costs 5.  About 3 TB/s at 1M: the window's
-// runs of some 16 nodes are shorter than what memory streams at (a copy: 5).
+// 9.1 (23.5) and 7.3 (12.3), where a launch costs 5.  At 1M k_gwce moves 270 MB in
+// and 81 out past the L2 (232 and 72 counted once), 2.3 TB/s, k_mom 294 and 62,
+// 3.25 TB/s; a copy reaches 5, the window's runs being some 16 nodes long.
 //
 // Every sum keeps the reference's order: a node's contributions are listed in
 // ascending element order.
