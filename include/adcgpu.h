@@ -388,9 +388,11 @@ int adcgpu_jcg_noalloc(int n, int ndim, int maxnz, int32_t *jcoef, double *coef,
                        double *u, int32_t *iparm, double *rparm);
 
 /* Upper bound, in seconds of device wall clock, of every wait inside the
- * persistent JCG kernel (grid barrier, neighbour flags); default 0.5.  A wait
- * that runs out sets an error flag that every block sees, so the launch drains
- * and the call returns ADCGPU_E_HIP.  No counterpart in the reference; for
+ * persistent JCG kernel (grid barrier, neighbour flags, partials); default 0.5.
+ * A wait that runs out sets an error flag that every block sees, so the launch
+ * drains and the call returns ADCGPU_E_HIP.  (While some block of a small solve's
+ * ordinary launch has not started, the bound is 2 ms instead: the launch is then
+ * given up and the solve done by two blocks.)  No counterpart in the reference; for
  * failure-handling tests (a tiny bound forces the error path from the host). */
 int adcgpu_set_wait_limit(double seconds);
 
